@@ -327,7 +327,8 @@ int mimir_prefixlm_bwd_stages(const MimirPrefixLMBwdParams* p, int stages, void*
     float* const dout_s = (float*)((char*)p->workspace + ws.dout);
     e = mimir::launch_prologue(pro, stream);
     if (e == hipSuccess && (stages & MIMIR_BWD_STAGE_DELTA))
-      e = mimir::launch_gate_bwd_f32(*p, dout_s, (float*)((char*)p->workspace + ws.delta), stream);
+      e = mimir::launch_gate_bwd_f32(*p, dout_s, (float*)((char*)p->workspace + ws.delta),
+                                     (float*)((char*)p->workspace + ws.lse2), stream);
     if (e == hipSuccess) {
       MimirPrefixLMBwdParams q = *p;
       q.dout = dout_s;

@@ -750,8 +750,9 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
 // Layer kernels (prefixlm_layer.hip).
 hipError_t launch_rope(const MimirRopeParams& p, hipStream_t stream);
 hipError_t launch_gate_fwd_f32(const MimirPrefixLMFwdParams& p, hipStream_t stream);
-// float32 gate backward rows: dout_s = dout * s, delta, dgate (one thread per row).
-hipError_t launch_gate_bwd_f32(const MimirPrefixLMBwdParams& p, float* dout_s, float* delta, hipStream_t stream);
+// float32 gate backward rows: dout_s = dout * s, delta, lse * log2(e), dgate (one thread per row).
+hipError_t launch_gate_bwd_f32(const MimirPrefixLMBwdParams& p, float* dout_s, float* delta, float* lse2,
+                               hipStream_t stream);
 }  // namespace mimir
 
 namespace mimir {

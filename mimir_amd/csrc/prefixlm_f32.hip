@@ -2,20 +2,52 @@
 //
 // The fp32 path serves the reference's CPU training precision
 // (flash_attention_prefixlm_dense.py runs in fp32) and is held to the fp32
-// oracle at 1e-5, so it keeps every product and sum in fp32 on the vector ALUs:
-// four lanes share one row (D/4 contiguous values each; eight in the forward) and
-// combine dot products with cross-lane adds.  K/V (forward, dQ) or Q/dO (dK/dV) tiles are staged in
-// LDS and read as broadcasts.  Structure and ownership follow the Metal kernels
-// of flash_attention_prefixlm_mps.py (forward 391-476, dQ 967-1039, dK/dV
-// 1245-1322), extended to GQA.
+// oracle at 1e-5: every product and sum stays in fp32, the products on the fp32
+// matrix instruction v_mfma_f32_32x32x2_f32 (64 cycles for 4096 FLOP, 157
+// TFLOP/s over the chip; measured 154 in a large matrix product).  Ownership
+// follows the Metal kernels of flash_attention_prefixlm_mps.py (forward
+// 391-476, dQ 967-1039, dK/dV 1245-1322), extended to GQA.
+//
+// A workgroup owns 32 rows (queries, or keys for dK / dV) of one head; its four
+// waves take the 32-row tiles of the other side in turn, each with accumulators
+// of its own that are added through LDS at the end.  Small fp32 batches (a few
+// thousand tokens) then still put two waves on every SIMD, and the tile loop
+// holds no barrier.  With the owned rows on the columns of every product, S^T =
+// K Q^T (dK / dV: S = Q K^T) leaves the probabilities in registers exactly as
+// the B operand of the next product wants them: register r of lane half hi is
+// row 8 (r / 4) + 4 hi + r % 4, and one matrix step sums over the two rows that
+// the two halves hold.
+//
+//  * The owned rows (B operand) sit in LDS, [32][D + 4]: a lane reads 16 bytes
+//    per four steps, and the row stride of an odd number of 16-byte units keeps
+//    the sixteen rows of a read in distinct banks.
+//  * The streamed rows (A operand) come straight from memory into registers, in
+//    row form (lane = row, 16 bytes of it per four steps) for S and dP, and in
+//    column form (lane = D / 32 neighbouring columns, one row per step) for the
+//    second products, so that no transpose is needed.  They are re-read from
+//    the caches by every workgroup of a head: 16 KiB per 4096 matrix cycles and
+//    wave at head_dim 64, well under what L1 and L2 deliver.  Each operand is
+//    requested one product (D / 2 matrix steps, 2048 cycles at head_dim 64)
+//    before its use, which covers the latency without double buffers.
+//    Row ranges are enforced by the buffer resource of the tile: rows past the
+//    end read as zeros.
+//
+// Bound by the matrix unit and, on small batches, by the number of workgroups:
+// 4 x 512 tokens, 8 heads, head_dim 64 (1.2 GFLOP forward, 5.0 executed in the
+// backward): forward 86 -> 25 us (a workgroup's start-up and merge are a third
+// of it), dQ + dK / dV 310 -> 77 us against the vector-ALU kernels these
+// replace; one sequence of 4096 tokens, same heads, forward + backward 3.20 ->
+// 0.68 ms.
 #include "prefixlm_common.h"
 
 namespace {
 using namespace mimir;
 
-constexpr int kThreads = 256;
-constexpr int kRowsPerBlock = kThreads / 4;  // 64 rows, 4 lanes per row
-constexpr int kTile = 32;                    // keys (or queries) per LDS tile
+constexpr int kWaves = 4;
+constexpr int kThreads = kWaves * 64;
+constexpr int kRows = 32;            // rows per workgroup, and per streamed tile
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int kDeltaRows = kThreads / 4;  // delta: 64 rows, 4 lanes per row
 
 struct F32Args {
   const float* q;
@@ -23,18 +55,20 @@ struct F32Args {
   const float* v;
   float* o;
   float* lse;
-  const float* olse;  // bwd: forward lse
+  const float* olse;  // delta: forward lse
   const float* out;   // bwd: forward output
   const float* dout;
   float* dq;
   float* dk;
   float* dv;
-  float* delta;
+  float* delta;       // [Hq, T], workspace
+  float* lse2;        // [Hq, T], lse * log2(e), workspace
   const int32_t* prefix_lens;
   const int32_t* cu_seqlens;
   int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh, do_st, do_sh;
   int64_t dq_st, dq_sh, dk_st, dk_sh, dv_st, dv_sh, lse_sh;
-  int T, Hq, Hkv, group, total_seqlen, is_causal, num_tiles;
+  int T, Hq, Hkv, group, total_seqlen, is_causal, num_tiles, numseqs;
+  int z0;  // backward: first role of the grid (0: dK / dV, 1 + g: dQ of q head g of the group)
   float scale, scale_log2;
 };
 
@@ -44,324 +78,459 @@ __device__ __forceinline__ float sum4(float x) {
   return x;
 }
 
+// delta = rowsum(O * dO) and lse * log2(e) of every (token, head) row.
 template <int D>
-__device__ __forceinline__ void load_row(float (&dst)[D / 4], const float* row, int sub, bool valid) {
-#pragma unroll
-  for (int e = 0; e < D / 4; e += 4) {
-    f32x4 t = valid ? *(const f32x4*)&row[sub * (D / 4) + e] : f32x4{0.f, 0.f, 0.f, 0.f};
-    dst[e] = t[0]; dst[e + 1] = t[1]; dst[e + 2] = t[2]; dst[e + 3] = t[3];
-  }
-}
-
-// Cooperative load of `kTile` rows [r0, r0 + kTile) of a [rows][stride] fp32
-// matrix into an LDS tile [kTile][D]; rows >= nrows are zero-filled.
-template <int D>
-__device__ __forceinline__ void stage(float* tile, const float* base, int64_t stride, int r0, int nrows) {
-  constexpr int V4 = D / 4;
-  for (int i = threadIdx.x; i < kTile * V4; i += kThreads) {
-    const int row = i / V4, c = i % V4;
-    const int r = r0 + row;
-    f32x4 t = r < nrows ? *(const f32x4*)&base[(int64_t)r * stride + 4 * c] : f32x4{0.f, 0.f, 0.f, 0.f};
-    *(f32x4*)&tile[row * D + 4 * c] = t;
-  }
-}
-
-template <int D>
-__device__ __forceinline__ float dot_tile(const float (&x)[D / 4], const float* tile_row, int sub) {
-  float acc = 0.f;
-#pragma unroll
-  for (int e = 0; e < D / 4; e += 4) {
-    const f32x4 t = *(const f32x4*)&tile_row[sub * (D / 4) + e];
-    acc = __builtin_fmaf(x[e], t[0], acc);
-    acc = __builtin_fmaf(x[e + 1], t[1], acc);
-    acc = __builtin_fmaf(x[e + 2], t[2], acc);
-    acc = __builtin_fmaf(x[e + 3], t[3], acc);
-  }
-  return sum4(acc);
-}
-
-// The forward gives each row eight lanes (D / 8 values each; the dot products
-// combine with three cross-lane adds), so 32 rows per workgroup: twice the
-// workgroups, and waves, of four lanes per row on the same batch, which the
-// tile loop's LDS broadcast reads need to hide their latency.  K / V tiles are
-// double-buffered: each thread loads its share of the next tile into registers
-// before the current tile's arithmetic and stores it to the other LDS buffer
-// after, so one barrier per tile remains and the global loads' latency hides
-// behind the arithmetic (staged synchronously, it was paid once per tile).
-constexpr int kFwdLanes = 8;
-constexpr int kFwdRows = kThreads / kFwdLanes;
-
-template <int D>
-__global__ __launch_bounds__(kThreads) void fwd_f32_kernel(const F32Args a) {
-  constexpr int EPL = D / kFwdLanes;
-  static_assert(EPL % 4 == 0, "whole float4 per lane");
-  constexpr int V4 = D / 4;
-  constexpr int kVecs = kTile * V4 / kThreads;  // float4 of K (and of V) per thread per tile
-  static_assert(kVecs * kThreads == kTile * V4, "a tile divides evenly over the threads");
-  __shared__ __attribute__((aligned(16))) float sK[2][kTile * D];
-  __shared__ __attribute__((aligned(16))) float sV[2][kTile * D];
-  const int h = blockIdx.x % a.Hq;
-  const int s = blockIdx.x / a.Hq;
-  const int tile = a.num_tiles - 1 - (int)blockIdx.y;
-  const SeqGeom g = load_seq<true>(a.cu_seqlens, a.prefix_lens, s, a.total_seqlen, a.is_causal, a.T);
-  const int m0 = tile * kFwdRows;
-  if (m0 >= g.nq) return;
-  const int hk = h / a.group;
-  const int sub = threadIdx.x % kFwdLanes;
-  const int qpos = m0 + threadIdx.x / kFwdLanes;
-  const bool valid = qpos < g.nq;
-  const int kend = kend_of(g.p, qpos);
-  const int wg_kend = max(g.p, min(m0 + kFwdRows, g.nq));
-
-  float qv[EPL], acc[EPL];
-  {
-    const float* qrow = a.q + (int64_t)(g.start + qpos) * a.q_st + (int64_t)h * a.q_sh + sub * EPL;
-#pragma unroll
-    for (int e = 0; e < EPL; e += 4) {
-      const f32x4 t = valid ? *(const f32x4*)&qrow[e] : f32x4{0.f, 0.f, 0.f, 0.f};
-      qv[e] = t[0]; qv[e + 1] = t[1]; qv[e + 2] = t[2]; qv[e + 3] = t[3];
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
-  const float* kb = a.k + (int64_t)g.start * a.k_st + (int64_t)hk * a.k_sh;
-  const float* vb = a.v + (int64_t)g.start * a.v_st + (int64_t)hk * a.v_sh;
-
-  // this thread's share of a tile: float4 column c of row `row`, kVecs of them
-  f32x4 nk[kVecs], nv[kVecs];
-  auto fetch = [&](int k0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < kVecs; ++i) {
-      const int idx = (int)threadIdx.x + i * kThreads, row = idx / V4, c = idx % V4;
-      const bool in = k0 + row < g.n;
-      nk[i] = in ? *(const f32x4*)&kb[(int64_t)(k0 + row) * a.k_st + 4 * c] : f32x4{0.f, 0.f, 0.f, 0.f};
-      nv[i] = in ? *(const f32x4*)&vb[(int64_t)(k0 + row) * a.v_st + 4 * c] : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-  };
-  auto put = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < kVecs; ++i) {
-      const int idx = (int)threadIdx.x + i * kThreads, row = idx / V4, c = idx % V4;
-      *(f32x4*)&sK[buf][row * D + 4 * c] = nk[i];
-      *(f32x4*)&sV[buf][row * D + 4 * c] = nv[i];
-    }
-  };
-  // The tile's arithmetic; false: no allowed key yet (only for rows with kend <= k0).
-  auto tile_step = [&](int k0, const float* tK, const float* tV) __attribute__((always_inline)) {
-    float sc[kTile];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < kTile; ++j) {
-      float x = 0.f;
-#pragma unroll
-      for (int e = 0; e < EPL; e += 4) {
-        const f32x4 t = *(const f32x4*)&tK[j * D + sub * EPL + e];
-        x = __builtin_fmaf(qv[e], t[0], x);
-        x = __builtin_fmaf(qv[e + 1], t[1], x);
-        x = __builtin_fmaf(qv[e + 2], t[2], x);
-        x = __builtin_fmaf(qv[e + 3], t[3], x);
-      }
-      x += __shfl_xor(x, 1, 64);
-      x += __shfl_xor(x, 2, 64);
-      x += __shfl_xor(x, 4, 64);
-      if (k0 + j >= kend) x = -INFINITY;
-      sc[j] = x;
-      mx = fmaxf(mx, x);
-    }
-    const float m_new = fmaxf(m_run, mx);
-    if (m_new == -INFINITY) return;
-    const float alpha = fast_exp2((m_run - m_new) * a.scale_log2);
-    const float mb = m_new * a.scale_log2;
-    l_run *= alpha;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] *= alpha;
-#pragma unroll
-    for (int j = 0; j < kTile; ++j) {
-      const float pr = fast_exp2(__builtin_fmaf(sc[j], a.scale_log2, -mb));
-      l_run += pr;
-#pragma unroll
-      for (int e = 0; e < EPL; e += 4) {
-        const f32x4 t = *(const f32x4*)&tV[j * D + sub * EPL + e];
-        acc[e] = __builtin_fmaf(pr, t[0], acc[e]);
-        acc[e + 1] = __builtin_fmaf(pr, t[1], acc[e + 1]);
-        acc[e + 2] = __builtin_fmaf(pr, t[2], acc[e + 2]);
-        acc[e + 3] = __builtin_fmaf(pr, t[3], acc[e + 3]);
-      }
-    }
-    m_run = m_new;
-  };
-
-  if (wg_kend > 0) {
-    fetch(0);
-    put(0);
-  }
-  __syncthreads();
-  for (int k0 = 0, buf = 0; k0 < wg_kend; k0 += kTile, buf ^= 1) {
-    const bool more = k0 + kTile < wg_kend;
-    if (more) fetch(k0 + kTile);  // in flight during this tile's arithmetic
-    tile_step(k0, sK[buf], sV[buf]);
-    // The other buffer's last readers finished this tile's predecessor before the
-    // barrier that ended it; this tile's readers finish before the next barrier.
-    if (more) put(buf ^ 1);
-    __syncthreads();
-  }
-  if (!valid) return;
-  const float inv = 1.f / l_run;
-  float* orow = a.o + (int64_t)(g.start + qpos) * a.o_st + (int64_t)h * a.o_sh + sub * EPL;
-#pragma unroll
-  for (int e = 0; e < EPL; e += 4)
-    *(f32x4*)&orow[e] = f32x4{acc[e] * inv, acc[e + 1] * inv, acc[e + 2] * inv, acc[e + 3] * inv};
-  if (sub == 0 && a.lse != nullptr)
-    a.lse[(int64_t)h * a.lse_sh + g.start + qpos] = m_run * a.scale + logf(l_run);
-}
-
-template <int D>
-__global__ __launch_bounds__(256) void delta_f32_kernel(const F32Args a) {
-  const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 2);
+__global__ __launch_bounds__(kThreads) void delta_f32_kernel(const F32Args a) {
+  const int64_t row = (int64_t)blockIdx.x * kDeltaRows + (threadIdx.x >> 2);
   const int sub = threadIdx.x & 3;
   const bool valid = row < (int64_t)a.T * a.Hq;
   const int t = valid ? (int)(row / a.Hq) : 0;
   const int h = valid ? (int)(row % a.Hq) : 0;
   float acc = 0.f;
   if (valid) {
-    const float* orow = a.out + (int64_t)t * a.o_st + (int64_t)h * a.o_sh + sub * (D / 4);
-    const float* drow = a.dout + (int64_t)t * a.do_st + (int64_t)h * a.do_sh + sub * (D / 4);
-    for (int e = 0; e < D / 4; ++e) acc = __builtin_fmaf(orow[e], drow[e], acc);
+    const float* orow = a.out + (int64_t)t * a.o_st + (int64_t)h * a.o_sh + 4 * sub;
+    const float* drow = a.dout + (int64_t)t * a.do_st + (int64_t)h * a.do_sh + 4 * sub;
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c) {
+      const f32x4 o = *(const f32x4*)&orow[16 * c], d = *(const f32x4*)&drow[16 * c];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_fmaf(o[e], d[e], acc);
+    }
   }
   acc = sum4(acc);
-  if (valid && sub == 0) a.delta[(int64_t)h * a.T + t] = acc;
+  if (valid && sub == 0) {
+    a.delta[(int64_t)h * a.T + t] = acc;
+    a.lse2[(int64_t)h * a.T + t] = a.olse[(int64_t)h * a.lse_sh + t] * kLog2e;
+  }
 }
 
+__device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
+// Keeps the instruction scheduler from moving the loads in front of it behind
+// the products (it otherwise sinks them to their use, which then waits for
+// memory: forward 26.5 -> 25.3 us).  Not in the backward, whose registers are
+// full (28 spilled with it, 85 -> 99 us).
+__device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(0); }
+
+// Row of accumulator register r in lane half hi.
+__device__ __forceinline__ constexpr int acc_row(int r, int hi) { return 8 * (r >> 2) + 4 * hi + (r & 3); }
+
+// LDS of a workgroup: up to two owned operands, later the partial sums of the
+// four waves.
 template <int D>
-__global__ __launch_bounds__(kThreads) void dq_f32_kernel(const F32Args a) {
-  constexpr int EPL = D / 4;
-  __shared__ __attribute__((aligned(16))) float sK[kTile * D];
-  __shared__ __attribute__((aligned(16))) float sV[kTile * D];
+struct Smem {
+  static constexpr int kStride = D + 4;
+  static constexpr int kTile = kRows * kStride;
+  float x[kWaves * kTile];
+  float m[kWaves][kRows], l[kWaves][kRows];
+};
+
+// One streamed 32-row tile of a [rows, D] fp32 matrix (row stride in elements).
+template <int D>
+struct Tile {
+  static constexpr int kChunks = D / 8;   // 16-byte reads per lane in row form
+  static constexpr int kCols = D / 32;    // columns per lane in column form
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ Tile(const float* base, int64_t stride, int row0, int nrows) {
+    const int left = min(kRows, nrows - row0);
+    r = make_rsrc(base + (int64_t)row0 * stride, left > 0 ? (uint32_t)(((left - 1) * stride + D) * 4) : 0u);
+  }
+  // Row form: lane = row lane % 32, columns 8 c + 4 hi .. + 3 in chunk c.
+  __device__ __forceinline__ void rows(f32x4 (&x)[kChunks], uint32_t lane_off) const {
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) x[c] = __builtin_bit_cast(f32x4, buf_load16(r, lane_off + 32 * c));
+  }
+  // Column form: step s holds row acc_row(s, hi), columns kCols * (lane % 32) + 0 ..
+  __device__ __forceinline__ void cols(float (&x)[16][kCols], uint32_t lane_off, uint32_t row_bytes) const {
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const int off = (int)(lane_off + acc_row(s, 0) * row_bytes);
+      if constexpr (kCols == 1) {
+        x[s][0] = buf_load_f32(r, off);
+      } else if constexpr (kCols == 2) {
+        const f32x2 t = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+        x[s][0] = t[0]; x[s][1] = t[1];
+      } else if constexpr (kCols == 3) {
+        const auto t = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 3; ++e) x[s][e] = __uint_as_float(t[e]);
+      } else {
+        const f32x4 t = __builtin_bit_cast(f32x4, buf_load16(r, off));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[s][e] = t[e];
+      }
+    }
+  }
+};
+
+// The lane's byte offsets into a tile in the two forms.
+template <int D>
+struct LaneOff {
+  uint32_t row, col, row_bytes;
+  __device__ __forceinline__ LaneOff(int64_t stride, int l32, int hi) {
+    row_bytes = (uint32_t)stride * 4u;
+    row = (uint32_t)l32 * row_bytes + 16u * hi;
+    col = 4u * hi * row_bytes + (uint32_t)(4 * (D / 32) * l32);
+  }
+};
+
+// The workgroup's 32 owned rows -> LDS; rows past nrows are zero.
+template <int D>
+__device__ __forceinline__ void stage_owned(float* dst, const float* base, int64_t stride, int row0, int nrows) {
+  constexpr int N = kRows * (D / 4) / kThreads;  // 16-byte units per thread
+  const Tile<D> t(base, stride, row0, nrows);
+  i32x4 v[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int i = threadIdx.x + j * kThreads, row = i / (D / 4), c = i % (D / 4);
+    v[j] = buf_load16(t.r, (uint32_t)(row * stride + 4 * c) * 4u);
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int i = threadIdx.x + j * kThreads, row = i / (D / 4), c = i % (D / 4);
+    *(i32x4*)&dst[row * Smem<D>::kStride + 4 * c] = v[j];
+  }
+}
+
+// X W^T for a streamed tile x in row form and the owned rows w in LDS: 32 x 32.
+template <int D>
+__device__ __forceinline__ f32x16 product_rows(const f32x4 (&x)[D / 8], const float* w, int l32, int hi) {
+  f32x16 acc = f32x16{};
+  const float* row = w + l32 * Smem<D>::kStride + 4 * hi;
+#pragma unroll
+  for (int c = 0; c < D / 8; ++c) {
+    const f32x4 b = *(const f32x4*)&row[8 * c];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = mfma_f32(x[c][e], b[e], acc);
+  }
+  return acc;
+}
+
+// acc[dt] += X^T P: X the streamed tile in column form, P [32 x 32] in accumulator
+// form.  acc[dt] row i is column D / 32 * i + dt of the result, its lane the owned row.
+template <int D>
+__device__ __forceinline__ void product_cols(f32x16 (&acc)[D / 32], const float (&x)[16][D / 32], f32x16 p) {
+#pragma unroll
+  for (int s = 0; s < 16; ++s)
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) acc[dt] = mfma_f32(x[s][dt], p[s], acc[dt]);
+}
+
+// This wave's partial result (row = owned row) -> its LDS region.
+template <int D>
+__device__ __forceinline__ void put_partial(float* dst, const f32x16 (&acc)[D / 32], float scale, int l32, int hi) {
+  constexpr int C = D / 32;
+  float* row = dst + l32 * Smem<D>::kStride;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {  // registers 4 g .. + 3: columns C * (8 g + 4 hi) .. + 4 C
+    float v[4 * C];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int dt = 0; dt < C; ++dt) v[e * C + dt] = acc[dt][4 * g + e] * scale;
+#pragma unroll
+    for (int e = 0; e < C; ++e)
+      *(f32x4*)&row[C * (8 * g + 4 * hi) + 4 * e] = f32x4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
+  }
+}
+
+// Sum of the four partials times `scale(row)` -> global rows row0 .. of [rows, D].
+template <int D, typename Scale>
+__device__ __forceinline__ void store_sum(const float* x, float* base, int64_t stride, int row0, int nrows,
+                                          Scale&& scale) {
+  using S = Smem<D>;
+  for (int i = threadIdx.x; i < kRows * (D / 4); i += kThreads) {
+    const int row = i / (D / 4), c = i % (D / 4);
+    if (row0 + row >= nrows) continue;
+    f32x4 t = *(const f32x4*)&x[row * S::kStride + 4 * c];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) t += *(const f32x4*)&x[w * S::kTile + row * S::kStride + 4 * c];
+    *(f32x4*)&base[(int64_t)(row0 + row) * stride + 4 * c] = t * scale(row);
+  }
+}
+
+struct Lanes {
+  int wave, l32, hi;
+  __device__ __forceinline__ Lanes() {
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    l32 = threadIdx.x & 31;
+    hi = (threadIdx.x >> 5) & 1;
+  }
+};
+
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(const F32Args a) {
+  constexpr int C = D / 32;
+  __shared__ __attribute__((aligned(16))) Smem<D> sm;
   const int h = blockIdx.x % a.Hq;
   const int s = blockIdx.x / a.Hq;
-  const int tile = a.num_tiles - 1 - (int)blockIdx.y;
+  const int tile = a.num_tiles - 1 - (int)blockIdx.y;  // heaviest first
   const SeqGeom g = load_seq<true>(a.cu_seqlens, a.prefix_lens, s, a.total_seqlen, a.is_causal, a.T);
-  const int m0 = tile * kRowsPerBlock;
+  const int m0 = tile * kRows;
   if (m0 >= g.nq) return;
   const int hk = h / a.group;
-  const int sub = threadIdx.x & 3;
-  const int qpos = m0 + (threadIdx.x >> 2);
-  const bool valid = qpos < g.nq;
-  const int kend = kend_of(g.p, qpos);
-  const int wg_kend = max(g.p, min(m0 + kRowsPerBlock, g.nq));
-
-  float qv[EPL], dov[EPL], acc[EPL];
-  load_row<D>(qv, a.q + (int64_t)(g.start + qpos) * a.q_st + (int64_t)h * a.q_sh, sub, valid);
-  load_row<D>(dov, a.dout + (int64_t)(g.start + qpos) * a.do_st + (int64_t)h * a.do_sh, sub, valid);
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
-  const float lse2 = valid ? a.olse[(int64_t)h * a.lse_sh + g.start + qpos] * kLog2e : 0.f;
-  const float dlt = valid ? a.delta[(int64_t)h * a.T + g.start + qpos] : 0.f;
+  const Lanes ln;
+  const int kend = kend_of(g.p, m0 + ln.l32);
+  const int n_tiles = (max(g.p, min(m0 + kRows, g.nq)) + kRows - 1) / kRows;
+  const int kend_min = max(g.p, m0 + 1);  // every row sees the keys before this one
   const float* kb = a.k + (int64_t)g.start * a.k_st + (int64_t)hk * a.k_sh;
   const float* vb = a.v + (int64_t)g.start * a.v_st + (int64_t)hk * a.v_sh;
+  const LaneOff<D> ko(a.k_st, ln.l32, ln.hi), vo(a.v_st, ln.l32, ln.hi);
 
-  for (int k0 = 0; k0 < wg_kend; k0 += kTile) {
-    __syncthreads();
-    stage<D>(sK, kb, a.k_st, k0, g.n);
-    stage<D>(sV, vb, a.v_st, k0, g.n);
-    __syncthreads();
-#pragma unroll 4
-    for (int j = 0; j < kTile; ++j) {
-      const float sc = dot_tile<D>(qv, &sK[j * D], sub);
-      const float dp = dot_tile<D>(dov, &sV[j * D], sub);
-      float pr = fast_exp2(__builtin_fmaf(sc, a.scale_log2, -lse2));
-      if (!valid || k0 + j >= kend) pr = 0.f;
-      const float ds = pr * (dp - dlt);
+  f32x4 kx[Tile<D>::kChunks];
+  float vx[16][C];
+  int kt = ln.wave;
+  if (kt < n_tiles) Tile<D>(kb, a.k_st, kt * kRows, g.n).rows(kx, ko.row);
+  stage_owned<D>(sm.x, a.q + (int64_t)g.start * a.q_st + (int64_t)h * a.q_sh, a.q_st, m0, g.nq);
+  __syncthreads();
+
+  f32x16 acc[C];
 #pragma unroll
-      for (int e = 0; e < EPL; e += 4) {
-        const f32x4 t = *(const f32x4*)&sK[j * D + sub * EPL + e];
-        acc[e] = __builtin_fmaf(ds, t[0], acc[e]);
-        acc[e + 1] = __builtin_fmaf(ds, t[1], acc[e + 1]);
-        acc[e + 2] = __builtin_fmaf(ds, t[2], acc[e + 2]);
-        acc[e + 3] = __builtin_fmaf(ds, t[3], acc[e + 3]);
-      }
+  for (int dt = 0; dt < C; ++dt) acc[dt] = f32x16{};
+  float m_run = -INFINITY, l_run = 0.f;
+  for (; kt < n_tiles; kt += kWaves) {
+    const int k0 = kt * kRows;
+    Tile<D>(vb, a.v_st, k0, g.n).cols(vx, vo.col, vo.row_bytes);
+    pin();
+    f32x16 st = product_rows<D>(kx, sm.x, ln.l32, ln.hi);
+    // the next tile's rows (none past the last: an empty range reads zeros)
+    Tile<D>(kb, a.k_st, k0 + kWaves * kRows, kt + kWaves < n_tiles ? g.n : 0).rows(kx, ko.row);
+    pin();
+    if (k0 + kRows > kend_min) {
+      __asm__ volatile("");
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (k0 + acc_row(r, ln.hi) >= kend) st[r] = -INFINITY;
     }
-  }
-  if (!valid) return;
-  float* drow = a.dq + (int64_t)(g.start + qpos) * a.dq_st + (int64_t)h * a.dq_sh + sub * EPL;
+    float mx = st[0];
 #pragma unroll
-  for (int e = 0; e < EPL; e += 4)
-    *(f32x4*)&drow[e] = f32x4{acc[e] * a.scale, acc[e + 1] * a.scale, acc[e + 2] * a.scale, acc[e + 3] * a.scale};
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, st[r]);
+    const float m_new = fmaxf(m_run, xor32_max(mx));
+    if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {  // else every factor is 1
+      const float alpha = m_run == -INFINITY ? 0.f : fast_exp2((m_run - m_new) * a.scale_log2);
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < C; ++dt) acc[dt] *= alpha;
+    }
+    const float mb = m_new == -INFINITY ? 0.f : m_new * a.scale_log2;  // -inf: no allowed key yet
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      st[r] = fast_exp2(__builtin_fmaf(st[r], a.scale_log2, -mb));
+      l_run += st[r];
+    }
+    m_run = m_new;
+    product_cols<D>(acc, vx, st);
+  }
+
+  // Merge: every wave scales its sums to the row's largest maximum.
+  const float l_tot = xor32_sum(l_run);
+  if (ln.hi == 0) {
+    sm.m[ln.wave][ln.l32] = m_run;
+    sm.l[ln.wave][ln.l32] = l_tot;
+  }
+  __syncthreads();  // also: every wave is done with the owned rows
+  float M = sm.m[0][ln.l32];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) M = fmaxf(M, sm.m[w][ln.l32]);
+  const float wt = m_run == -INFINITY ? 0.f : fast_exp2((m_run - M) * a.scale_log2);
+  put_partial<D>(sm.x + ln.wave * Smem<D>::kTile, acc, wt, ln.l32, ln.hi);
+  float l_sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const float m = sm.m[w][ln.l32];
+    l_sum += m == -INFINITY ? 0.f : sm.l[w][ln.l32] * fast_exp2((m - M) * a.scale_log2);
+  }
+  __syncthreads();
+  if (threadIdx.x < kRows) {
+    sm.l[0][threadIdx.x] = 1.f / l_sum;
+    if (m0 + (int)threadIdx.x < g.nq && a.lse != nullptr)
+      a.lse[(int64_t)h * a.lse_sh + g.start + m0 + threadIdx.x] = M * a.scale + logf(l_sum);
+  }
+  __syncthreads();
+  store_sum<D>(sm.x, a.o + (int64_t)g.start * a.o_st + (int64_t)h * a.o_sh, a.o_st, m0, g.nq,
+               [&](int row) { return sm.l[0][row]; });
 }
 
+// dQ of one (head, sequence, 32-query tile): dQ^T += K^T dS^T over the key tiles.
 template <int D>
-__global__ __launch_bounds__(kThreads) void dkdv_f32_kernel(const F32Args a) {
-  constexpr int EPL = D / 4;
-  __shared__ __attribute__((aligned(16))) float sQ[kTile * D];
-  __shared__ __attribute__((aligned(16))) float sO[kTile * D];
-  __shared__ float sL[kTile];
-  __shared__ float sD[kTile];
-  const int hk = blockIdx.x % a.Hkv;
-  const int s = blockIdx.x / a.Hkv;
-  const int tile = blockIdx.y;
+__device__ __forceinline__ void dq_body(const F32Args& a, Smem<D>& sm, int h, int s, int tile) {
+  constexpr int C = D / 32;
   const SeqGeom g = load_seq<true>(a.cu_seqlens, a.prefix_lens, s, a.total_seqlen, a.is_causal, a.T);
-  const int k0 = tile * kRowsPerBlock;
+  const int m0 = tile * kRows;
+  if (m0 >= g.nq) return;
+  const int hk = h / a.group;
+  const Lanes ln;
+  const int qpos = m0 + ln.l32;
+  const bool valid = qpos < g.nq;
+  const int kend = valid ? kend_of(g.p, qpos) : 0;
+  const int n_tiles = (max(g.p, min(m0 + kRows, g.nq)) + kRows - 1) / kRows;
+  const int kend_min = m0 + kRows <= g.nq ? max(g.p, m0 + 1) : 0;
+  const float* kb = a.k + (int64_t)g.start * a.k_st + (int64_t)hk * a.k_sh;
+  const float* vb = a.v + (int64_t)g.start * a.v_st + (int64_t)hk * a.v_sh;
+  const LaneOff<D> ko(a.k_st, ln.l32, ln.hi), vo(a.v_st, ln.l32, ln.hi);
+
+  f32x4 kx[Tile<D>::kChunks], vx[Tile<D>::kChunks];
+  float kc[16][C];
+  int kt = ln.wave;
+  {
+    const int n = kt < n_tiles ? g.n : 0;
+    Tile<D>(kb, a.k_st, kt * kRows, n).rows(kx, ko.row);
+    Tile<D>(vb, a.v_st, kt * kRows, n).rows(vx, vo.row);
+  }
+  const float lse2 = valid ? a.lse2[(int64_t)h * a.T + g.start + qpos] : 0.f;
+  const float dlt = valid ? a.delta[(int64_t)h * a.T + g.start + qpos] : 0.f;
+  float* const sq = sm.x;
+  float* const sdo = sm.x + Smem<D>::kTile;
+  stage_owned<D>(sq, a.q + (int64_t)g.start * a.q_st + (int64_t)h * a.q_sh, a.q_st, m0, g.nq);
+  stage_owned<D>(sdo, a.dout + (int64_t)g.start * a.do_st + (int64_t)h * a.do_sh, a.do_st, m0, g.nq);
+  __syncthreads();
+
+  f32x16 acc[C];
+#pragma unroll
+  for (int dt = 0; dt < C; ++dt) acc[dt] = f32x16{};
+  for (; kt < n_tiles; kt += kWaves) {
+    const int k0 = kt * kRows;
+    const int n_next = kt + kWaves < n_tiles ? g.n : 0;
+    Tile<D>(kb, a.k_st, k0, g.n).cols(kc, ko.col, ko.row_bytes);
+    f32x16 st = product_rows<D>(kx, sq, ln.l32, ln.hi);
+    Tile<D>(kb, a.k_st, k0 + kWaves * kRows, n_next).rows(kx, ko.row);
+    const f32x16 dp = product_rows<D>(vx, sdo, ln.l32, ln.hi);
+    Tile<D>(vb, a.v_st, k0 + kWaves * kRows, n_next).rows(vx, vo.row);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st[r] = fast_exp2(__builtin_fmaf(st[r], a.scale_log2, -lse2));
+    if (k0 + kRows > kend_min) {
+      __asm__ volatile("");
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (k0 + acc_row(r, ln.hi) >= kend) st[r] = 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st[r] *= dp[r] - dlt;
+    product_cols<D>(acc, kc, st);
+  }
+  __syncthreads();  // every wave is done with the owned rows
+  put_partial<D>(sm.x + ln.wave * Smem<D>::kTile, acc, a.scale, ln.l32, ln.hi);
+  __syncthreads();
+  store_sum<D>(sm.x, a.dq + (int64_t)g.start * a.dq_st + (int64_t)h * a.dq_sh, a.dq_st, m0, g.nq,
+               [](int) { return 1.f; });
+}
+
+// dK and dV of one (kv head, sequence, 32-key tile): the waves take the (q head,
+// 32-query tile) steps in turn; dV^T += dO^T P, dK^T += Q^T dS.
+template <int D>
+__device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk, int s, int tile) {
+  constexpr int C = D / 32;
+  const SeqGeom g = load_seq<true>(a.cu_seqlens, a.prefix_lens, s, a.total_seqlen, a.is_causal, a.T);
+  const int k0 = tile * kRows;
   if (k0 >= g.n) return;
-  const int sub = threadIdx.x & 3;
-  const int kpos = k0 + (threadIdx.x >> 2);
+  const Lanes ln;
+  const int kpos = k0 + ln.l32;
   const bool valid = kpos < g.n;
-  const int qs = qstart_of(g.p, kpos);
-  const int q_begin = qstart_of(g.p, k0);
+  const int qs = valid ? qstart_of(g.p, kpos) : 0x7fffffff;
+  const int qs_max = k0 + kRows <= g.n ? (k0 + kRows <= g.p ? 0 : k0 + kRows - 1) : 0x7fffffff;
+  const int t0 = qstart_of(g.p, k0) / kRows;                      // first query tile with an attended pair
+  const int n_q = max((g.nq + kRows - 1) / kRows - t0, 0);        // query tiles per head
+  const int steps = n_q * a.group;
+  const float* qb = a.q + (int64_t)g.start * a.q_st + (int64_t)hk * a.group * a.q_sh;
+  const float* ob = a.dout + (int64_t)g.start * a.do_st + (int64_t)hk * a.group * a.do_sh;
+  const LaneOff<D> qo(a.q_st, ln.l32, ln.hi), oo(a.do_st, ln.l32, ln.hi);
 
-  float kv[EPL], vv[EPL], dka[EPL], dva[EPL];
-  load_row<D>(kv, a.k + (int64_t)(g.start + kpos) * a.k_st + (int64_t)hk * a.k_sh, sub, valid);
-  load_row<D>(vv, a.v + (int64_t)(g.start + kpos) * a.v_st + (int64_t)hk * a.v_sh, sub, valid);
+  f32x4 qx[Tile<D>::kChunks], ox[Tile<D>::kChunks];
+  float qc[16][C], oc[16][C];
+  // this wave's step: q head `hh` of the group and query tile t0 + t; advanced by kWaves
+  int hh = 0, t = ln.wave;
+  auto wrap = [&]() __attribute__((always_inline)) {
+    while (hh < a.group && t >= n_q) { t -= n_q; ++hh; }
+  };
+  auto tile_of = [&](const float* base, int64_t st, int64_t sh) __attribute__((always_inline)) {
+    return Tile<D>(base + (int64_t)min(hh, a.group - 1) * sh, st, (t0 + t) * kRows, hh < a.group ? g.nq : 0);
+  };
+  if (steps > 0) {
+    wrap();
+    tile_of(qb, a.q_st, a.q_sh).rows(qx, qo.row);
+    tile_of(ob, a.do_st, a.do_sh).rows(ox, oo.row);
+  }
+  float* const sk = sm.x;
+  float* const sv = sm.x + Smem<D>::kTile;
+  stage_owned<D>(sk, a.k + (int64_t)g.start * a.k_st + (int64_t)hk * a.k_sh, a.k_st, k0, g.n);
+  stage_owned<D>(sv, a.v + (int64_t)g.start * a.v_st + (int64_t)hk * a.v_sh, a.v_st, k0, g.n);
+  __syncthreads();
+
+  f32x16 dka[C], dva[C];
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) { dka[e] = 0.f; dva[e] = 0.f; }
-
-  for (int hh = 0; hh < a.group; ++hh) {
+  for (int dt = 0; dt < C; ++dt) dka[dt] = dva[dt] = f32x16{};
+  for (int it = ln.wave; it < steps; it += kWaves) {
+    const int q0 = (t0 + t) * kRows;
     const int h = hk * a.group + hh;
-    const float* qb = a.q + (int64_t)g.start * a.q_st + (int64_t)h * a.q_sh;
-    const float* ob = a.dout + (int64_t)g.start * a.do_st + (int64_t)h * a.do_sh;
-    for (int q0 = q_begin; q0 < g.nq; q0 += kTile) {
-      __syncthreads();
-      stage<D>(sQ, qb, a.q_st, q0, g.nq);
-      stage<D>(sO, ob, a.do_st, q0, g.nq);
-      if (threadIdx.x < kTile) {
-        const int qr = q0 + threadIdx.x;
-        const bool ok = qr < g.nq;
-        sL[threadIdx.x] = ok ? a.olse[(int64_t)h * a.lse_sh + g.start + qr] * kLog2e : 0.f;
-        sD[threadIdx.x] = ok ? a.delta[(int64_t)h * a.T + g.start + qr] : 0.f;
-      }
-      __syncthreads();
-#pragma unroll 4
-      for (int i = 0; i < kTile; ++i) {
-        const int qp = q0 + i;
-        const float sc = dot_tile<D>(kv, &sQ[i * D], sub);
-        const float dp = dot_tile<D>(vv, &sO[i * D], sub);
-        float pr = fast_exp2(__builtin_fmaf(sc, a.scale_log2, -sL[i]));
-        if (!valid || qp < qs || qp >= g.nq) pr = 0.f;
-        const float ds = pr * (dp - sD[i]);
+    const Tile<D> qt = tile_of(qb, a.q_st, a.q_sh), ot = tile_of(ob, a.do_st, a.do_sh);
+    ot.cols(oc, oo.col, oo.row_bytes);
+    // Rows of the tile past the last query are read too (other rows, or the
+    // workspace section behind the array) and masked below.
+    const f32x4u* const lp = (const f32x4u*)(a.lse2 + (int64_t)h * a.T + g.start + q0 + 4 * ln.hi);
+    const f32x4u* const dp = (const f32x4u*)(a.delta + (int64_t)h * a.T + g.start + q0 + 4 * ln.hi);
+    f32x4 lse[4], dlt[4];
 #pragma unroll
-        for (int e = 0; e < EPL; e += 4) {
-          const f32x4 tq = *(const f32x4*)&sQ[i * D + sub * EPL + e];
-          const f32x4 to = *(const f32x4*)&sO[i * D + sub * EPL + e];
-          dva[e] = __builtin_fmaf(pr, to[0], dva[e]);
-          dva[e + 1] = __builtin_fmaf(pr, to[1], dva[e + 1]);
-          dva[e + 2] = __builtin_fmaf(pr, to[2], dva[e + 2]);
-          dva[e + 3] = __builtin_fmaf(pr, to[3], dva[e + 3]);
-          dka[e] = __builtin_fmaf(ds, tq[0], dka[e]);
-          dka[e + 1] = __builtin_fmaf(ds, tq[1], dka[e + 1]);
-          dka[e + 2] = __builtin_fmaf(ds, tq[2], dka[e + 2]);
-          dka[e + 3] = __builtin_fmaf(ds, tq[3], dka[e + 3]);
-        }
+    for (int e = 0; e < 4; ++e) lse[e] = lp[2 * e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dlt[e] = dp[2 * e];
+    t += kWaves;
+    wrap();
+    f32x16 p = product_rows<D>(qx, sk, ln.l32, ln.hi);
+    qt.cols(qc, qo.col, qo.row_bytes);
+    f32x16 ds = product_rows<D>(ox, sv, ln.l32, ln.hi);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      p[r] = fast_exp2(__builtin_fmaf(p[r], a.scale_log2, -lse[r >> 2][r & 3]));
+      ds[r] = p[r] * (ds[r] - dlt[r >> 2][r & 3]);
+    }
+    if (q0 < qs_max || q0 + kRows > g.nq) {
+      __asm__ volatile("");
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int qp = q0 + acc_row(r, ln.hi);
+        if (qp < qs || qp >= g.nq) p[r] = ds[r] = 0.f;
       }
     }
+    product_cols<D>(dva, oc, p);
+    tile_of(qb, a.q_st, a.q_sh).rows(qx, qo.row);
+    product_cols<D>(dka, qc, ds);
+    tile_of(ob, a.do_st, a.do_sh).rows(ox, oo.row);
   }
-  if (!valid) return;
-  float* krow = a.dk + (int64_t)(g.start + kpos) * a.dk_st + (int64_t)hk * a.dk_sh + sub * EPL;
-  float* vrow = a.dv + (int64_t)(g.start + kpos) * a.dv_st + (int64_t)hk * a.dv_sh + sub * EPL;
-#pragma unroll
-  for (int e = 0; e < EPL; e += 4) {
-    *(f32x4*)&krow[e] = f32x4{dka[e] * a.scale, dka[e + 1] * a.scale, dka[e + 2] * a.scale, dka[e + 3] * a.scale};
-    *(f32x4*)&vrow[e] = f32x4{dva[e], dva[e + 1], dva[e + 2], dva[e + 3]};
-  }
+  const float* const base = sm.x;
+  float* const mine = sm.x + ln.wave * Smem<D>::kTile;
+  __syncthreads();  // every wave is done with the owned rows
+  put_partial<D>(mine, dva, 1.f, ln.l32, ln.hi);
+  __syncthreads();
+  store_sum<D>(base, a.dv + (int64_t)g.start * a.dv_st + (int64_t)hk * a.dv_sh, a.dv_st, k0, g.n,
+               [](int) { return 1.f; });
+  __syncthreads();
+  put_partial<D>(mine, dka, a.scale, ln.l32, ln.hi);
+  __syncthreads();
+  store_sum<D>(base, a.dk + (int64_t)g.start * a.dk_st + (int64_t)hk * a.dk_sh, a.dk_st, k0, g.n,
+               [](int) { return 1.f; });
+}
+
+// dK / dV units, then dQ units, in one launch: independent work, and the lighter
+// dQ units fill the end of the dK / dV ones (4 x 512 tokens, 8 heads, head_dim
+// 64: 78 us; the two interleaved tile by tile 85).  blockIdx.x: (sequence, kv
+// head); blockIdx.y: the tile, heaviest first (the first key tiles, the last
+// query tiles); blockIdx.z + z0: 0 for dK / dV, 1 + q head of the group for dQ.
+// Workgroups are dealt round-robin to the XCDs and, inside one, to its shader
+// engines, whether or not the next one has room, so the sequences rotate by one
+// per row of tiles: a long or prefix-heavy one then does not land on one engine
+// while the others idle (78 -> 76.7 us).
+template <int D>
+__global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void bwd_f32_kernel(const F32Args a) {
+  __shared__ __attribute__((aligned(16))) Smem<D> sm;
+  const int hk = blockIdx.x % a.Hkv, y = blockIdx.y;
+  const int s = (int)(blockIdx.x / a.Hkv + y) % a.numseqs;
+  const int z = blockIdx.z + a.z0;
+  if (z == 0)
+    dkdv_body<D>(a, sm, hk, s, y);
+  else
+    dq_body<D>(a, sm, hk * a.group + z - 1, s, a.num_tiles - 1 - y);
 }
 
 F32Args common_args(int T, int Hq, int Hkv, int total_seqlen, int is_causal, float scale,
@@ -391,7 +560,8 @@ hipError_t launch_fwd(const MimirPrefixLMFwdParams& p, hipStream_t stream) {
   a.v_st = p.v_stride_token; a.v_sh = p.v_stride_head;
   a.o_st = p.out_stride_token; a.o_sh = p.out_stride_head;
   a.lse_sh = p.lse_stride_head;
-  a.num_tiles = (p.max_seqlen_all + kFwdRows - 1) / kFwdRows;
+  a.num_tiles = (p.max_seqlen_all + kRows - 1) / kRows;
+  a.numseqs = p.numseqs;
   if (a.num_tiles == 0 || p.numseqs == 0) return hipSuccess;
   hipLaunchKernelGGL(fwd_f32_kernel<D>, dim3(p.num_q_heads * p.numseqs, a.num_tiles), dim3(kThreads), 0,
                      stream, a);
@@ -405,7 +575,9 @@ hipError_t launch_bwd(const MimirPrefixLMBwdParams& p, hipStream_t stream, int s
   a.q = (const float*)p.q; a.k = (const float*)p.k; a.v = (const float*)p.v;
   a.out = (const float*)p.out; a.dout = (const float*)p.dout; a.olse = p.lse;
   a.dq = (float*)p.dq; a.dk = (float*)p.dk; a.dv = (float*)p.dv;
-  a.delta = (float*)p.workspace;
+  const BwdWorkspace ws = bwd_workspace_layout(p.total_tokens, p.num_q_heads, p.numseqs, p.max_seqlen_all);
+  a.delta = (float*)((char*)p.workspace + ws.delta);
+  a.lse2 = (float*)((char*)p.workspace + ws.lse2);
   a.q_st = p.q_stride_token; a.q_sh = p.q_stride_head;
   a.k_st = p.k_stride_token; a.k_sh = p.k_stride_head;
   a.v_st = p.v_stride_token; a.v_sh = p.v_stride_head;
@@ -415,19 +587,17 @@ hipError_t launch_bwd(const MimirPrefixLMBwdParams& p, hipStream_t stream, int s
   a.dk_st = p.dk_stride_token; a.dk_sh = p.dk_stride_head;
   a.dv_st = p.dv_stride_token; a.dv_sh = p.dv_stride_head;
   a.lse_sh = p.lse_stride_head;
-  a.num_tiles = (p.max_seqlen_all + kRowsPerBlock - 1) / kRowsPerBlock;
+  a.num_tiles = (p.max_seqlen_all + kRows - 1) / kRows;
+  a.numseqs = p.numseqs;
   const int64_t rows = (int64_t)p.total_tokens * p.num_q_heads;
   if (rows > 0 && (stages & MIMIR_BWD_STAGE_DELTA))
-    hipLaunchKernelGGL(delta_f32_kernel<D>, dim3((unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock)),
-                       dim3(256), 0, stream, a);
-  if (a.num_tiles > 0 && p.numseqs > 0) {
-    if (stages & MIMIR_BWD_STAGE_DQ)
-      hipLaunchKernelGGL(dq_f32_kernel<D>, dim3(p.num_q_heads * p.numseqs, a.num_tiles), dim3(kThreads), 0,
-                         stream, a);
-    if (stages & MIMIR_BWD_STAGE_DKDV)
-      hipLaunchKernelGGL(dkdv_f32_kernel<D>, dim3(p.num_kv_heads * p.numseqs, a.num_tiles), dim3(kThreads), 0,
-                         stream, a);
-  }
+    hipLaunchKernelGGL(delta_f32_kernel<D>, dim3((unsigned)((rows + kDeltaRows - 1) / kDeltaRows)),
+                       dim3(kThreads), 0, stream, a);
+  a.z0 = stages & MIMIR_BWD_STAGE_DKDV ? 0 : 1;
+  const int z1 = stages & MIMIR_BWD_STAGE_DQ ? 1 + a.group : 1;
+  if (a.num_tiles > 0 && p.numseqs > 0 && z1 > a.z0)
+    hipLaunchKernelGGL(bwd_f32_kernel<D>, dim3(p.num_kv_heads * p.numseqs, a.num_tiles, z1 - a.z0), dim3(kThreads), 0,
+                       stream, a);
   return hipGetLastError();
 }
 

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void gate_fwd_f32_kernel(const GateArgs a) {
 
 // float32 gate backward, one thread per (token, head) row: dout_s = dout * s
 // (the attention's upstream gradient, contiguous [T, H, D]), delta = rowsum(dout_s * O)
-// ([H, T]) and dgate = (dout * O) * (1 - s) * s.
+// and lse2 = lse * log2(e) (both [H, T]) and dgate = (dout * O) * (1 - s) * s.
 struct GateBwdArgs {
   const float* o;
   const float* dy;
@@ -124,7 +124,9 @@ struct GateBwdArgs {
   float* dgate;
   float* dout_s;
   float* delta;
-  int64_t o_st, o_sh, dy_st, dy_sh, g_st, g_sh, dg_st, dg_sh;
+  const float* lse;
+  float* lse2;
+  int64_t o_st, o_sh, dy_st, dy_sh, g_st, g_sh, dg_st, dg_sh, lse_sh;
   int T, H, D;
 };
 
@@ -148,6 +150,7 @@ __global__ __launch_bounds__(256) void gate_bwd_f32_kernel(const GateBwdArgs a) 
       acc += dso * o[d];
     }
     a.delta[(int64_t)h * a.T + t] = acc;
+    a.lse2[(int64_t)h * a.T + t] = a.lse[(int64_t)h * a.lse_sh + t] * kLog2e;
   }
 }
 
@@ -198,7 +201,8 @@ hipError_t launch_gate_fwd_f32(const MimirPrefixLMFwdParams& p, hipStream_t stre
   return hipGetLastError();
 }
 
-hipError_t launch_gate_bwd_f32(const MimirPrefixLMBwdParams& p, float* dout_s, float* delta, hipStream_t stream) {
+hipError_t launch_gate_bwd_f32(const MimirPrefixLMBwdParams& p, float* dout_s, float* delta, float* lse2,
+                               hipStream_t stream) {
   GateBwdArgs a;
   a.o = (const float*)p.out;
   a.dy = (const float*)p.dout;
@@ -206,6 +210,9 @@ hipError_t launch_gate_bwd_f32(const MimirPrefixLMBwdParams& p, float* dout_s, f
   a.dgate = (float*)p.dgate;
   a.dout_s = dout_s;
   a.delta = delta;
+  a.lse = p.lse;
+  a.lse2 = lse2;
+  a.lse_sh = p.lse_stride_head;
   a.o_st = p.out_stride_token; a.o_sh = p.out_stride_head;
   a.dy_st = p.dout_stride_token; a.dy_sh = p.dout_stride_head;
   a.g_st = p.gate_stride_token; a.g_sh = p.gate_stride_head;

@@ -194,6 +194,30 @@ def test_f32_small(device, idx):
     check(case, device, label=f"f32small{idx}")
 
 
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+@pytest.mark.parametrize("hq,hkv,causal", [(3, 3, False), (6, 2, False), (4, 1, True)])
+def test_f32_tile_edges(device, d, hq, hkv, causal):
+    """Lengths around the 32-row tiles and the four waves' turns of them (128 rows), prefixes on
+    and off tile boundaries, a total_seqlen inside the last sequence, and q / k / v as strided
+    slices of one projection: the fp32 bar, and bitwise the contiguous result."""
+    seq_lens = [1, 31, 32, 33, 127, 128, 129, 161, 40]
+    prefixes = [1, 0, 32, 7, 96, 128, 5, 33, 40]
+    case = make_case(seq_lens, prefixes, hq, hkv, d, seed=d + hq, dtype=torch.float32, pad_to=sum(seq_lens) + 5,
+                     is_causal=causal)
+    case.total_seqlen = torch.tensor(sum(seq_lens) - 21)
+    got = check(case, device, label=f"f32 tiles d{d}")
+    c = case.to(device)
+    fused = torch.randn((c.T, hq + 2 * hkv, d), device=device)
+    views = fused.split((hq, hkv, hkv), dim=1)
+    for dst, src in zip(views, (c.q, c.k, c.v)):
+        dst.copy_(src)
+    leaves = [x.detach().requires_grad_(True) for x in views]
+    out, lse = prefixlm_attn_fwd(*leaves, causal, *c.oracle_args()[:5], c.max_seqlen_all)
+    grads = torch.autograd.grad(out, leaves, c.dout)
+    for name, x in zip(("o", "lse", "dq", "dk", "dv"), (out, lse, *grads)):
+        assert torch.equal(x.detach().cpu(), got[name]), name
+
+
 def test_config1_fp32_forward(device):
     case = make_config(1, seed=0)
     check(case, device, backward=False, label="cfg1")
