@@ -6,21 +6,21 @@
 // (and j <= cache_lengths[b] + i when causal).  The reference materializes the
 // repeated K/V heads and a [B, S, max_kv_len] mask for SDPA; here:
 //
-//   cache_append_kernel   the scatter of k_new / v_new into the cache rows (it
-//                         also clears the split arrival counters)
-//   cache_attn_kernel     one workgroup per (batch row, kv head, 128 query rows,
-//                         key split): the G query heads of a kv head share its
-//                         K / V tiles (rows are (token, head) pairs, token-major),
-//                         64-key tiles stream through two LDS stages, S^T = K Q^T
-//                         and O^T += V^T P^T on bf16 MFMA with an online softmax
-//                         (the forward kernel's arithmetic).  With several
-//                         splits, each publishes its partial (max, sum, O) rows
-//                         and the last to arrive merges them into the output.
-//
-// Decode (S = 1) has only G rows per kv head, so each batch row's key range is
-// split evenly over enough workgroups to cover the chip (flash-decoding); the
-// kernel is then bound by the HBM read of the cache.  Prefill with a long S
-// fills the row tiles and runs on the MFMA like the forward kernel.
+//   decode (at most 32 query rows per kv head, e.g. S = 1):
+//     cache_decode_*_kernel  appends the new rows and attends, each workgroup an
+//                            equal share of all key tiles of the call
+//     cache_merge_kernel     adds the partial rows of the shares
+//   otherwise:
+//     cache_append_kernel    the scatter of k_new / v_new into the cache rows (it
+//                            also clears the split arrival counters)
+//     cache_attn_kernel      one workgroup per (batch row, kv head, 128 query rows,
+//                            key split): the G query heads of a kv head share its
+//                            K / V tiles (rows are (token, head) pairs, token-major),
+//                            64-key tiles stream through two LDS stages, S^T = K Q^T
+//                            and O^T += V^T P^T on bf16 MFMA with an online softmax
+//                            (the forward kernel's arithmetic).  With several
+//                            splits, each publishes its partial (max, sum, O) rows
+//                            and the last to arrive merges them into the output.
 #include "prefixlm_common.h"
 
 namespace mimir {
@@ -52,6 +52,7 @@ struct CacheArgs {
   float* part_ml;  // [unit, kRows, 2]: running max (exp2 domain) and sum
   int* counters;   // [B * Hkv * n_rt] split arrivals per row tile (splits > 1), cleared by the append kernel
   int n_counters;
+  int shares;      // decode: workgroups the key tiles of the call are dealt to
 };
 
 __device__ __forceinline__ int64_t load_index(const void* p, int i, int idx64) {
@@ -375,16 +376,44 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
 }
 
 // ---------------------------------------------------------------------------
-// Decode: at most 32 query rows per kv head (S * G <= 32, e.g. S = 1).  The
-// rows fit one wave, so instead of sharing 64-key tiles behind workgroup
-// barriers, each of the four waves streams its own 32-key tiles of the split
-// (tiles t0 + w, t0 + w + 4, ...) through two LDS stages of its own and waits
-// only for its own copies: four independent copy pipelines per workgroup, one
-// workgroup per CU.  The waves' partial rows are merged through LDS, and the
-// splits of a batch row through memory as in cache_attn_kernel.
+// Decode: at most 32 query rows per kv head (R = S * G <= 32, e.g. S = 1); bound
+// by the read of the cache, and for a few rows by the chain of memory round
+// trips.  The 32-key tiles of all (batch row, kv head) pairs form one line,
+// batch rows outermost; every workgroup takes an equal share of it (at least
+// kMinShare tiles), so rows of very different lengths keep all CUs busy to the
+// end.  A share covers one or more segments (tiles of one pair).  The rows of a
+// segment fit one wave, so instead of sharing 64-key tiles behind workgroup
+// barriers, each of the four waves streams its own tiles of the segment through
+// two LDS stages of its own and waits only for its own copies: four independent
+// copy pipelines per workgroup, one workgroup per CU.  The waves' partial rows
+// are merged through LDS.  A pair inside one share is finished there; the parts
+// of the others go to the workspace and cache_merge_kernel adds them.  A second
+// kernel needs no arrival counters, whose clearing took a launch of its own, and
+// no device-coherent round trips: merging in the last share to arrive (flags with
+// a value of the call's own instead of counters) left one launch, but 12.5 us of
+// it instead of 7.4 + 4.4 for one row and 22.5 instead of 12.6 + 4.3 for eight.
+//
+// The new rows are appended here too: the wave whose tile holds one stores it to
+// the cache and to its LDS copy of the tile.  Batch rows that share a cache row
+// see each other's new rows as if all had been appended first: the tile copy is
+// overlaid with the new rows of every batch row of the same cache row.
+//
+// Measured against an append kernel, one workgroup of four waves per (pair, equal
+// split) and a counted merge in it (Hq 16, Hkv 4, D 128): 64 rows of 512 to 8000 keys
+// 138 -> 119 us (5.0 TB/s), 32 rows of 100 to 4000 41 -> 33, one row of 8000 24 -> 15;
+// 8 rows of 1000 to 3600 18.2 -> 17.7, of which the two launches and their chains of
+// round trips (lengths, tiles, parts) are 9.
 // ---------------------------------------------------------------------------
 constexpr int kDecKeys = 32;  // keys per wave tile
 constexpr int kDecRows = 32;  // query rows of the decode kernel (one wave's columns)
+// Shares of the line: two waves and two workgroups per CU, whose starts and ends
+// overlap; a unit of the line is both stages of every wave.
+constexpr int kShareWaves = 2;
+constexpr int kShareUnit = 2 * kShareWaves;
+// One workgroup per pair: four waves, one workgroup per CU, a unit is all tiles of a
+// pair, so every pair is whole and nothing is left to merge.
+constexpr int kPairWaves = 4;
+constexpr int kPairUnit = 1 << 24;
 
 template <int D>
 struct DecTile {
@@ -401,20 +430,94 @@ __device__ __forceinline__ void wait_vmcnt_wide() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
 }
 
-template <int D>
+// Workgroup barrier for LDS data alone: unlike __syncthreads(), tile copies and
+// stores stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __asm__ volatile("" ::: "memory");
+  wait_lds();
+  __builtin_amdgcn_s_barrier();
+  __asm__ volatile("" ::: "memory");
+}
+
+// Inclusive sum over the wave's lanes (DPP adds; LDS-permute shuffles would cost
+// six LDS round trips before the first copy).
+__device__ __forceinline__ int wave_inclusive_sum(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
+// The line of key tiles, in units of kUnit tiles, as one wave sees it: 64 batch
+// rows at a time, one per lane.
+template <int kUnit>
+struct TileLine {
+  int first;  // batch row of lane 0
+  int pos;    // position of the lane's batch row: cache_lengths clamped to [-S, L] (new row i goes to pos + i)
+  int row;    // its cache row, -1 outside the cache
+  int keys;   // keys it attends: cached and new ones inside the cache
+  int units;  // units per kv head
+  int incl;   // units per kv head of all batch rows up to this one
+  __device__ __forceinline__ void load(const CacheArgs& a, int first_, int before, int lane) {
+    first = first_;
+    const int b = first + lane;
+    row = -1;
+    pos = keys = 0;
+    if (b < a.B) {
+      const int64_t n = load_index(a.cache_lengths, b, a.idx64), r = cache_row(a, b);
+      pos = n < -(int64_t)a.S ? -a.S : (n > a.L ? a.L : (int)n);
+      row = r >= 0 && r < a.rows ? (int)r : -1;
+      keys = row >= 0 ? min(max(pos, 0) + a.S, a.L) : 0;
+    }
+    units = ((keys + kDecKeys - 1) / kDecKeys + kUnit - 1) / kUnit;
+    incl = before + wave_inclusive_sum(units);
+  }
+  __device__ __forceinline__ int end() const { return __builtin_amdgcn_readlane(incl, 63); }
+};
+
+// Units per share for a line of `total` units.
+__device__ __forceinline__ int share_of(const CacheArgs& a, int total) {
+  return max(1, (total + a.shares - 1) / a.shares);
+}
+// Part slot (of two per share) of the segment that starts at position u of the line.
+__device__ __forceinline__ int part_slot(int u, int per) { return 2 * (u / per) + (u % per != 0); }
+
+// Zero output for the batch rows without keys (outside the cache) among the
+// loaded ones, dealt to the workgroups.
+template <int D, int kUnit>
+__device__ __forceinline__ void zero_keyless(const CacheArgs& a, const TileLine<kUnit>& line, int lane) {
+  uint64_t none = __builtin_amdgcn_ballot_w64(line.first + lane < a.B && line.keys == 0);
+  for (; none != 0; none &= none - 1) {
+    const int b = line.first + __builtin_ctzll(none);
+    if (b % (int)gridDim.x != (int)blockIdx.x) continue;
+    const int Hq = a.Hkv * a.G;
+    for (int i = threadIdx.x; i < a.S * Hq * (D / 8); i += blockDim.x) {
+      const int c = i % (D / 8), row = i / (D / 8);
+      *(bf16x8*)&a.out[(int64_t)b * a.o_sb + (int64_t)(row / Hq) * a.o_st + (int64_t)(row % Hq) * a.o_sh + c * 8] =
+          bf16x8{};
+    }
+  }
+}
+
+template <int D, int kDecWaves, int kUnit>
 __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   constexpr int DT = D / 32;
   constexpr int KS = D / 16;
   using L = TileLayout<D>;
   using T = DecTile<D>;
-  // two stages of (K, V) per wave; each stage array holds the four waves' tiles
-  __shared__ __attribute__((aligned(16))) bf16_t sK0[kWaves * T::kElems];
-  __shared__ __attribute__((aligned(16))) bf16_t sV0[kWaves * T::kElems];
-  __shared__ __attribute__((aligned(16))) bf16_t sK1[kWaves * T::kElems];
-  __shared__ __attribute__((aligned(16))) bf16_t sV1[kWaves * T::kElems];
-  __shared__ __attribute__((aligned(16))) float sMl[kWaves][kDecRows][2];  // per wave and row: max (exp2), sum
-  static_assert(2 * kDecRows * D * 4 <= kWaves * T::kElems * 2, "two waves' partial O fit one stage array");
-  __shared__ int last;
+  // two stages of (K, V) per wave; each stage array holds all waves' tiles
+  __shared__ __attribute__((aligned(16))) bf16_t sK0[kDecWaves * T::kElems];
+  __shared__ __attribute__((aligned(16))) bf16_t sV0[kDecWaves * T::kElems];
+  __shared__ __attribute__((aligned(16))) bf16_t sK1[kDecWaves * T::kElems];
+  __shared__ __attribute__((aligned(16))) bf16_t sV1[kDecWaves * T::kElems];
+  __shared__ __attribute__((aligned(16))) float sMl[kDecWaves][kDecRows][2];  // per wave and row: max (exp2), sum
+  // the waves' partial O, kMergeRows rows at a time (two workgroups share the
+  // CU's 160 KiB); a padded row keeps the rows in distinct banks
+  constexpr int kMergeRows = D == 128 ? 4 : 8;
+  __shared__ __attribute__((aligned(16))) float sO[kDecWaves][kMergeRows][D + 4];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -422,58 +525,121 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   const int l32 = lane & 31;
   const int hi = lane >> 5;
 
-  const int split = blockIdx.x % a.splits;
-  const int group = blockIdx.x / a.splits;  // (batch row, kv head); one row tile
-  const int hk = group % a.Hkv;
-  const int b = group / a.Hkv;
-  const int64_t crow = cache_row(a, b);
-  const bool row_in_cache = crow >= 0 && crow < a.rows;
-  const int clen = cache_len_of(a, b);
-  const int kv = row_in_cache ? min(clen + a.S, a.L) : 0;
-  // This batch row's 32-key tiles, spread evenly over the splits.
-  const int tiles_b = (kv + kDecKeys - 1) / kDecKeys;
-  const int per = max(1, (tiles_b + a.splits - 1) / a.splits);
-  const int n_valid = (tiles_b + per - 1) / per;
-  if (split > 0 && split >= n_valid) return;
-  const int t0 = split * per;
-  const int R = a.S * a.G;  // <= kDecRows
-  const int row = l32;
-  const bool row_ok = row < R;
-  const int ti = row_ok ? row / a.G : 0;
-  const int h = hk * a.G + (row_ok ? row - ti * a.G : 0);
-  const int kend_lane = row_ok ? (a.causal ? min(clen + ti + 1, kv) : kv) : 0;
-  const int kend_max = a.causal ? min(clen + (R - 1) / a.G + 1, kv) : kv;
-  const int kend_min = a.causal ? min(clen + 1, kv) : kv;
-  const int t_end = min(min(tiles_b, t0 + per), (kend_max + kDecKeys - 1) / kDecKeys);
-  const int n_my = t0 + wave < t_end ? (t_end - t0 - wave + kWaves - 1) / kWaves : 0;  // this wave's tiles
-
-  // Q^T B-operand fragments first (their loads are older than every tile copy).
-  bf16x8 qf[KS];
-  {
-    const bf16_t* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)ti * a.q_st + (int64_t)h * a.q_sh;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = row_ok ? *(const bf16x8*)&qrow[16 * ks + 8 * hi] : bf16x8{};
+  // This share [u_begin, u_end) of the line, and the first batch row it touches:
+  // lane j of the loaded rows, its units at `base` on the line.
+  TileLine<kUnit> line;
+  line.load(a, 0, 0, lane);
+  zero_keyless<D>(a, line, lane);
+  int total = line.end();
+  for (int first = 64; first < a.B; first += 64) {
+    line.load(a, first, total, lane);
+    zero_keyless<D>(a, line, lane);
+    total = line.end();
   }
+  const int per = share_of(a, total * a.Hkv);
+  const int u_begin = (int)blockIdx.x * per;
+  const int u_end = min(total * a.Hkv, u_begin + per);
+  if (u_begin >= u_end) return;
+  if (a.B > 64) line.load(a, 0, 0, lane);
+  while (line.end() * a.Hkv <= u_begin) line.load(a, line.first + 64, line.end(), lane);
+  int j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl * a.Hkv > u_begin));
 
+  const int R = a.S * a.G;  // <= kDecRows
+  const bool row_ok = l32 < R;
+  const int ti = row_ok ? l32 / a.G : 0;
+  const float c2 = a.scale_log2;
+  const TileLanes<D> tl(lane);
+  bf16_t* const mk0 = sK0 + wave * T::kElems;
+  bf16_t* const mv0 = sV0 + wave * T::kElems;
+  bf16_t* const mk1 = sK1 + wave * T::kElems;
+  bf16_t* const mv1 = sV1 + wave * T::kElems;
   // This wave's copies of one 32-key tile: instruction i writes units
   // [64 i, 64 i + 64) of the wave's region; units past the 32 rows read zeros.
-  const bf16_t* kbase = a.ck + (row_in_cache ? crow : 0) * a.ck_sb + (int64_t)hk * a.ck_sh;
-  const bf16_t* vbase = a.cv + (row_in_cache ? crow : 0) * a.cv_sb + (int64_t)hk * a.cv_sh;
   uint32_t voffk[T::kInst], voffv[T::kInst];
+  {
+    const uint32_t stk = (uint32_t)a.ck_st * 2u, stv = (uint32_t)a.cv_st * 2u;
+    int prow = lane / L::kRowUnits, c = lane % L::kRowUnits;  // of unit 64 i + lane
 #pragma unroll
-  for (int i = 0; i < T::kInst; ++i) {
-    const int u = i * 64 + lane;
-    const int prow = u / L::kRowUnits;
-    const int c = u - prow * L::kRowUnits;
-    const int k = L::unperm(prow);
-    const bool ok = c < L::kUnits && k < kDecKeys;
-    voffk[i] = ok ? (uint32_t)((k * a.ck_st + c * 8) * 2) : 0x80000000u;
-    voffv[i] = ok ? (uint32_t)((k * a.cv_st + c * 8) * 2) : 0x80000000u;
+    for (int i = 0; i < T::kInst; ++i) {
+      const uint32_t k = (uint32_t)L::unperm(prow);
+      const bool ok = c < L::kUnits && prow < kDecKeys;
+      voffk[i] = ok ? k * stk + c * 16 : 0x80000000u;
+      voffv[i] = ok ? k * stv + c * 16 : 0x80000000u;
+      prow += 64 / L::kRowUnits;
+      c += 64 % L::kRowUnits;
+      const int carry = c >= L::kRowUnits ? 1 : 0;
+      prow += carry;
+      c -= carry * L::kRowUnits;
+    }
   }
+  // The arguments that only a segment's start, its new rows and its end need,
+  // loaded there: held across the tile loop they would spill.
+  auto cold_args = []() __attribute__((always_inline)) -> const CacheArgs& {
+    uint64_t seg = kernel_segment();
+    __asm__ volatile("" : "+s"(seg));
+    return segment_args<CacheArgs>(seg);
+  };
+  // The current segment: tiles [t0, t_end) of (batch row b, kv head hk), the
+  // first at position u0 of the line.
+  const int ck_st = (int)a.ck_st, cv_st = (int)a.cv_st;  // a span check bounds them
+  int u0 = u_begin;
+  int b, hk, kv, pos_b, crow, t0, n_my, kend_lane, kend_min, u_next, u_row;  // u_row: where the next batch row begins
+  bool whole;
+  int new_lo, new_hi;  // positions [new_lo, new_hi) may hold new rows
+  bf16_t *kbase, *vbase;
+  bf16x8 qf[KS];
+
+  // The other batch rows on the segment's cache row: f(batch row, its position).
+  auto for_others = [&](auto&& f) __attribute__((always_inline)) {
+    if (a.batch_indices == nullptr) return;
+    TileLine<kUnit> other = line;
+    for (int first = 0; first < a.B; first += 64) {
+      if (a.B > 64) other.load(a, first, 0, lane);
+      uint64_t same = __builtin_amdgcn_ballot_w64(other.row == crow && first + lane != b);
+      for (; same != 0; same &= same - 1) {
+        const int o = __builtin_ctzll(same);
+        f(first + o, __builtin_amdgcn_readlane(other.pos, o));
+      }
+    }
+  };
+  // Overlay tile t's copy with the new rows (of batch row o, at position p on)
+  // among its keys; the batch row's own are also stored to the cache.
+  auto overlay_from = [&](int o, int p, int t, bf16_t* tk, bf16_t* tv) {
+    constexpr int kUnits = D / 8;
+    const CacheArgs& c = cold_args();
+    const bf16_t* kn = c.kn + (int64_t)o * c.kn_sb + (int64_t)hk * c.kn_sh;
+    const bf16_t* vn = c.vn + (int64_t)o * c.vn_sb + (int64_t)hk * c.vn_sh;
+    const int64_t kn_st = c.kn_st, vn_st = c.vn_st;
+    const int key0 = t * kDecKeys;
+    const int lo = max(key0 - p, 0), end = min(a.S, min(key0 + kDecKeys, kv) - p);  // new rows inside the tile
+    for (int i0 = lo; i0 < end; i0 += 64 / kUnits) {
+      const int i = i0 + lane / kUnits, col = lane % kUnits * 8;
+      if (i < end) {
+        const bf16x8 kx = *(const bf16x8*)&kn[(int64_t)i * kn_st + col];
+        const bf16x8 vx = *(const bf16x8*)&vn[(int64_t)i * vn_st + col];
+        *(bf16x8*)&tk[L::off(p + i - key0, col)] = kx;
+        *(bf16x8*)&tv[L::off(p + i - key0, col)] = vx;
+        if (o == b) {
+          *(bf16x8*)&kbase[(int64_t)(p + i) * ck_st + col] = kx;
+          *(bf16x8*)&vbase[(int64_t)(p + i) * cv_st + col] = vx;
+        }
+      }
+    }
+  };
+  auto overlay = [&](int t, bf16_t* tk, bf16_t* tv) {
+    const int key0 = t * kDecKeys;
+    if (key0 >= new_hi || key0 + kDecKeys <= new_lo) return;
+    for_others([&](int o, int p) { overlay_from(o, p, t, tk, tv); });
+    overlay_from(b, pos_b, t, tk, tv);
+    __asm__ volatile("" ::: "memory");
+    wait_lds();
+  };
+
+
   auto issue = [&](int t, bf16_t* tk, bf16_t* tv) {
     const int key0 = t * kDecKeys;
-    const __amdgpu_buffer_rsrc_t rk = make_rsrc(kbase + (int64_t)key0 * a.ck_st, rows_bytes(kv - key0, a.ck_st, D));
-    const __amdgpu_buffer_rsrc_t rv = make_rsrc(vbase + (int64_t)key0 * a.cv_st, rows_bytes(kv - key0, a.cv_st, D));
+    const __amdgpu_buffer_rsrc_t rk = make_rsrc(kbase + (int64_t)key0 * ck_st, rows_bytes32(kv - key0, ck_st, D));
+    const __amdgpu_buffer_rsrc_t rv = make_rsrc(vbase + (int64_t)key0 * cv_st, rows_bytes32(kv - key0, cv_st, D));
 #pragma unroll
     for (int i = 0; i < T::kInst; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)(tk + i * 512), 16,
@@ -483,21 +649,48 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (__attribute__((address_space(3))) void*)(tv + i * 512), 16,
                                                voffv[i], 0, 0, 0);
   };
-  bf16_t* const mk0 = sK0 + wave * T::kElems;
-  bf16_t* const mv0 = sV0 + wave * T::kElems;
-  bf16_t* const mk1 = sK1 + wave * T::kElems;
-  bf16_t* const mv1 = sV1 + wave * T::kElems;
-  if (n_my > 0) issue(t0 + wave, mk0, mv0);
-  if (n_my > 1) issue(t0 + wave + kWaves, mk1, mv1);
+  // Makes the segment at u0 (lane j of the line) the current one: its Q rows and
+  // this wave's first two tiles are requested.
+  auto begin = [&]() __attribute__((always_inline)) {
+    const CacheArgs& c = cold_args();
+    b = line.first + j;
+    const int units_b = __builtin_amdgcn_readlane(line.units, j);
+    const int base = (__builtin_amdgcn_readlane(line.incl, j) - units_b) * c.Hkv;
+    kv = __builtin_amdgcn_readlane(line.keys, j);
+    pos_b = __builtin_amdgcn_readlane(line.pos, j);
+    crow = __builtin_amdgcn_readlane(line.row, j);
+    hk = (u0 - base) / units_b;
+    const int unit0 = (u0 - base) - hk * units_b;
+    const int unit1 = min(units_b, unit0 + u_end - u0);
+    whole = unit0 == 0 && unit1 == units_b;
+    u_next = u0 + unit1 - unit0;
+    u_row = base + units_b * c.Hkv;
+    t0 = unit0 * kUnit;
+    const int t_end = min((int64_t)unit1 * kUnit, (int64_t)(kv + kDecKeys - 1) / kDecKeys);
+    n_my = t0 + wave < t_end ? (t_end - t0 - wave + kDecWaves - 1) / kDecWaves : 0;  // this wave's tiles
+    const int clen = max(pos_b, 0);
+    kend_lane = row_ok ? (c.causal ? min(clen + ti + 1, kv) : kv) : 0;
+    kend_min = c.causal ? min(clen + 1, kv) : kv;
+    kbase = c.ck + (int64_t)crow * c.ck_sb + (int64_t)hk * c.ck_sh;
+    vbase = c.cv + (int64_t)crow * c.cv_sb + (int64_t)hk * c.cv_sh;
+    // Q^T B-operand fragments first (their loads are older than the tile copies);
+    // lanes past the R rows take row 0: their columns are never read
+    const bf16_t* qrow = c.q + (int64_t)b * c.q_sb + (int64_t)ti * c.q_st +
+                         (int64_t)(hk * c.G + (row_ok ? l32 - ti * c.G : 0)) * c.q_sh + 8 * hi;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const bf16x8*)&qrow[16 * ks];
+    if (n_my > 0) issue(t0 + wave, mk0, mv0);
+    if (n_my > 1) issue(t0 + wave + kDecWaves, mk1, mv1);
+    new_lo = pos_b;
+    new_hi = pos_b + a.S;
+    for_others([&](int, int p) {
+      new_lo = min(new_lo, p);
+      new_hi = max(new_hi, p + a.S);
+    });
+  };
 
   f32x16 oacc[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x16{};
-  float m_run = -INFINITY;
-  float l_run = 0.f;
-  const float c2 = a.scale_log2;
-  const TileLanes<D> tl(lane);
-
+  float m_run, l_run;
   auto compute = [&](int t, const bf16_t* sK, const bf16_t* sV) {
     const int kb = t * kDecKeys;
     f32x16 st = f32x16{};
@@ -552,112 +745,213 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
       }
   };
 
-  // Each wave waits only for its own copies: tile i has landed once at most the
-  // copies of tile i + 1 are outstanding.
-  for (int i = 0; i < n_my; i += 2) {
-    if (i + 1 < n_my)
-      wait_vmcnt_wide<2 * T::kInst>();
-    else
-      wait_vmcnt_wide<0>();
-    compute(t0 + wave + kWaves * i, mk0, mv0);
-    if (i + 2 < n_my) {
-      wait_lds();  // this wave's reads of the stage are done before it is refilled
-      issue(t0 + wave + kWaves * (i + 2), mk0, mv0);
-    }
-    if (i + 1 >= n_my) break;
-    if (i + 2 < n_my)
-      wait_vmcnt_wide<2 * T::kInst>();
-    else
-      wait_vmcnt_wide<0>();
-    compute(t0 + wave + kWaves * (i + 1), mk1, mv1);
-    if (i + 3 < n_my) {
-      wait_lds();
-      issue(t0 + wave + kWaves * (i + 3), mk1, mv1);
-    }
-  }
-
-  // Merge the four waves' partial rows through LDS (the stages are free once
-  // every wave is past its tile loop): O of waves 0-1 in sK0, of waves 2-3 in sV0.
-  __syncthreads();
-  {
-    float* po = (float*)(wave < 2 ? sK0 : sV0) + (wave & 1) * kDecRows * D + l32 * D;
+  begin();
+  for (;;) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        f32x4 tv;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) tv[e] = oacc[dt][4 * rg + e];
-        *(f32x4*)&po[32 * dt + 8 * rg + 4 * hi] = tv;
+    for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x16{};
+    m_run = -INFINITY;
+    l_run = 0.f;
+    // Each wave waits only for its own copies: tile i has landed once at most the
+    // copies of tile i + 1 are outstanding.
+    for (int i = 0; i < n_my; i += 2) {
+      if (i + 1 < n_my)
+        wait_vmcnt_wide<2 * T::kInst>();
+      else
+        wait_vmcnt_wide<0>();
+      overlay(t0 + wave + kDecWaves * i, mk0, mv0);
+      compute(t0 + wave + kDecWaves * i, mk0, mv0);
+      if (i + 2 < n_my) {
+        wait_lds();  // this wave's reads of the stage are done before it is refilled
+        issue(t0 + wave + kDecWaves * (i + 2), mk0, mv0);
       }
+      if (i + 1 >= n_my) break;
+      if (i + 2 < n_my)
+        wait_vmcnt_wide<2 * T::kInst>();
+      else
+        wait_vmcnt_wide<0>();
+      overlay(t0 + wave + kDecWaves * (i + 1), mk1, mv1);
+      compute(t0 + wave + kDecWaves * (i + 1), mk1, mv1);
+      if (i + 3 < n_my) {
+        wait_lds();
+        issue(t0 + wave + kDecWaves * (i + 3), mk1, mv1);
+      }
+    }
+
+    // The next segment's copies go out before this one's merge (this wave's reads
+    // of its stages are done; the merge has LDS of its own), so that a share of
+    // several short segments does not pay a memory round trip for each.
+    const int cur_b = b, cur_hk = hk;
+    const bool cur_whole = whole;
+    const int64_t slot = (int64_t)part_slot(u0, per) * R;
+    const bool more = u_next < u_end;
+    wait_lds();
+    if (more) {
+      u0 = u_next;
+      if (u0 == u_row) {  // the next batch row with keys
+        while (line.end() * a.Hkv <= u0) line.load(a, line.first + 64, line.end(), lane);
+        j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl * a.Hkv > u0));
+      }
+      begin();
+    }
+    // Merge the waves' partial rows through LDS, kMergeRows at a time.
     const float l_tot = xor32_sum(l_run);
     if (hi == 0) {
       sMl[wave][l32][0] = m_run == -INFINITY ? -INFINITY : m_run * c2;
       sMl[wave][l32][1] = l_tot;
     }
-  }
-  __syncthreads();
-  constexpr int cpl = D / 64;
-  const int64_t units = (int64_t)gridDim.x;
-  const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.part_o, (uint32_t)(units * kRows * D * 4));
-  const __amdgpu_buffer_rsrc_t rml = make_rsrc(a.part_ml, (uint32_t)(units * kRows * 2 * 4));
-  for (int rr = wave; rr < R; rr += kWaves) {  // one wave per row, D / 64 columns per lane
-    float M = -INFINITY;
+    constexpr int cpl = D / 64;
+    for (int r0 = 0; r0 < R; r0 += kMergeRows) {
+      if (l32 >= r0 && l32 < r0 + kMergeRows) {
+        float* po = sO[wave][l32 - r0];
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, sMl[w][rr][0]);
-    float lsum = 0.f;
-    float acc[cpl] = {};
-    if (M != -INFINITY) {
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float m = sMl[w][rr][0];
-        const float wt = m == -INFINITY ? 0.f : fast_exp2(m - M);
-        lsum += sMl[w][rr][1] * wt;
-        const float* po = (const float*)(w < 2 ? sK0 : sV0) + (w & 1) * kDecRows * D + rr * D + lane * cpl;
+          for (int rg = 0; rg < 4; ++rg) {
+            f32x4 tv;
 #pragma unroll
-        for (int j = 0; j < cpl; ++j) acc[j] += po[j] * wt;
+            for (int e = 0; e < 4; ++e) tv[e] = oacc[dt][4 * rg + e];
+            *(f32x4*)&po[32 * dt + 8 * rg + 4 * hi] = tv;
+          }
       }
-    }
-    if (n_valid <= 1) {
-      const float inv = lsum > 0.f ? 1.f / lsum : 0.f;  // no keys (row outside the cache): zeros
-      const int ti_r = rr / a.G;
-      const int h_r = hk * a.G + (rr - ti_r * a.G);
-      bf16_t* orow = a.out + (int64_t)b * a.o_sb + (int64_t)ti_r * a.o_st + (int64_t)h_r * a.o_sh + lane * cpl;
+      lds_barrier();
+      for (int rr = r0 + wave; rr < min(R, r0 + kMergeRows); rr += kDecWaves) {  // D / 64 columns per lane
+        float M = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < cpl; ++j) orow[j] = (bf16_t)(acc[j] * inv);
-    } else {
-      // this split's partial row, published with device-coherent stores
-      const uint32_t slot = (uint32_t)blockIdx.x * kRows + rr;
-      if constexpr (cpl == 2)
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, f32x2{acc[0], acc[1]}), ro,
-                                              (slot * D + lane * 2) * 4, 0, kDevScope);
-      else
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, acc[0]), ro, (slot * D + lane) * 4, 0,
-                                              kDevScope);
-      if (lane == 0)
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, f32x2{M, lsum}), rml, slot * 8, 0,
-                                              kDevScope);
+        for (int w = 0; w < kDecWaves; ++w) M = fmaxf(M, sMl[w][rr][0]);
+        float lsum = 0.f;
+        float acc[cpl] = {};
+        if (M != -INFINITY) {
+#pragma unroll
+          for (int w = 0; w < kDecWaves; ++w) {
+            const float m = sMl[w][rr][0];
+            const float wt = m == -INFINITY ? 0.f : fast_exp2(m - M);
+            lsum += sMl[w][rr][1] * wt;
+#pragma unroll
+            for (int e = 0; e < cpl; ++e) acc[e] += sO[w][rr - r0][lane * cpl + e] * wt;
+          }
+        }
+        const CacheArgs& c = cold_args();
+        if (cur_whole) {
+          const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+          const int ti_r = rr / a.G;
+          const int h_r = cur_hk * a.G + (rr - ti_r * a.G);
+          bf16_t* orow = c.out + (int64_t)cur_b * c.o_sb + (int64_t)ti_r * c.o_st + (int64_t)h_r * c.o_sh + lane * cpl;
+#pragma unroll
+          for (int e = 0; e < cpl; ++e) orow[e] = (bf16_t)(acc[e] * inv);
+        } else {
+          float* prow = c.part_o + (slot + rr) * D + lane * cpl;
+#pragma unroll
+          for (int e = 0; e < cpl; ++e) prow[e] = acc[e];
+          if (lane == 0) *(f32x2*)&c.part_ml[(slot + rr) * 2] = f32x2{M, lsum};
+        }
+      }
+      if (!more && r0 + kMergeRows >= R) return;
+      lds_barrier();  // the merge area is written again
     }
   }
-  if (n_valid <= 1) return;
-  __asm__ volatile("" ::: "memory");
-  wait_vmem();  // the partial rows are stored
-  __syncthreads();
-  if (tid == 0)
-    last = __hip_atomic_fetch_add(&a.counters[group], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n_valid - 1;
-  __syncthreads();
-  if (!last) return;
-  merge_split_rows<D>(a, ro, rml, group, n_valid, b, hk, 0, R, wave, lane);
 }
 
 // One kernel per head_dim, by name: two instantiations of one kernel template
 // launched from the two branches below lost one host stub in this toolchain.
-__global__ __launch_bounds__(kThreads, 1) void cache_decode_d128_kernel(const CacheArgs a) {
-  cache_decode_body<128>(a);
+__global__ __launch_bounds__(kShareWaves * 64, 1) void cache_decode_d128_kernel(const CacheArgs a) {
+  cache_decode_body<128, kShareWaves, kShareUnit>(a);
 }
-__global__ __launch_bounds__(kThreads, 1) void cache_decode_d64_kernel(const CacheArgs a) {
-  cache_decode_body<64>(a);
+__global__ __launch_bounds__(kShareWaves * 64, 1) void cache_decode_d64_kernel(const CacheArgs a) {
+  cache_decode_body<64, kShareWaves, kShareUnit>(a);
 }
+__global__ __launch_bounds__(kPairWaves * 64, 1) void cache_decode_pairs_d128_kernel(const CacheArgs a) {
+  cache_decode_body<128, kPairWaves, kPairUnit>(a);
+}
+__global__ __launch_bounds__(kPairWaves * 64, 1) void cache_decode_pairs_d64_kernel(const CacheArgs a) {
+  cache_decode_body<64, kPairWaves, kPairUnit>(a);
+}
+
+// Output rows of the (batch row, kv head) pairs whose key tiles lie in several
+// shares: out = sum_c O_c 2^(m_c - M) / sum_c l_c 2^(m_c - M) over the parts c in
+// the order of the line; zeros for batch rows without keys (outside the cache).
+// One wave per row: lane c takes part c's (max, sum), and the O rows are read one
+// part per D / 4 lanes with kChunk loads in flight beside it, so up to 32 parts
+// (D 128) cost one memory round trip.
+template <int D>
+__device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
+  constexpr int kLanes = D / 4;        // lanes per part row, four columns each
+  constexpr int kParts = 64 / kLanes;  // part rows per load
+  constexpr int kChunk = 16;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int R = a.S * a.G;
+  const int groups = (R + kWaves - 1) / kWaves;  // workgroups per pair
+  const int rr = blockIdx.x % groups * kWaves + wave;
+  const int hk = blockIdx.x / groups % a.Hkv;
+  const int b = blockIdx.x / groups / a.Hkv;
+  TileLine<kShareUnit> line;
+  line.load(a, 0, 0, lane);
+  int total = line.end(), units_b = 0, before = 0;
+  for (int first = 0;;) {
+    if (b >= first && b < first + 64) {
+      units_b = __builtin_amdgcn_readlane(line.units, b - first);
+      before = __builtin_amdgcn_readlane(line.incl, b - first) - units_b;
+    }
+    first += 64;
+    if (first >= a.B) break;
+    line.load(a, first, total, lane);
+    total = line.end();
+  }
+  const int per = share_of(a, total * a.Hkv);
+  const int g0 = before * a.Hkv + hk * units_b;  // the pair's units [g0, g0 + units_b) of the line
+  const int w0 = g0 / per, n = units_b > 0 ? (g0 + units_b - 1) / per - w0 + 1 : 0;  // shares it lies in
+  if (n <= 1 || rr >= R) return;  // written by its share
+  const int sub = lane / kLanes, col = lane % kLanes * 4;
+  float M = -INFINITY, lsum = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};  // this lane's columns over the parts of its lane group
+  for (int c0 = 0; c0 < n; c0 += 64) {
+    const int c = c0 + lane, in_chunk = min(n - c0, 64);
+    const int row = part_slot(c == 0 ? g0 : (w0 + min(c, n - 1)) * per, per) * R + rr;
+    f32x2 ml = *(const f32x2*)&a.part_ml[2 * (int64_t)row];
+    f32x4 ov[kChunk];
+    auto load_rows = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < kChunk; ++i)
+        ov[i] = *(const f32x4*)&a.part_o[(int64_t)__shfl(row, min(i0 + i * kParts + sub, in_chunk - 1), 64) * D + col];
+    };
+    load_rows(0);  // in flight beside the weights
+    if (c >= n) ml = f32x2{-INFINITY, 0.f};
+    float m = ml[0];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    const float m_new = fmaxf(M, m);
+    const float alpha = M == -INFINITY ? 0.f : fast_exp2(M - m_new);
+    const float w = ml[0] == -INFINITY ? 0.f : fast_exp2(ml[0] - m_new);  // -inf: no allowed key in this part
+    float l = ml[1] * w;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) l += __shfl_xor(l, off, 64);
+    lsum = lsum * alpha + l;
+    acc *= alpha;
+    M = m_new;
+    for (int i0 = 0;;) {
+#pragma unroll
+      for (int i = 0; i < kChunk; ++i) {
+        const int src = i0 + i * kParts + sub;
+        const float wi = __shfl(w, min(src, 63), 64);
+        if (src < in_chunk && wi != 0.f) acc += ov[i] * wi;
+      }
+      i0 += kChunk * kParts;
+      if (i0 >= in_chunk) break;
+      load_rows(i0);
+    }
+  }
+#pragma unroll
+  for (int off = kLanes; off < 64; off <<= 1)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
+  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+  const int ti = rr / a.G;
+  if (sub == 0)
+    *(bf16x4*)&a.out[(int64_t)b * a.o_sb + (int64_t)ti * a.o_st + (int64_t)(hk * a.G + rr - ti * a.G) * a.o_sh + col] =
+        __builtin_convertvector(acc * inv, bf16x4);
+}
+__global__ __launch_bounds__(kThreads) void cache_merge_d128_kernel(const CacheArgs a) { cache_merge_body<128>(a); }
+__global__ __launch_bounds__(kThreads) void cache_merge_d64_kernel(const CacheArgs a) { cache_merge_body<64>(a); }
 
 unsigned grid_for(int64_t items) {
   const int64_t blocks = (items + 255) / 256;
@@ -667,7 +961,7 @@ unsigned grid_for(int64_t items) {
 }  // namespace
 
 CacheSplit cache_split(const MimirCacheAttnParams& p) {
-  CacheSplit s;
+  CacheSplit s = {};
   const int G = p.num_kv_heads > 0 ? p.num_q_heads / p.num_kv_heads : 1;
   const int64_t R = (int64_t)p.seqlen * G;
   s.decode = R <= kDecRows;  // the decode kernels: 32-key wave tiles, one workgroup per CU
@@ -677,8 +971,26 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
   const int tile_keys = s.decode ? kDecKeys : kKeys;
   const int tiles = (max_kv + tile_keys - 1) / tile_keys;
   s.groups = (int64_t)p.batch * p.num_kv_heads * s.n_rt;
-  // workgroups to cover the chip: one per CU for the decode kernel, two for the other
-  const int64_t target = (s.decode ? 1 : 2) * (int64_t)device_cu_count();
+  if (s.decode) {
+    // One workgroup per pair while that fills the chip about evenly: from 256 keys
+    // for any batch (two rounds of copies) up to 2048 for a pair per CU.  64 x 4
+    // pairs (one launch against two, no merge): 100 to 1000 keys 25.5 -> 19.0 us, 100
+    // to 2000 keys 37.5 / 37.9, 100 to 4000 keys 65 / 72 (the longest pair runs alone).
+    const int64_t pair_keys = 8 * s.groups;
+    s.pairs = max_kv <= (pair_keys < 256 ? 256 : (pair_keys < 2048 ? pair_keys : 2048));
+    if (s.pairs) {  // one workgroup per pair
+      s.units = s.groups;
+    } else {
+      // two shares of the line per CU, or one per unit if there cannot be as many;
+      // two part slots per share: partial O, then (max, sum) rows
+      const int64_t most = s.groups * ((tiles + kShareUnit - 1) / kShareUnit), two = 2 * (int64_t)device_cu_count();
+      s.units = most < two ? most : two;
+      s.workspace_bytes = (size_t)s.units * 2 * (size_t)R * ((size_t)p.head_dim + 2) * sizeof(float);
+    }
+    s.splits = 1;
+    return s;
+  }
+  const int64_t target = 2 * (int64_t)device_cu_count();  // two workgroups per CU
   int64_t splits = s.groups > 0 ? (target + s.groups - 1) / s.groups : 1;
   if (splits < 1) splits = 1;
   if (splits > tiles) splits = tiles;
@@ -721,6 +1033,30 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   a.splits = sp.splits;
   a.scale_log2 = p.softmax_scale * kLog2e;
   a.part_o = (float*)p.workspace;
+  if (sp.decode) {
+    if (sp.units == 0) return hipSuccess;
+    if (!sp.pairs && p.workspace == nullptr) return hipErrorInvalidValue;
+    const int64_t rows = (int64_t)a.S * a.G;
+    a.shares = (int)sp.units;
+    a.part_ml = a.part_o + (size_t)sp.units * 2 * rows * p.head_dim;
+    const dim3 grid((unsigned)sp.units);
+    if (sp.pairs) {
+      if (p.head_dim == 128)
+        hipLaunchKernelGGL(cache_decode_pairs_d128_kernel, grid, dim3(kPairWaves * 64), 0, stream, a);
+      else
+        hipLaunchKernelGGL(cache_decode_pairs_d64_kernel, grid, dim3(kPairWaves * 64), 0, stream, a);
+      return hipGetLastError();
+    }
+    const dim3 merge((unsigned)(sp.groups * ((rows + kWaves - 1) / kWaves)));
+    if (p.head_dim == 128) {
+      hipLaunchKernelGGL(cache_decode_d128_kernel, grid, dim3(kShareWaves * 64), 0, stream, a);
+      hipLaunchKernelGGL(cache_merge_d128_kernel, merge, dim3(kThreads), 0, stream, a);
+    } else {
+      hipLaunchKernelGGL(cache_decode_d64_kernel, grid, dim3(kShareWaves * 64), 0, stream, a);
+      hipLaunchKernelGGL(cache_merge_d64_kernel, merge, dim3(kThreads), 0, stream, a);
+    }
+    return hipGetLastError();
+  }
   a.part_ml = a.part_o + (size_t)sp.units * kRows * p.head_dim;
   a.counters = (int*)(a.part_ml + (size_t)sp.units * kRows * 2);
   a.n_counters = sp.splits > 1 ? (int)sp.groups : 0;
@@ -730,13 +1066,6 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   if (appends > 0) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || sp.units == 0) return e;
-  if (sp.decode) {
-    if (p.head_dim == 128)
-      hipLaunchKernelGGL(cache_decode_d128_kernel, dim3((unsigned)sp.units), dim3(kThreads), 0, stream, a);
-    else
-      hipLaunchKernelGGL(cache_decode_d64_kernel, dim3((unsigned)sp.units), dim3(kThreads), 0, stream, a);
-    return hipGetLastError();
-  }
   if (p.head_dim == 128)
     hipLaunchKernelGGL(cache_attn_kernel<128>, dim3((unsigned)sp.units), dim3(kThreads), 0, stream, a);
   else

@@ -738,10 +738,11 @@ hipError_t launch_prologue(const Prologue& pro, hipStream_t stream);
 
 // KV-cache attention (prefixlm_cache_bf16.hip): the key split and its workspace.
 struct CacheSplit {
-  bool decode;     // at most 32 query rows per kv head: the decode kernel
+  bool decode;     // at most 32 query rows per kv head: the decode kernels ...
+  bool pairs;      // ... one workgroup per (batch row, kv head) pair instead of equal shares of all key tiles
   int n_rt, splits;
   int64_t groups;  // (batch row, kv head, row tile) triples
-  int64_t units;   // groups * splits workgroups
+  int64_t units;   // workgroups: groups * splits, or the decode kernels' shares
   size_t workspace_bytes;
 };
 CacheSplit cache_split(const MimirCacheAttnParams& p);

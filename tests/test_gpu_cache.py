@@ -57,6 +57,33 @@ def test_short_chunks_around_the_decode_kernel(device, S, causal):
     _run(device, B=3, S=S, hq=16, hkv=2, d=128, L=900, lens=[0, 451, 880], causal=causal, seed=20 + S)
 
 
+@pytest.mark.parametrize("B,S,hq,hkv,d,L,seed", [
+    (70, 1, 8, 2, 64, 300, 1),      # one workgroup per pair; more batch rows than a wave has lanes
+    (300, 2, 4, 1, 128, 70, 2),
+    (2, 32, 2, 2, 128, 200, 3),     # 32 new rows over two tiles, 32 query rows
+    (3, 1, 4, 4, 128, 9000, 4),     # equal shares: pairs over many shares
+    (70, 1, 4, 1, 64, 3000, 5),     # shares over several pairs, batch rows past the first 64
+    (5, 8, 4, 1, 128, 700, 6),      # 32 query rows merged over parts
+])
+def test_decode_work_split(device, B, S, hq, hkv, d, L, seed):
+    """One workgroup per pair, and the line of key tiles dealt to equal shares: ragged lengths
+    (0 keys to the whole cache), shuffled cache rows, new rows across a tile edge."""
+    gen = torch.Generator().manual_seed(seed)
+    lens = torch.randint(0, L - S + 1, (B,), generator=gen).tolist()
+    lens[0], lens[-1] = 0, L - S
+    _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=True,
+         rows=torch.randperm(B, generator=gen).tolist(), seed=seed)
+
+
+def test_decode_rows_sharing_a_cache_row(device):
+    """Batch rows on one cache row attend each other's new keys, as after appending all of them
+    first: consecutive tokens of a sequence fed as separate batch rows, and one far behind."""
+    _run(device, B=5, S=1, hq=8, hkv=2, d=128, L=700, lens=[63, 64, 65, 10, 300], causal=False,
+         rows=[1, 1, 1, 1, 0], cache_rows=2, seed=31)
+    _run(device, B=3, S=2, hq=4, hkv=2, d=64, L=200, lens=[30, 32, 150], causal=False, rows=[0, 0, 0], cache_rows=1,
+         seed=32)  # one workgroup per pair
+
+
 def test_decode_uneven_rows(device):
     """Rows whose key ranges split into different numbers of parts (1 key to the whole cache)."""
     _run(device, B=8, S=1, hq=16, hkv=4, d=128, L=4096, lens=[0, 63, 64, 65, 1000, 4095, 2048, 129],
@@ -113,8 +140,8 @@ def test_rows_outside_the_cache_are_skipped(device):
 
 
 def test_repeated_calls_and_graph_replay(device):
-    """The split arrival counters are cleared by each call: back-to-back calls and replays of a
-    captured decode step (no host synchronisation, no memset) match the eager result."""
+    """Back-to-back calls and replays of a captured decode step (no host synchronisation, no
+    memset) match the eager result."""
     gen = torch.Generator().manual_seed(11)
     B, hq, hkv, d, L = 4, 8, 2, 128, 2048
     q = torch.randn(B, 1, hq, d, generator=gen).to(BF16).to(device)
