@@ -10,12 +10,15 @@ codes onto the exception types the reference raises for the same conditions
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 from pathlib import Path
 
 # MIMIR_PREFIXLM_LIB overrides the in-tree library (e.g. to A/B two builds).
 LIB_PATH = Path(os.environ.get("MIMIR_PREFIXLM_LIB") or Path(__file__).resolve().parent / "_lib" / "libmimir_prefixlm.so")
+HOST_PATH = Path(__file__).resolve().parent / "_lib" / "_host_calls.so"
 ABI_VERSION = 8
 
 DTYPE_FLOAT32 = 0
@@ -194,6 +197,31 @@ def load() -> ctypes.CDLL:
             raise ImportError(f"{LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it")
         _lib = lib
         return lib
+
+
+_host = None
+
+
+def host():
+    """The native host calls (csrc/host_calls.cpp), bound to the library; ImportError if not built.
+
+    ``fwd`` / ``bwd`` / ``rope`` / ``cache_attn`` check, allocate and launch a
+    well-formed call and return None for any other, which then takes the general path."""
+    global _host
+    if _host is not None:
+        return _host
+    load()
+    with _lock:
+        if _host is None:
+            if not HOST_PATH.exists():
+                raise ImportError(f"mimir_amd prefix-LM attention requires {HOST_PATH}; "
+                                  "build it with `python -m mimir_amd.build`")
+            loader = importlib.machinery.ExtensionFileLoader("_host_calls", str(HOST_PATH))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host_calls", loader))
+            loader.exec_module(module)
+            module.bind(str(LIB_PATH))
+            _host = module
+    return _host
 
 
 def raise_for_status(lib: ctypes.CDLL, status: int) -> None:

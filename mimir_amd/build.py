@@ -1,10 +1,11 @@
-"""Build libmimir_prefixlm.so (the C-ABI HIP library) in-tree for gfx950.
+"""Build libmimir_prefixlm.so (the C-ABI HIP library) and the native host calls in-tree for gfx950.
 
 Every HIP source under ``mimir_amd/csrc`` is compiled with hipcc for
 ``--offload-arch=gfx950`` and linked into ``mimir_amd/_lib/libmimir_prefixlm.so``.
 No torch extension machinery is involved: the library exports only the
 ``extern "C"`` entry points declared in ``include/mimir_prefixlm.h`` and is loaded
-with ctypes.  Run ``python -m mimir_amd.build`` (or ``__graft_entry__.build()``).
+with ctypes.  ``csrc/host_calls.cpp`` (no device code; torch's C++ headers) becomes
+``mimir_amd/_lib/_host_calls.so``, the Python module that makes the common calls.  Run ``python -m mimir_amd.build`` (or ``__graft_entry__.build()``).
 """
 
 from __future__ import annotations
@@ -20,6 +21,8 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libmimir_prefixlm.so"
+HOST_SOURCE = CSRC / "host_calls.cpp"
+HOST_PATH = LIB_DIR / "_host_calls.so"
 ARCH = "gfx950"
 
 # Packed FP32 (v_pk_*_f32) is disabled: hipcc otherwise forms them from float2
@@ -75,13 +78,34 @@ def _compile(src: Path, obj: Path) -> None:
         print(err, file=sys.stderr)
 
 
+def _build_host() -> None:
+    """Compile the native host calls against the running Python and torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    libs = Path(torch.__file__).resolve().parent / "lib"
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(x for p in include_paths() for x in ("-isystem", p)), f"-I{sysconfig.get_paths()['include']}",
+           str(HOST_SOURCE), "-o", str(tmp), f"-L{libs}", f"-Wl,-rpath,{libs}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"compiling {HOST_SOURCE.name} failed:\n{res.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(verbose: bool = True) -> Path:
-    """Compile every HIP source and link the shared library; returns its path."""
+    """Compile every source and link the shared library; returns its path."""
     obj_dir = LIB_DIR / "obj"
     obj_dir.mkdir(parents=True, exist_ok=True)
     objs = [obj_dir / (s.rsplit(".", 1)[0] + ".o") for s in SOURCES]
     with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as ex:
+        host = ex.submit(_build_host)
         list(ex.map(lambda so: _compile(CSRC / so[0], so[1]), zip(SOURCES, objs)))
+        host.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     res = subprocess.run(cmd, capture_output=True, text=True)

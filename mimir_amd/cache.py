@@ -60,6 +60,13 @@ def attention_with_cache(query: Tensor, key: Tensor, value: Tensor, cache: Cache
     """
     if query.dtype != torch.bfloat16:
         raise TypeError(f"KV-cache attention supports bfloat16 tensors only, got {query.dtype}")
+    if query.is_cuda and query.dim() == 4 and not P._validate_metadata:
+        out = _capi.host().cache_attn(query, key, value, cache.keys, cache.values, cache_lengths, causal,
+                                      cache_batch_indices,
+                                      1.0 / math.sqrt(query.shape[3]) if softmax_scale is None else float(softmax_scale),
+                                      torch.empty, P._stream(query.device))
+        if out is not None:
+            return out
     B, S, hq, d = query.shape
     hkv = key.shape[2]
     if key.shape != (B, S, hkv, d) or value.shape != key.shape:

@@ -1,0 +1,392 @@
+// The host side of the common calls in native code: argument checks, output
+// allocation, the parameter struct and the C-ABI launch of the forward, the
+// backward, RoPE and the KV-cache attention.
+//
+// Through ctypes these cost 24 us (forward), 32 us (backward) and 17 us (decode) of
+// Python per call, and the backward pays about twice that in a training step: the
+// autograd engine runs it on a thread of its own, on a cold core.  A step on a few
+// short documents (70 us of GPU work) went from 182 to 113 us with the calls here (64
+// of which an autograd function of one multiplication takes too), a decode step of
+// one row from 16.3 to 11.7.
+//
+// Every function here serves only well-formed calls: anything else (another device
+// or dtype, a layout the kernels cannot read in place, metadata to convert, a failed
+// allocation or launch) returns None, and the caller takes the general path in
+// Python, which converts, falls back or raises.
+#include <Python.h>
+#include <dlfcn.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <torch/csrc/DynamicTypes.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/mimir_prefixlm.h"
+
+namespace {
+
+struct Library {
+  decltype(&mimir_prefixlm_fwd) fwd = nullptr;
+  decltype(&mimir_prefixlm_fwd_workspace_size) fwd_workspace_size = nullptr;
+  decltype(&mimir_prefixlm_fwd_workspace_bytes) fwd_workspace_bytes = nullptr;
+  decltype(&mimir_prefixlm_bwd) bwd = nullptr;
+  decltype(&mimir_prefixlm_bwd_workspace_size) bwd_workspace_size = nullptr;
+  decltype(&mimir_prefixlm_bwd_dscore_bytes) bwd_dscore_bytes = nullptr;
+  decltype(&mimir_prefixlm_rope) rope = nullptr;
+  decltype(&mimir_prefixlm_cache_attn) cache_attn = nullptr;
+  decltype(&mimir_prefixlm_cache_attn_workspace_bytes) cache_workspace = nullptr;
+} lib;
+
+struct Fallback {};  // thrown where the general path takes over
+void need(bool ok) {
+  if (!ok) throw Fallback();
+}
+
+const at::Tensor& tensor(PyObject* o) {
+  need(THPVariable_CheckExact(o));
+  return THPVariable_Unpack(o);
+}
+bool is_none(PyObject* o) { return o == Py_None; }
+int32_t int32(PyObject* o) {  // an int, or a one-element int64 CPU tensor (the reference's scalars)
+  int64_t x;
+  if (PyLong_CheckExact(o)) {
+    x = PyLong_AsLongLong(o);
+  } else {
+    const at::Tensor& t = tensor(o);
+    need(t.device().is_cpu() && t.scalar_type() == at::kLong && t.numel() == 1);
+    x = *t.const_data_ptr<int64_t>();
+  }
+  need(x >= 0 && x <= 0x7fffffff);
+  return (int32_t)x;
+}
+bool truth(PyObject* o) { return PyObject_IsTrue(o) == 1; }
+void* stream(PyObject* o) { return PyLong_AsVoidPtr(o); }
+
+// A [.., heads, head_dim] operand the kernels read or write in place: unit stride on
+// head_dim, 16-byte aligned rows that do not overlap.
+void in_place(const at::Tensor& t, const at::Tensor& like) {
+  const int64_t vec = 16 / (int64_t)t.element_size(), d = t.dim();
+  need(t.device() == like.device() && t.scalar_type() == like.scalar_type() && t.has_storage());
+  need(t.stride(d - 1) == 1 && t.stride(d - 3) >= t.size(d - 1) && (uintptr_t)t.const_data_ptr() % 16 == 0);
+  for (int64_t i = 0; i < d - 1; ++i) need(t.stride(i) % vec == 0);
+}
+void shaped(const at::Tensor& t, int64_t a, int64_t b, int64_t c) {
+  need(t.dim() == 3 && t.size(0) == a && t.size(1) == b && t.size(2) == c);
+}
+const int32_t* metadata(PyObject* o, int64_t n, const at::Tensor& like) {
+  const at::Tensor& t = tensor(o);
+  need(t.dim() == 1 && t.size(0) >= n && t.scalar_type() == at::kInt && t.device() == like.device() && t.is_contiguous());
+  return t.const_data_ptr<int32_t>();
+}
+
+at::Tensor empty(at::IntArrayRef shape, const at::Tensor& like, at::ScalarType type) {
+  return at::empty(shape, at::TensorOptions().dtype(type).device(like.device()));
+}
+
+// Workspaces come from the caller's torch.empty (float32): it raises where there is no room.
+at::Tensor workspace(PyObject* torch_empty, size_t bytes, PyObject* like) {
+  const size_t n = bytes / 4 < 4 ? 4 : bytes / 4;
+  PyObject* device = PyObject_GetAttrString(like, "device");
+  PyObject* args = Py_BuildValue("(n)", (Py_ssize_t)n);
+  PyObject* kw = Py_BuildValue("{s:O,s:N}", "dtype", (PyObject*)torch::getTHPDtype(at::kFloat), "device", device);
+  PyObject* t = args && kw ? PyObject_Call(torch_empty, args, kw) : nullptr;
+  Py_XDECREF(args);
+  Py_XDECREF(kw);
+  need(t != nullptr);
+  need(THPVariable_Check(t));
+  at::Tensor out = THPVariable_Unpack(t);
+  Py_DECREF(t);
+  return out;
+}
+
+template <typename P>
+void launch(int (*entry)(const P*, void*), const P& p, void* s) {
+  need(PyErr_Occurred() == nullptr);  // an argument did not convert
+  int status;
+  Py_BEGIN_ALLOW_THREADS;
+  status = entry(&p, s);
+  Py_END_ALLOW_THREADS;
+  need(status == MIMIR_OK);
+}
+
+// The checks and fields the forward and the backward share.
+struct Geometry {
+  int64_t T, hq, hkv, d;
+  int dtype;
+};
+Geometry geometry(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
+  need(q.is_cuda() && q.dim() == 3 && k.dim() == 3 && v.dim() == 3);
+  const Geometry g{q.size(0), q.size(1), k.size(1), q.size(2),
+                   q.scalar_type() == at::kBFloat16 ? MIMIR_DTYPE_BFLOAT16 : MIMIR_DTYPE_FLOAT32};
+  need(q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kFloat);
+  need(g.T > 0 && g.T <= 0x7fffffff && g.hq > 0 && g.hkv > 0 && g.hq % g.hkv == 0 && g.d > 0);
+  shaped(k, g.T, g.hkv, g.d);
+  shaped(v, g.T, g.hkv, g.d);
+  in_place(q, q);
+  in_place(k, q);
+  in_place(v, q);
+  return g;
+}
+
+#define STRIDES(p, name, t) (p).name##_stride_token = (t).stride(0), (p).name##_stride_head = (t).stride(1)
+
+PyObject* wrap(std::initializer_list<at::Tensor> ts) {
+  PyObject* out = PyTuple_New((Py_ssize_t)ts.size());
+  Py_ssize_t i = 0;
+  for (const at::Tensor& t : ts) PyTuple_SET_ITEM(out, i++, THPVariable_Wrap(t));
+  return out;
+}
+
+template <typename F>
+PyObject* guarded(Py_ssize_t given, Py_ssize_t wanted, F&& body) {
+  if (given != wanted) {
+    PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", wanted, given);
+    return nullptr;
+  }
+  try {
+    if (PyObject* out = body()) return out;
+  } catch (const Fallback&) {
+  } catch (const std::exception&) {  // e.g. out of memory: the general path raises it
+  }
+  PyErr_Clear();
+  Py_RETURN_NONE;
+}
+
+// fwd(q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen, numseqs, max_seqlen_all,
+//     softmax_scale, split_mode, key_chunks, want_lo, gate, gated_out, torch_empty, stream)
+//   -> (out, lse, out_lo, split_flag)
+PyObject* py_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 18, [&]() -> PyObject* {
+    const at::Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]);
+    const Geometry g = geometry(q, k, v);
+    MimirPrefixLMFwdParams p = {};
+    p.is_causal = truth(a[3]);
+    p.total_seqlen = int32(a[7]);
+    p.numseqs = int32(a[8]);
+    p.max_seqlen_all = int32(a[9]);
+    p.softmax_scale = (float)PyFloat_AsDouble(a[10]);
+    p.split_mode = int32(a[11]);
+    p.prefix_lens = metadata(a[4], p.numseqs, q);
+    p.causal_lens = metadata(a[5], p.numseqs, q);
+    p.cu_seqlens = metadata(a[6], p.numseqs + 1, q);
+    p.total_tokens = (int32_t)g.T, p.num_q_heads = (int32_t)g.hq, p.num_kv_heads = (int32_t)g.hkv;
+    p.head_dim = (int32_t)g.d, p.dtype = g.dtype;
+    const bool bf16 = g.dtype == MIMIR_DTYPE_BFLOAT16;
+    at::Tensor out = empty({g.T, g.hq, g.d}, q, q.scalar_type()), lse = empty({g.hq, g.T}, q, at::kFloat);
+    at::Tensor lo = truth(a[13]) ? empty({g.T, g.hq, g.d}, q, q.scalar_type()) : empty({0}, q, q.scalar_type());
+    at::Tensor flag = empty({bf16 ? 1 : 0}, q, at::kInt);
+    p.q = q.const_data_ptr(), p.k = k.const_data_ptr(), p.v = v.const_data_ptr();
+    p.out = out.mutable_data_ptr(), p.lse = (float*)lse.mutable_data_ptr();
+    STRIDES(p, q, q), STRIDES(p, k, k), STRIDES(p, v, v), STRIDES(p, out, out);
+    p.lse_stride_head = g.T;
+    if (lo.numel() > 0) p.out_lo = lo.mutable_data_ptr(), STRIDES(p, out_lo, lo);
+    if (bf16) p.split_flag = (int32_t*)flag.mutable_data_ptr();
+    if (!is_none(a[14])) {
+      const at::Tensor &gate = tensor(a[14]), &gated = tensor(a[15]);
+      shaped(gate, g.T, g.hq, g.d);
+      shaped(gated, g.T, g.hq, g.d);
+      in_place(gate, q);
+      in_place(gated, q);
+      p.gate = gate.const_data_ptr(), p.gated_out = gated.mutable_data_ptr();
+      STRIDES(p, gate, gate), STRIDES(p, gated_out, gated);
+    }
+    p.workspace_bytes = truth(a[12]) ? lib.fwd_workspace_size(&p)
+                                     : lib.fwd_workspace_bytes(p.total_tokens, p.numseqs, p.max_seqlen_all);
+    at::Tensor ws = workspace(a[16], p.workspace_bytes, a[0]);
+    p.workspace = ws.mutable_data_ptr();
+    launch(lib.fwd, p, stream(a[17]));
+    return wrap({out, lse, lo, flag});
+  });
+}
+
+// bwd(dout, q, k, v, out, lse, out_lo, split_flag, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen,
+//     numseqs, max_seqlen_all, softmax_scale, split_mode, key_chunks, dscore_limit, region_limit, gate, grads,
+//     torch_empty, stream) -> (dq, dk, dv)
+// grads: None, or (dgate, dq, dk, dv) views to write.  A score-gradient region above
+// region_limit needs the general path's look at the free memory.
+PyObject* py_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 24, [&]() -> PyObject* {
+    const at::Tensor &dout = tensor(a[0]), &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]);
+    const at::Tensor &out = tensor(a[4]), &lse = tensor(a[5]), &lo = tensor(a[6]), &flag = tensor(a[7]);
+    const Geometry g = geometry(q, k, v);
+    shaped(dout, g.T, g.hq, g.d);
+    shaped(out, g.T, g.hq, g.d);
+    in_place(dout, q);
+    in_place(out, q);
+    need(lse.dim() == 2 && lse.size(0) == g.hq && lse.size(1) == g.T && lse.scalar_type() == at::kFloat &&
+         lse.device() == q.device() && lse.is_contiguous());
+    MimirPrefixLMBwdParams p = {};
+    p.is_causal = truth(a[8]);
+    p.total_seqlen = int32(a[12]);
+    p.numseqs = int32(a[13]);
+    p.max_seqlen_all = int32(a[14]);
+    p.softmax_scale = (float)PyFloat_AsDouble(a[15]);
+    p.split_mode = int32(a[16]);
+    p.prefix_lens = metadata(a[9], p.numseqs, q);
+    p.causal_lens = metadata(a[10], p.numseqs, q);
+    p.cu_seqlens = metadata(a[11], p.numseqs + 1, q);
+    p.total_tokens = (int32_t)g.T, p.num_q_heads = (int32_t)g.hq, p.num_kv_heads = (int32_t)g.hkv;
+    p.head_dim = (int32_t)g.d, p.dtype = g.dtype;
+    at::Tensor dq, dk, dv;
+    if (is_none(a[21])) {
+      dq = empty({g.T, g.hq, g.d}, q, q.scalar_type());
+      dk = empty({g.T, g.hkv, g.d}, q, q.scalar_type());
+      dv = empty({g.T, g.hkv, g.d}, q, q.scalar_type());
+    } else {
+      need(PyTuple_Check(a[21]) && PyTuple_GET_SIZE(a[21]) == 4 && !is_none(a[20]));
+      const at::Tensor &gate = tensor(a[20]), &dgate = tensor(PyTuple_GET_ITEM(a[21], 0));
+      dq = tensor(PyTuple_GET_ITEM(a[21], 1));
+      dk = tensor(PyTuple_GET_ITEM(a[21], 2));
+      dv = tensor(PyTuple_GET_ITEM(a[21], 3));
+      shaped(gate, g.T, g.hq, g.d);
+      shaped(dgate, g.T, g.hq, g.d);
+      shaped(dq, g.T, g.hq, g.d);
+      shaped(dk, g.T, g.hkv, g.d);
+      shaped(dv, g.T, g.hkv, g.d);
+      for (const at::Tensor* t : {&gate, &dgate, (const at::Tensor*)&dq, (const at::Tensor*)&dk, (const at::Tensor*)&dv})
+        in_place(*t, q);
+      p.gate = gate.const_data_ptr(), p.dgate = dgate.mutable_data_ptr();
+      STRIDES(p, gate, gate), STRIDES(p, dgate, dgate);
+    }
+    p.q = q.const_data_ptr(), p.k = k.const_data_ptr(), p.v = v.const_data_ptr();
+    p.out = out.const_data_ptr(), p.dout = dout.const_data_ptr(), p.lse = (const float*)lse.const_data_ptr();
+    p.dq = dq.mutable_data_ptr(), p.dk = dk.mutable_data_ptr(), p.dv = dv.mutable_data_ptr();
+    STRIDES(p, q, q), STRIDES(p, k, k), STRIDES(p, v, v), STRIDES(p, out, out), STRIDES(p, dout, dout);
+    STRIDES(p, dq, dq), STRIDES(p, dk, dk), STRIDES(p, dv, dv);
+    p.lse_stride_head = g.T;
+    if (lo.numel() > 0) {
+      shaped(lo, g.T, g.hq, g.d);
+      in_place(lo, q);
+      p.out_lo = lo.const_data_ptr(), STRIDES(p, out_lo, lo);
+    }
+    if (flag.numel() > 0) {
+      need(flag.scalar_type() == at::kInt && flag.device() == q.device());
+      p.split_flag = flag.const_data_ptr<int32_t>();
+    }
+    p.dq_key_chunks = truth(a[17]);
+    p.dscore_limit_bytes = (size_t)PyLong_AsUnsignedLongLong(a[18]);
+    if (p.dscore_limit_bytes > 0) need(lib.bwd_dscore_bytes(&p) <= (size_t)PyLong_AsUnsignedLongLong(a[19]));
+    p.workspace_bytes = lib.bwd_workspace_size(&p);
+    at::Tensor ws = workspace(a[22], p.workspace_bytes, a[1]);
+    p.workspace = ws.mutable_data_ptr();
+    launch(lib.bwd, p, stream(a[23]));
+    return wrap({dq, dk, dv});
+  });
+}
+
+// rope(x, cos, sin, inverse, out_or_None, stream) -> out
+PyObject* py_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 6, [&]() -> PyObject* {
+    const at::Tensor &x = tensor(a[0]), &cos = tensor(a[1]), &sin = tensor(a[2]);
+    need(x.is_cuda() && x.dim() == 3 && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat));
+    in_place(x, x);
+    const int64_t T = x.size(0), d = x.size(2);
+    need(T <= 0x7fffffff && x.size(1) > 0);
+    for (const at::Tensor* t : {&cos, &sin})
+      need(t->dim() == 2 && t->size(0) == T && t->size(1) == d && t->scalar_type() == at::kFloat &&
+           t->device() == x.device() && t->stride(1) == 1 && t->stride(0) == cos.stride(0) && t->stride(0) % 4 == 0 &&
+           (uintptr_t)t->const_data_ptr() % 16 == 0);
+    at::Tensor out;
+    if (is_none(a[4])) {
+      out = empty({T, x.size(1), d}, x, x.scalar_type());
+    } else {
+      out = tensor(a[4]);
+      shaped(out, T, x.size(1), d);
+      in_place(out, x);
+    }
+    MimirRopeParams p = {};
+    p.x = x.const_data_ptr(), p.y = out.mutable_data_ptr();
+    p.cos = cos.const_data_ptr<float>(), p.sin = sin.const_data_ptr<float>();
+    p.x_stride_token = x.stride(0), p.x_stride_head = x.stride(1);
+    p.y_stride_token = out.stride(0), p.y_stride_head = out.stride(1);
+    p.cs_stride_token = cos.stride(0);
+    p.total_tokens = (int32_t)T, p.num_heads = (int32_t)x.size(1), p.head_dim = (int32_t)d;
+    p.dtype = x.scalar_type() == at::kBFloat16 ? MIMIR_DTYPE_BFLOAT16 : MIMIR_DTYPE_FLOAT32;
+    p.inverse = truth(a[3]);
+    launch(lib.rope, p, stream(a[5]));
+    return THPVariable_Wrap(out);
+  });
+}
+
+// cache_attn(query, key, value, cache_keys, cache_values, cache_lengths, causal, batch_indices, softmax_scale,
+//            torch_empty, stream) -> out
+PyObject* py_cache_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded(n, 11, [&]() -> PyObject* {
+    const at::Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]), &ck = tensor(a[3]), &cv = tensor(a[4]);
+    const at::Tensor& lens = tensor(a[5]);
+    need(q.is_cuda() && q.scalar_type() == at::kBFloat16 && q.dim() == 4 && k.dim() == 4 && v.dim() == 4 &&
+         ck.dim() == 4 && cv.dim() == 4);
+    const int64_t B = q.size(0), S = q.size(1), hq = q.size(2), d = q.size(3), hkv = k.size(2), L = ck.size(1);
+    need(B > 0 && S > 0 && hq > 0 && hkv > 0 && hq % hkv == 0 && L > 0 && B <= 0x7fffffff && S <= 0x7fffffff &&
+         L <= 0x7fffffff && ck.size(0) <= 0x7fffffff);
+    for (const at::Tensor* t : {&k, &v}) need(t->size(0) == B && t->size(1) == S && t->size(2) == hkv && t->size(3) == d);
+    for (const at::Tensor* t : {&ck, &cv}) need(t->size(2) == hkv && t->size(3) == d && t->sizes() == ck.sizes());
+    for (const at::Tensor* t : {&q, &k, &v, &ck, &cv}) in_place(*t, q);
+    MimirCacheAttnParams p = {};
+    for (PyObject* o : {a[5], a[7]}) {
+      if (is_none(o)) continue;
+      const at::Tensor& t = tensor(o);
+      need(t.dim() == 1 && t.size(0) == B && t.device() == q.device() && t.is_contiguous() &&
+           t.scalar_type() == lens.scalar_type() && (t.scalar_type() == at::kLong || t.scalar_type() == at::kInt));
+    }
+    p.cache_lengths = lens.const_data_ptr();
+    if (!is_none(a[7])) p.batch_indices = tensor(a[7]).const_data_ptr();
+    p.index_int64 = lens.scalar_type() == at::kLong;
+    at::Tensor out = empty({B, S, hq, d}, q, at::kBFloat16);
+    p.q = q.const_data_ptr(), p.k_new = k.const_data_ptr(), p.v_new = v.const_data_ptr();
+    p.cache_k = ck.mutable_data_ptr(), p.cache_v = cv.mutable_data_ptr(), p.out = out.mutable_data_ptr();
+#define STRIDES4(name, t) p.name##_stride_batch = (t).stride(0), p.name##_stride_token = (t).stride(1), p.name##_stride_head = (t).stride(2)
+    STRIDES4(q, q), STRIDES4(kn, k), STRIDES4(vn, v), STRIDES4(ck, ck), STRIDES4(cv, cv), STRIDES4(out, out);
+    p.batch = (int32_t)B, p.seqlen = (int32_t)S, p.cache_len = (int32_t)L, p.cache_rows = (int32_t)ck.size(0);
+    p.max_kv_len = (int32_t)L, p.num_q_heads = (int32_t)hq, p.num_kv_heads = (int32_t)hkv, p.head_dim = (int32_t)d;
+    p.causal = truth(a[6]);
+    p.dtype = MIMIR_DTYPE_BFLOAT16;
+    p.softmax_scale = (float)PyFloat_AsDouble(a[8]);
+    p.workspace_bytes = lib.cache_workspace(&p);
+    at::Tensor ws;
+    if (p.workspace_bytes > 0) {
+      ws = workspace(a[9], p.workspace_bytes, a[0]);
+      p.workspace = ws.mutable_data_ptr();
+    }
+    launch(lib.cache_attn, p, stream(a[10]));
+    return THPVariable_Wrap(out);
+  });
+}
+
+// bind(path): the entry points of the (already loaded) C-ABI library.
+PyObject* py_bind(PyObject*, PyObject* path) {
+  const char* file = PyUnicode_AsUTF8(path);
+  if (file == nullptr) return nullptr;
+  void* h = dlopen(file, RTLD_NOW | RTLD_LOCAL);
+  if (h == nullptr) return PyErr_Format(PyExc_ImportError, "%s", dlerror());
+  bool ok = true;
+  auto get = [&](auto& f, const char* name) {
+    f = (std::remove_reference_t<decltype(f)>)dlsym(h, name);
+    ok = ok && f != nullptr;
+  };
+  get(lib.fwd, "mimir_prefixlm_fwd");
+  get(lib.fwd_workspace_size, "mimir_prefixlm_fwd_workspace_size");
+  get(lib.fwd_workspace_bytes, "mimir_prefixlm_fwd_workspace_bytes");
+  get(lib.bwd, "mimir_prefixlm_bwd");
+  get(lib.bwd_workspace_size, "mimir_prefixlm_bwd_workspace_size");
+  get(lib.bwd_dscore_bytes, "mimir_prefixlm_bwd_dscore_bytes");
+  get(lib.rope, "mimir_prefixlm_rope");
+  get(lib.cache_attn, "mimir_prefixlm_cache_attn");
+  get(lib.cache_workspace, "mimir_prefixlm_cache_attn_workspace_bytes");
+  if (!ok) return PyErr_Format(PyExc_ImportError, "%s lacks an entry point", file);
+  Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"bind", py_bind, METH_O, nullptr},
+    {"fwd", (PyCFunction)(void*)py_fwd, METH_FASTCALL, nullptr},
+    {"bwd", (PyCFunction)(void*)py_bwd, METH_FASTCALL, nullptr},
+    {"rope", (PyCFunction)(void*)py_rope, METH_FASTCALL, nullptr},
+    {"cache_attn", (PyCFunction)(void*)py_cache_attn, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host_calls() { return PyModule_Create(&module); }

@@ -66,6 +66,9 @@ def rope(x: Tensor, cos: Tensor, sin: Tensor, *, inverse: bool = False, out: Opt
     head_dim stride; by default a new tensor is returned.
     """
     P._check_device_tensor("x", x)
+    res = _capi.host().rope(x, cos, sin, inverse, out, P._stream(x.device))
+    if res is not None:
+        return res if out is None else out
     if x.dim() != 3:
         raise ValueError(f"x must be [tokens, heads, head_dim], got shape {tuple(x.shape)}")
     if x.dtype not in _DTYPES:
@@ -129,13 +132,21 @@ class _GatedAttention(torch.autograd.Function):
         # bf16: the split decision and, when the kernels split, the low half of the
         # attention output (for the backward's delta row sums)
         lo = P._wants_lo(y)
-        out_lo = torch.empty_like(y) if lo else y.new_empty(0)
-        flag = torch.empty(1 if bf16 else 0, dtype=torch.int32, device=y.device)
-        p, out, lse, keep = P.prepare_fwd(q_in if fused else q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens,
-                                          total_seqlen, numseqs, max_seqlen_all, softmax_scale, gate=gate,
-                                          gated_out=y, out_lo=out_lo if lo else None, split_flag=flag,
-                                          rope=(cos, sin) if fused else None, q_rope=q if fused else None)
-        _capi.raise_for_status(lib, lib.mimir_prefixlm_fwd(ctypes.byref(p), P._stream(y.device)))
+        res = None
+        if not fused and not P._validate_metadata:
+            res = _capi.host().fwd(q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen, numseqs,
+                                   max_seqlen_all, softmax_scale, P._split_mode, P._key_chunks, lo, gate, y,
+                                   torch.empty, P._stream(y.device))
+        if res is not None:
+            out, lse, out_lo, flag = res
+        else:
+            out_lo = torch.empty_like(y) if lo else y.new_empty(0)
+            flag = torch.empty(1 if bf16 else 0, dtype=torch.int32, device=y.device)
+            p, out, lse, keep = P.prepare_fwd(q_in if fused else q, k, v, is_causal, prefix_lens, causal_lens,
+                                              cu_seqlens, total_seqlen, numseqs, max_seqlen_all, softmax_scale,
+                                              gate=gate, gated_out=y, out_lo=out_lo if lo else None, split_flag=flag,
+                                              rope=(cos, sin) if fused else None, q_rope=q if fused else None)
+            _capi.raise_for_status(lib, lib.mimir_prefixlm_fwd(ctypes.byref(p), P._stream(y.device)))
         ctx.save_for_backward(gqkv, q, k, out, lse, out_lo, flag, cos, sin, prefix_lens, causal_lens, cu_seqlens)
         ctx.meta = (hq, hkv, is_causal, total_seqlen, numseqs, max_seqlen_all, softmax_scale)
         return y.reshape(*gqkv.shape[:-1], hq * d)
@@ -150,11 +161,18 @@ class _GatedAttention(torch.autograd.Function):
         dgate, dq, dk, dv = dg3[:, :hq], dg3[:, hq:2 * hq], dg3[:, 2 * hq:2 * hq + hkv], dg3[:, 2 * hq + hkv:]
         dy3 = dy.reshape(T, hq, d)
         fused = gqkv.dtype == torch.bfloat16 and cos is not None and "bwd" in _ROPE_IN_KERNELS
-        p, dq, dk, dv, keep = P.prepare_bwd(dy3, q, k, v, out, lse, is_causal, prefix_lens, causal_lens, cu_seqlens,
-                                            total_seqlen, numseqs, max_seqlen_all, softmax_scale, gate=gate,
-                                            dgate=dgate, dq=dq, dk=dk, dv=dv, out_lo=out_lo, split_flag=flag,
-                                            rope=(cos, sin) if fused else None)
-        _capi.raise_for_status(lib, lib.mimir_prefixlm_bwd(ctypes.byref(p), P._stream(dg3.device)))
+        res = None
+        if not fused:
+            res = _capi.host().bwd(dy3, q, k, v, out, lse, out_lo, flag, is_causal, prefix_lens, causal_lens, cu_seqlens,
+                                   total_seqlen, numseqs, max_seqlen_all, softmax_scale, P._split_mode, P._key_chunks,
+                                   P._dscore_limit_bytes, P._total_device_bytes(q.device) // 64, gate,
+                                   (dgate, dq, dk, dv), torch.empty, P._stream(dg3.device))
+        if res is None:
+            p, dq, dk, dv, keep = P.prepare_bwd(dy3, q, k, v, out, lse, is_causal, prefix_lens, causal_lens, cu_seqlens,
+                                                total_seqlen, numseqs, max_seqlen_all, softmax_scale, gate=gate,
+                                                dgate=dgate, dq=dq, dk=dk, dv=dv, out_lo=out_lo, split_flag=flag,
+                                                rope=(cos, sin) if fused else None)
+            _capi.raise_for_status(lib, lib.mimir_prefixlm_bwd(ctypes.byref(p), P._stream(dg3.device)))
         if cos is not None and not fused:
             dqk = dg3[:, hq:2 * hq + hkv]  # dQ and dK, adjacent: one pass maps both back
             rope(dqk, cos, sin, inverse=True, out=dqk)

@@ -346,6 +346,12 @@ def _fwd_impl(q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens, total_se
     # bf16: the split decision and, when it splits, the output's low half (for the
     # backward's delta = rowsum(dO * O)); float32 needs neither
     lo = _wants_lo(q)
+    if q.is_cuda and not _validate_metadata:
+        res = _capi.host().fwd(q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen, numseqs,
+                               max_seqlen_all, softmax_scale, _split_mode, _key_chunks, lo, None, None, torch.empty,
+                               _stream(q.device))
+        if res is not None:
+            return res
     out_lo = torch.empty(q.shape, dtype=q.dtype, device=q.device) if lo else q.new_empty(0)
     flag = torch.empty(1 if q.dtype == torch.bfloat16 else 0, dtype=torch.int32, device=q.device)
     p, out, lse, keep = prepare_fwd(q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen,
@@ -464,6 +470,13 @@ def _free_device_bytes(device) -> int:
 def _bwd_impl(dout, q, k, v, out, lse, out_lo, split_flag, is_causal, prefix_lens, causal_lens, cu_seqlens,
               total_seqlen, numseqs, max_seqlen_all, softmax_scale):
     lib = _capi.load()
+    if q.is_cuda:
+        res = _capi.host().bwd(dout, q, k, v, out, lse, out_lo, split_flag, is_causal, prefix_lens, causal_lens,
+                               cu_seqlens, total_seqlen, numseqs, max_seqlen_all, softmax_scale, _split_mode,
+                               _key_chunks, _dscore_limit_bytes, _total_device_bytes(q.device) // 64, None, None,
+                               torch.empty, _stream(q.device))
+        if res is not None:
+            return res
     p, dq, dk, dv, keep = prepare_bwd(dout, q, k, v, out, lse, is_causal, prefix_lens, causal_lens, cu_seqlens,
                                       total_seqlen, numseqs, max_seqlen_all, softmax_scale, out_lo=out_lo,
                                       split_flag=split_flag)
@@ -538,7 +551,10 @@ class PrefixLMAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen, numseqs,
                 max_seqlen_all, softmax_scale):
-        fwd = _fwd_impl if _direct(q) else _prefixlm_fwd_op
+        direct = _direct(q)
+        if direct:  # no zeros for lse's gradient (a fill launch per step); not under tracing
+            ctx.set_materialize_grads(False)
+        fwd = _fwd_impl if direct else _prefixlm_fwd_op
         out, lse, out_lo, flag = fwd(q, k, v, is_causal, prefix_lens, causal_lens, cu_seqlens, total_seqlen,
                                      numseqs, max_seqlen_all, softmax_scale)
         ctx.save_for_backward(q, k, v, out, lse, out_lo, flag, prefix_lens, causal_lens, cu_seqlens, total_seqlen,
