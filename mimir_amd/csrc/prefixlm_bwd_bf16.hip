@@ -113,7 +113,7 @@ hipError_t launch(const MimirPrefixLMBwdParams& p, Prologue pro, hipStream_t str
     pro.has_delta = 1;
     // both tile lists: the dK/dV stage reads kind 1, the dQ stage kind 0
     PlanArgs pk = plan_args(p.cu_seqlens, p.prefix_lens, p.numseqs, p.total_seqlen, p.is_causal, p.total_tokens,
-                            /*kind=*/1, a.group, a.cap_k, a.plan_k);
+                            p.max_seqlen_all, /*kind=*/1, a.group, a.cap_k, a.plan_k);
     if (D == 128 && ws.pair_heads >= a.Hkv) {  // the paired kernel (one workgroup per CU) adds split partials
       pk.split_heads = a.Hkv;
       pk.max_pairs = ws.pair_heads / a.Hkv;
@@ -127,7 +127,7 @@ hipError_t launch(const MimirPrefixLMBwdParams& p, Prologue pro, hipStream_t str
     pk.n_zero = ws.pair_heads + kCounterWordsAfterPairs;
     pro.plan[pro.nplan++] = pk;
     PlanArgs pq = plan_args(p.cu_seqlens, p.prefix_lens, p.numseqs, p.total_seqlen, p.is_causal, p.total_tokens,
-                            /*kind=*/2, a.group, a.cap_q, a.plan_q);
+                            p.max_seqlen_all, /*kind=*/2, a.group, a.cap_q, a.plan_q);
     if (ws.chunk_slots > 0) {  // key-range parts on small grids
       pq.split_heads = a.Hq;
       pq.slots = kChunkWgs;

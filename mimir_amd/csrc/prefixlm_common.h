@@ -504,6 +504,7 @@ struct PlanArgs {
   // parts stay within max_pairs); kind 1: a split item's first half in percent of
   // the per-CU average (0: half its steps)
   int span_pct;
+  int buckets_per_thread;  // cost buckets of the counting sort, per planner thread
   int* zero;  // n_zero int32 set to 0 (the consumer's counters)
   int n_zero;
 };
@@ -721,7 +722,7 @@ struct Prologue {
 };
 
 PlanArgs plan_args(const int32_t* cu_seqlens, const int32_t* prefix_lens, int numseqs, int total_seqlen,
-                   int is_causal, int total_tokens, int kind, int group, int cap, void* items);
+                   int is_causal, int total_tokens, int max_seqlen_all, int kind, int group, int cap, void* items);
 // Compute units of the current device (cached per device).
 int device_cu_count();
 

@@ -583,7 +583,7 @@ hipError_t launch(const MimirPrefixLMFwdParams& p, Prologue pro, hipStream_t str
   a.chunk_part = chunks ? (char*)p.workspace + ws.part : nullptr;
   if (cap > 0) {
     pro.plan[pro.nplan] = plan_args(p.cu_seqlens, p.prefix_lens, p.numseqs, p.total_seqlen, p.is_causal,
-                                    p.total_tokens, /*kind=*/2, a.group, cap, plan);
+                                    p.total_tokens, p.max_seqlen_all, /*kind=*/2, a.group, cap, plan);
     if (chunks) {
       pro.plan[pro.nplan].split_heads = p.num_q_heads;
       pro.plan[pro.nplan].slots = kChunkWgs;

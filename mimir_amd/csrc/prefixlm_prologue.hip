@@ -42,9 +42,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-constexpr int kPlanBuckets = 4096;  // costs above kPlanBuckets - 1 share the last bucket
-constexpr int kBucketsPerThread = kPlanBuckets / kThreads;
-constexpr int kFillRows = 16;
+constexpr int kPlanBuckets = 4096;  // cost buckets at most; higher costs share the last one
 constexpr int kFillWgs = 128;  // fill workgroups per target, at most
 
 struct PrologueArgs {
@@ -89,13 +87,17 @@ __device__ __forceinline__ int item_cost(int p, int nq, int kind, int group, int
   return nq > q0 ? group * ((nq - q0 + 63) / 64) : 0;
 }
 
-__device__ __forceinline__ int bucket_of(int cost) { return min(cost, kPlanBuckets - 1); }
-// LDS slot of bucket b: one padding word every 16 buckets, so that the 16
+// LDS slot of bucket b: one padding word every 16 buckets, so that the up to 16
 // consecutive buckets each thread owns in bucket_starts sit in distinct banks
 // across the wave.
 constexpr int kHistSlots = kPlanBuckets + kPlanBuckets / 16;
 __device__ __forceinline__ int bucket_slot(int b) { return b + (b >> 4); }
-__device__ __forceinline__ int hist_slot(int cost) { return bucket_slot(bucket_of(cost)); }
+// The list's buckets: a.buckets_per_thread for each thread, enough for the costs
+// its longest sequence can have.
+__device__ __forceinline__ int buckets_of(const PlanArgs& a) { return a.buckets_per_thread * kThreads; }
+__device__ __forceinline__ int hist_slot(const PlanArgs& a, int cost) {
+  return bucket_slot(min(cost, buckets_of(a) - 1));
+}
 
 struct PlanSmem {
   int hist[kHistSlots];
@@ -203,7 +205,7 @@ __device__ double walk_items(const PlanArgs& a, PlanSmem& sm, int cut, int span 
         if (kScatter) slot = wave_alloc(&sm.pairs, n);
         // the span-tile parts of every cut item share one bucket: one LDS atomic
         // per wave (per-lane atomics on one word serialize)
-        spos = wave_alloc(&sm.hist[hist_slot(span)], n > 0 ? n - 1 : 0);
+        spos = wave_alloc(&sm.hist[hist_slot(a, span)], n > 0 ? n - 1 : 0);
       } else if (kScatter && a.kind != 2 && cut != 0x7fffffff) {  // uniform
         slot = wave_alloc(&sm.pairs, valid && a.kind == 1 && c >= cut ? 1 : 0);
       }
@@ -212,30 +214,30 @@ __device__ double walk_items(const PlanArgs& a, PlanSmem& sm, int cut, int span 
         const int c0 = c - (parts - 1) * span;  // the first part's tiles, the others `span`
         const int z = (parts << 8) | (span << 16);
         if constexpr (kScatter) {  // parts 1.. take consecutive positions; every part its slot
-          put_item(a, atomicAdd(&sm.hist[hist_slot(c0)], 1), base + j, t, z, slot);
+          put_item(a, atomicAdd(&sm.hist[hist_slot(a, c0)], 1), base + j, t, z, slot);
           for (int q = 1; q < parts; ++q) put_item(a, spos + q - 1, base + j, t, q | z, slot + q);
         } else {
-          atomicAdd(&sm.hist[hist_slot(c0)], 1);
+          atomicAdd(&sm.hist[hist_slot(a, c0)], 1);
         }
       } else if (a.kind == 2) {
         if constexpr (kScatter) {
-          put_item(a, atomicAdd(&sm.hist[hist_slot(c)], 1), base + j, t, 1 << 8, -1);
+          put_item(a, atomicAdd(&sm.hist[hist_slot(a, c)], 1), base + j, t, 1 << 8, -1);
         } else {
-          atomicAdd(&sm.hist[hist_slot(c)], 1);
+          atomicAdd(&sm.hist[hist_slot(a, c)], 1);
         }
       } else if (c >= cut) {
         const int c1 = span > 0 ? span : c / 2, c2 = c - c1;
         if constexpr (kScatter) {  // half | first step of half 2 << 8 (0: the middle)
-          put_item(a, atomicAdd(&sm.hist[hist_slot(c1)], 1), base + j, t, 1 | (span << 8), slot);
-          put_item(a, atomicAdd(&sm.hist[hist_slot(c2)], 1), base + j, t, 2 | (span << 8), slot);
+          put_item(a, atomicAdd(&sm.hist[hist_slot(a, c1)], 1), base + j, t, 1 | (span << 8), slot);
+          put_item(a, atomicAdd(&sm.hist[hist_slot(a, c2)], 1), base + j, t, 2 | (span << 8), slot);
         } else {
-          atomicAdd(&sm.hist[hist_slot(c1)], 1);
-          atomicAdd(&sm.hist[hist_slot(c2)], 1);
+          atomicAdd(&sm.hist[hist_slot(a, c1)], 1);
+          atomicAdd(&sm.hist[hist_slot(a, c2)], 1);
         }
       } else if constexpr (kScatter) {
-        put_item(a, atomicAdd(&sm.hist[hist_slot(c)], 1), base + j, t, 0, -1);
+        put_item(a, atomicAdd(&sm.hist[hist_slot(a, c)], 1), base + j, t, 0, -1);
       } else {
-        atomicAdd(&sm.hist[hist_slot(c)], 1);
+        atomicAdd(&sm.hist[hist_slot(a, c)], 1);
       }
     }
     __syncthreads();  // the chunk arrays are rewritten by the next chunk
@@ -243,27 +245,27 @@ __device__ double walk_items(const PlanArgs& a, PlanSmem& sm, int cut, int span 
   return cost_sum;
 }
 
+__device__ __forceinline__ void clear_hist(const PlanArgs& a, PlanSmem& sm) {
+  for (int i = threadIdx.x; i <= bucket_slot(buckets_of(a) - 1); i += kThreads) sm.hist[i] = 0;
+}
+
 // Turns the bucket counts into start positions in descending cost order
 // (bucket c starts after all items of cost > c) and returns the item count.
-// Thread i owns buckets kPlanBuckets-1-16i down to kPlanBuckets-16-16i.  With
+// Thread i owns its share of consecutive buckets, counted from the last one down.  With
 // `max_pairs` > 0 it also finds the split cut: the smallest bucket above
 // `threshold` whose items and all heavier ones number at most max_pairs.
-__device__ int bucket_starts(PlanSmem& sm, double threshold, int max_pairs) {
-  int cnt[kBucketsPerThread];
+__device__ int bucket_starts(const PlanArgs& a, PlanSmem& sm, double threshold, int max_pairs) {
+  const int bpt = a.buckets_per_thread;
+  const int b0 = buckets_of(a) - 1 - bpt * (int)threadIdx.x;
   int local = 0;
-#pragma unroll
-  for (int j = 0; j < kBucketsPerThread; ++j) {
-    cnt[j] = sm.hist[bucket_slot(kPlanBuckets - 1 - (kBucketsPerThread * threadIdx.x + j))];
-    local += cnt[j];
-  }
+  for (int j = 0; j < bpt; ++j) local += sm.hist[bucket_slot(b0 - j)];
   int total;
   int run = block_exclusive_scan(local, sm.wave_sums, total);
   int cut = 0x7fffffff;
-#pragma unroll
-  for (int j = 0; j < kBucketsPerThread; ++j) {
-    const int b = kPlanBuckets - 1 - (kBucketsPerThread * threadIdx.x + j);
+  for (int j = 0; j < bpt; ++j) {
+    const int b = b0 - j, n = sm.hist[bucket_slot(b)];
     sm.hist[bucket_slot(b)] = run;  // becomes the next free position of bucket b
-    run += cnt[j];     // items of cost >= b
+    run += n;                       // items of cost >= b
     if (max_pairs > 0 && (double)b > threshold && run <= max_pairs) cut = b;
   }
   if (max_pairs > 0) {  // uniform
@@ -307,7 +309,7 @@ __device__ __forceinline__ SeqGeom prefetch_seq(const PlanArgs& a) {
 
 __device__ void plan_block_chunks(const PlanArgs& a, PlanSmem& sm) {
   const SeqGeom pre = prefetch_seq(a);
-  for (int i = threadIdx.x; i < kHistSlots; i += kThreads) sm.hist[i] = 0;
+  clear_hist(a, sm);
   if (threadIdx.x == 0) sm.pairs = 0;
   for (int i = threadIdx.x; i < a.n_zero; i += kThreads) a.zero[i] = 0;
   __syncthreads();
@@ -320,11 +322,11 @@ __device__ void plan_block_chunks(const PlanArgs& a, PlanSmem& sm) {
     // small grid: recount with the cut items' parts (the first counts are not used)
     const double target = block_sum(mine, sm) * a.split_heads / a.slots * (a.span_pct < 100 ? 100 : a.span_pct) / 100.0;
     span = target > (double)kChunkMinCost ? (int)ceil(target) : kChunkMinCost;
-    for (int i = threadIdx.x; i < kHistSlots; i += kThreads) sm.hist[i] = 0;
+    clear_hist(a, sm);
     __syncthreads();
     walk_items<false>(a, sm, 0x7fffffff, span, reuse);
   }
-  total = bucket_starts(sm, 0.0, 0);
+  total = bucket_starts(a, sm, 0.0, 0);
   walk_items<true>(a, sm, 0x7fffffff, span, reuse);
   for (int i = total + threadIdx.x; i < a.cap; i += kThreads) put_item(a, i, -1, -1, 0, -1);
 }
@@ -337,7 +339,7 @@ __device__ void plan_block(const PlanArgs& a) {
   }
   const bool split = a.kind == 1 && a.split_heads > 0 && a.max_pairs > 0 && a.slots > 0;
   const SeqGeom pre = prefetch_seq(a);
-  for (int i = threadIdx.x; i < kHistSlots; i += kThreads) sm.hist[i] = 0;
+  clear_hist(a, sm);
   if (threadIdx.x == 0) {
     sm.cut = 0x7fffffff;
     sm.pairs = 0;
@@ -356,13 +358,13 @@ __device__ void plan_block(const PlanArgs& a) {
       threshold = avg / 2.0;
     }
   }
-  int total = bucket_starts(sm, threshold, split ? a.max_pairs : 0);
+  int total = bucket_starts(a, sm, threshold, split ? a.max_pairs : 0);
   const int cut = sm.cut;  // > threshold: a split item's halves are non-empty
   if (cut != 0x7fffffff) {  // recount with the heavy items split
-    for (int i = threadIdx.x; i < kHistSlots; i += kThreads) sm.hist[i] = 0;
+    clear_hist(a, sm);
     __syncthreads();
     walk_items<false>(a, sm, cut, span, a.numseqs <= kThreads);
-    total = bucket_starts(sm, 0.0, 0);
+    total = bucket_starts(a, sm, 0.0, 0);
   }
   walk_items<true>(a, sm, cut, span, a.numseqs <= kThreads);
   for (int i = total + threadIdx.x; i < a.cap; i += kThreads) put_item(a, i, -1, -1, 0, -1);
@@ -508,9 +510,12 @@ __device__ void kscan_block(const KScanArgs& a, int b) {
 
 // Zeroes the padding rows of one tensor: the rows t < first or t >= last of
 // the packed rows, first = cu_seqlens[0], last = min(cu_seqlens[numseqs],
-// total_seqlen).  The fill_blocks workgroups of the target take 16-row chunks
-// of those rows in turn, so a batch without padding costs one bounded set of
-// workgroups that exit at once, not one per 16 rows of T.
+// total_seqlen).  The threads of the target's fill_blocks workgroups take the
+// 16-byte units of those rows in turn, so a batch without padding costs one
+// bounded set of workgroups that exit at once and a hundred padding rows are a
+// store or two per thread (dealt as 16-row chunks of 4-byte stores they kept seven
+// workgroups busy for 10 us: prologue of 100 padding rows x 16 heads 16.7 -> 5.7
+// us).  Rows are 16-byte aligned (the C ABI checks it).
 __device__ void fill_block(const FillArgs& a, int b, int fill_blocks) {
   int first = a.numseqs > 0 ? a.cu_seqlens[0] : a.T;
   int last = a.numseqs > 0 ? a.cu_seqlens[a.numseqs] : 0;
@@ -518,19 +523,18 @@ __device__ void fill_block(const FillArgs& a, int b, int fill_blocks) {
   if (last > a.total_seqlen) last = a.total_seqlen;
   last = last < first ? first : (last > a.T ? a.T : last);
   const int n_pad = first + (a.T - last);  // padding row j: j < first ? j : last + (j - first)
-  const int chunks = a.row_bytes / 4;      // row_bytes is a multiple of 4
-  for (int j0 = b * kFillRows; j0 < n_pad; j0 += fill_blocks * kFillRows) {
-    for (int i = threadIdx.x; i < kFillRows * a.H * chunks; i += kThreads) {
-      const int tt = i / (a.H * chunks);
-      const int rem = i % (a.H * chunks);
-      const int h = rem / chunks, c = rem % chunks;
-      const int j = j0 + tt;
-      if (j >= n_pad) continue;
-      const int t = j < first ? j : last + (j - first);
-      char* row = (char*)a.x + ((int64_t)t * a.st + (int64_t)h * a.sh) * a.elem_bytes;
-      ((uint32_t*)row)[c] = 0u;
-      if (c == 0 && a.lse != nullptr) a.lse[(int64_t)h * a.lse_sh + t] = -INFINITY;
-    }
+  if (n_pad == 0) return;
+  const uint32_t chunks = (uint32_t)a.row_bytes / 16u;  // head_dim is a multiple of 32
+  const uint32_t per_row = (uint32_t)a.H * chunks;
+  const int64_t total = (int64_t)n_pad * per_row;
+  for (int64_t i = (int64_t)b * kThreads + threadIdx.x; i < total; i += (int64_t)fill_blocks * kThreads) {
+    const int j = total <= 0x7fffffff ? (int)((uint32_t)i / per_row) : (int)(i / per_row);
+    const uint32_t rem = (uint32_t)(i - (int64_t)j * per_row);
+    const uint32_t h = rem / chunks, c = rem - h * chunks;
+    const int t = j < first ? j : last + (j - first);
+    char* row = (char*)a.x + ((int64_t)t * a.st + (int64_t)h * a.sh) * a.elem_bytes;
+    ((i32x4*)row)[c] = i32x4{0, 0, 0, 0};
+    if (c == 0 && a.lse != nullptr) a.lse[(int64_t)h * a.lse_sh + t] = -INFINITY;
   }
 }
 
@@ -582,7 +586,8 @@ KScanArgs kscan_args(const bf16_t* k, int64_t k_st, int64_t k_sh, int T, int Hkv
 }
 
 PlanArgs plan_args(const int32_t* cu_seqlens, const int32_t* prefix_lens, int numseqs, int total_seqlen,
-                   int is_causal, int total_tokens, int kind, int group, int cap, void* items) {
+                   int is_causal, int total_tokens, int max_seqlen_all, int kind, int group, int cap,
+                   void* items) {
   PlanArgs a;
   a.cu_seqlens = cu_seqlens;
   a.prefix_lens = prefix_lens;
@@ -594,6 +599,12 @@ PlanArgs plan_args(const int32_t* cu_seqlens, const int32_t* prefix_lens, int nu
   a.group = group;
   a.cap = cap;
   a.items = items;
+  // Buckets for the costs of sequences up to max_seqlen_all (a longer one's share the
+  // last bucket: out of order, still listed).  Clearing and scanning all 4096 took
+  // about a microsecond (forward prologue of 24576 tokens, 2 heads: 10.0 -> 9.0 us).
+  const int longest = max_seqlen_all < total_tokens ? max_seqlen_all : total_tokens;
+  const int64_t costs = (int64_t)(kind == 1 ? group : 1) * ((longest + 63) / 64) + 1;
+  a.buckets_per_thread = (int)(costs < kPlanBuckets ? (costs + kThreads - 1) / kThreads : kPlanBuckets / kThreads);
   a.split_heads = 0;
   a.max_pairs = 0;
   a.slots = 0;
@@ -691,8 +702,8 @@ hipError_t launch_prologue(const Prologue& pro, hipStream_t stream) {
   for (int i = 0; i < pro.nfill; ++i)
     if (pro.fill[i].T > 0 && pro.fill[i].H > 0) {
       a.fill[a.nfill++] = pro.fill[i];
-      // every target has the same T; at most kFillWgs workgroups each
-      const int rows = (pro.fill[i].T + kFillRows - 1) / kFillRows;
+      // every target has the same T: a workgroup per 16 rows, at most kFillWgs
+      const int rows = (pro.fill[i].T + 15) / 16;
       a.fill_blocks = rows < kFillWgs ? rows : kFillWgs;
     }
   const int64_t blocks = (int64_t)a.nplan + a.delta_blocks + a.kscan_blocks + (int64_t)a.nfill * a.fill_blocks;
