@@ -218,6 +218,36 @@ def test_f32_tile_edges(device, d, hq, hkv, causal):
         assert torch.equal(x.detach().cpu(), got[name]), name
 
 
+@pytest.mark.parametrize("lead,tail", [(1, 0), (37, 300), (0, 2500)])
+@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (32, torch.float32)], ids=["bf16", "fp32"])
+def test_padding_rows_before_and_after(device, lead, tail, d, dtype):
+    """Padding rows in front of the first sequence and behind the last (more than a turn of the
+    fill's workgroups): zeros and -inf there, the sequences' rows bitwise as without padding."""
+    case = make_case([70, 129], [30, 0], 6, 2, d, seed=61, dtype=dtype)
+    base = run_gpu(case, device)
+    pad = lambda t: torch.cat((torch.ones(lead, *t.shape[1:], dtype=dtype), t, torch.ones(tail, *t.shape[1:], dtype=dtype)))
+    T = lead + case.T + tail
+    wide = make_case([70, 129], [30, 0], 6, 2, d, seed=61, dtype=dtype, pad_to=T)
+    wide.q, wide.k, wide.v, wide.dout = (pad(t) for t in (case.q, case.k, case.v, case.dout))
+    wide.cu_seqlens[:3] += lead
+    wide.total_seqlen = wide.total_seqlen + lead
+    got = run_gpu(wide, device)
+    rows = slice(lead, lead + case.T)
+    for key in ("o", "dq", "dk", "dv"):
+        assert torch.equal(got[key][rows], base[key]), key
+        assert torch.count_nonzero(got[key]) == torch.count_nonzero(base[key]), key
+    assert torch.equal(got["lse"][:, rows], base["lse"])
+    assert torch.isneginf(got["lse"]).sum() == 6 * (lead + tail)
+
+
+def test_costs_above_the_planner_buckets(device):
+    """An understated max_seqlen_all sizes the planner's cost buckets too small (64 tokens: 256
+    buckets, while the first key tiles cost 8 x 36): those items share the last bucket."""
+    case = make_case([2300, 100], [2000, 0], 8, 1, 128, seed=62, dtype=torch.bfloat16)
+    case.max_seqlen_all = torch.tensor(64)
+    check(case, device, label="buckets")
+
+
 def test_config1_fp32_forward(device):
     case = make_config(1, seed=0)
     check(case, device, backward=False, label="cfg1")
