@@ -366,9 +366,8 @@ int mimir_prefixlm_rope(const MimirRopeParams* params, void* stream);
  * max_kv_len is an upper bound of max_b(c + S) (the reference's
  * kv_len.max().item(), layers.py:143) that sizes the key split; the split itself
  * follows the batch rows' own lengths.  bf16 only, head_dim 64 or 128.
- * The workspace holds the split partial results and, for more than 32 query rows
- * per kv head, one arrival counter per (batch row, kv head, 128-row tile), which
- * the call clears itself (no memset: the call can be captured in a graph). */
+ * The workspace holds the partial results of the split (no counters and no memset:
+ * the call can be captured in a graph). */
 typedef struct MimirCacheAttnParams {
   const void* q;              /* [B, S, Hq, D] */
   const void* k_new;          /* [B, S, Hkv, D] */

@@ -11,16 +11,14 @@
 //                            equal share of all key tiles of the call
 //     cache_merge_kernel     adds the partial rows of the shares
 //   otherwise:
-//     cache_append_kernel    the scatter of k_new / v_new into the cache rows (it
-//                            also clears the split arrival counters)
+//     cache_append_kernel    the scatter of k_new / v_new into the cache rows
 //     cache_attn_kernel      one workgroup per (batch row, kv head, 128 query rows,
 //                            key split): the G query heads of a kv head share its
 //                            K / V tiles (rows are (token, head) pairs, token-major),
 //                            64-key tiles stream through two LDS stages, S^T = K Q^T
 //                            and O^T += V^T P^T on bf16 MFMA with an online softmax
-//                            (the forward kernel's arithmetic).  With several
-//                            splits, each publishes its partial (max, sum, O) rows
-//                            and the last to arrive merges them into the output.
+//                            (the forward kernel's arithmetic)
+//     cache_merge_splits_*   with several splits: adds their partial rows
 #include "prefixlm_common.h"
 
 namespace mimir {
@@ -50,8 +48,6 @@ struct CacheArgs {
   float scale_log2;
   float* part_o;   // [unit, kRows, D] unnormalized O of each split (splits > 1)
   float* part_ml;  // [unit, kRows, 2]: running max (exp2 domain) and sum
-  int* counters;   // [B * Hkv * n_rt] split arrivals per row tile (splits > 1), cleared by the append kernel
-  int n_counters;
   int shares;      // decode: workgroups the key tiles of the call are dealt to
 };
 
@@ -69,7 +65,6 @@ __device__ __forceinline__ int cache_len_of(const CacheArgs& a, int b) {
 
 // k_new / v_new [b, i, h] -> cache [row(b), cache_lengths[b] + i, h]; 16 bytes per thread.
 __global__ __launch_bounds__(256) void cache_append_kernel(const CacheArgs a) {
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < a.n_counters; i += gridDim.x * 256) a.counters[i] = 0;
   const int chunks = a.D / 8;
   const int64_t total = (int64_t)a.B * a.S * a.Hkv * chunks;
   for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256) {
@@ -89,65 +84,77 @@ __global__ __launch_bounds__(256) void cache_append_kernel(const CacheArgs a) {
   }
 }
 
-constexpr int kDevScope = 16;  // buffer cache policy: coherent at device scope
-
-// Output rows [0, rt_rows) of row tile rt of (batch row b, kv head hk): the
-// merge of the partial (max in the exp2 domain, sum, unnormalized O) rows that
-// the n_valid splits of `group` published at slots (group * splits + c) * kRows
-// + row.  out = sum_c O_c 2^(m_c - M) / sum_c l_c 2^(m_c - M); one wave per row
-// (waves of a kWaves-wave workgroup), D / 64 columns per lane.  The splits are
-// merged online in chunks of eight whose loads ((max, sum) and the lane's O
-// columns) are all issued before any is used, so a chunk costs one memory
-// round trip.  The loads are device-coherent: the caller has seen every split
-// arrive.
-template <int D>
-__device__ void merge_split_rows(const CacheArgs& a, const __amdgpu_buffer_rsrc_t ro,
-                                 const __amdgpu_buffer_rsrc_t rml, int group, int n_valid, int b, int hk, int rt,
-                                 int rt_rows, int wave, int lane) {
-  const uint32_t unit0 = (uint32_t)group * a.splits;
-  constexpr int cpl = D / 64;
-  constexpr int kChunk = 8;
-  for (int rr = wave; rr < rt_rows; rr += kWaves) {
-    float M = -INFINITY, lsum = 0.f;
-    float acc[cpl] = {};
-    for (int c0 = 0; c0 < n_valid; c0 += kChunk) {
-      f32x2 ml[kChunk];
-      float ov[kChunk][cpl];
+// One output row (at `orow`) from its n partial rows (max in the exp2 domain, sum,
+// unnormalized O) at part_ml / part_o row slot(c), c < n:
+// out = sum_c O_c 2^(m_c - M) / sum_c l_c 2^(m_c - M).  One wave: lane c takes part
+// c's (max, sum), and the O rows are read one part per D / 4 lanes with kChunk
+// loads in flight beside it, so up to 32 parts (D 128) cost one memory round trip.
+template <int D, typename Slot>
+__device__ __forceinline__ void merge_row(const CacheArgs& a, int n, int lane, Slot&& slot, bf16_t* orow) {
+  constexpr int kLanes = D / 4;        // lanes per part row, four columns each
+  constexpr int kParts = 64 / kLanes;  // part rows per load
+  constexpr int kChunk = 16;
+  const int sub = lane / kLanes, col = lane % kLanes * 4;
+  float M = -INFINITY, lsum = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};  // this lane's columns over the parts of its lane group
+  for (int c0 = 0; c0 < n; c0 += 64) {
+    const int c = c0 + lane, in_chunk = min(n - c0, 64);
+    const int row = slot(min(c, n - 1));
+    f32x2 ml = *(const f32x2*)&a.part_ml[2 * (int64_t)row];
+    f32x4 ov[kChunk];
+    auto load_rows = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < kChunk; ++i) {
-        const uint32_t slot = (unit0 + min(c0 + i, n_valid - 1)) * kRows + rr;
-        ml[i] = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rml, slot * 8, 0, kDevScope));
-        const uint32_t off = (slot * D + lane * cpl) * 4;
-        if constexpr (cpl == 2) {
-          const f32x2 o = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(ro, off, 0, kDevScope));
-          ov[i][0] = o[0];
-          ov[i][1] = o[1];
-        } else {
-          ov[i][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ro, off, 0, kDevScope));
-        }
+        if (i0 + i * kParts >= in_chunk) break;  // uniform
+        ov[i] = *(const f32x4*)&a.part_o[(int64_t)__shfl(row, min(i0 + i * kParts + sub, in_chunk - 1), 64) * D + col];
       }
+    };
+    load_rows(0);  // in flight beside the weights
+    if (c >= n) ml = f32x2{-INFINITY, 0.f};
+    float m = ml[0];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    const float m_new = fmaxf(M, m);
+    const float alpha = M == -INFINITY ? 0.f : fast_exp2(M - m_new);
+    const float w = ml[0] == -INFINITY ? 0.f : fast_exp2(ml[0] - m_new);  // -inf: no allowed key in this part
+    float l = ml[1] * w;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) l += __shfl_xor(l, off, 64);
+    lsum = lsum * alpha + l;
+    acc *= alpha;
+    M = m_new;
+    for (int i0 = 0;;) {
 #pragma unroll
       for (int i = 0; i < kChunk; ++i) {
-        if (c0 + i >= n_valid) break;
-        const float m = ml[i][0];
-        if (m == -INFINITY) continue;  // no allowed key in this split
-        const float m_new = fmaxf(M, m);
-        const float alpha = M == -INFINITY ? 0.f : fast_exp2(M - m_new);  // rescale the running sums
-        const float w = fast_exp2(m - m_new);
-        lsum = lsum * alpha + ml[i][1] * w;
-#pragma unroll
-        for (int j = 0; j < cpl; ++j) acc[j] = acc[j] * alpha + ov[i][j] * w;
-        M = m_new;
+        if (i0 + i * kParts >= in_chunk) break;
+        const int src = i0 + i * kParts + sub;
+        const float wi = __shfl(w, min(src, 63), 64);
+        if (src < in_chunk && wi != 0.f) acc += ov[i] * wi;
       }
+      i0 += kChunk * kParts;
+      if (i0 >= in_chunk) break;
+      load_rows(i0);
     }
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-    const int row_g = rt * kRows + rr;
-    const int ti_r = row_g / a.G;
-    const int h_r = hk * a.G + (row_g - ti_r * a.G);
-    bf16_t* orow = a.out + (int64_t)b * a.o_sb + (int64_t)ti_r * a.o_st + (int64_t)h_r * a.o_sh + lane * cpl;
-#pragma unroll
-    for (int i = 0; i < cpl; ++i) orow[i] = (bf16_t)(acc[i] * inv);
   }
+#pragma unroll
+  for (int off = kLanes; off < 64; off <<= 1)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
+  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+  if (sub == 0) *(bf16x4*)&orow[col] = __builtin_convertvector(acc * inv, bf16x4);
+}
+
+// Key splits of a batch row with `keys` keys (cache_attn_kernel): tiles per split
+// and the splits that hold keys.
+struct RowSplit {
+  int per, n;
+};
+__device__ __forceinline__ RowSplit row_split(const CacheArgs& a, int keys) {
+  const int tiles = (keys + kKeys - 1) / kKeys;
+  RowSplit r;
+  r.per = max(1, (tiles + a.splits - 1) / a.splits);
+  r.n = (tiles + r.per - 1) / r.per;
+  return r;
 }
 
 template <int D>
@@ -180,9 +187,8 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
   const int kv = row_in_cache ? min(clen + a.S, a.L) : 0;  // keys of this batch row
   // This batch row's key tiles, spread evenly over the splits; n_valid splits
   // hold keys.  A row without keys (outside the cache) gets zeros from split 0.
-  const int tiles_b = (kv + kKeys - 1) / kKeys;
-  const int per = max(1, (tiles_b + a.splits - 1) / a.splits);
-  const int n_valid = (tiles_b + per - 1) / per;
+  const RowSplit rs = row_split(a, kv);
+  const int per = rs.per, n_valid = rs.n;
   if (split > 0 && split >= n_valid) return;
   const int k0 = split * per * kKeys;
   const int k1 = min(kv, k0 + per * kKeys);
@@ -335,44 +341,51 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
     return;
   }
 
-  // Several splits hold keys of this row tile: publish this split's partial
-  // rows -- unnormalized O, the max in the exp2 domain (-inf: no allowed key)
-  // and the sum -- with device-coherent stores; the last split to arrive (per
-  // row tile) reads them all back the same way and writes the merged rows.
-  // The stores are complete before the arrival count, and the loads are issued
-  // after it has returned, so no cache flush is needed.
-  const int64_t units = (int64_t)gridDim.x;
-  const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.part_o, (uint32_t)(units * kRows * D * 4));
-  const __amdgpu_buffer_rsrc_t rml = make_rsrc(a.part_ml, (uint32_t)(units * kRows * 2 * 4));
-  const int rt_rows = min(kRows, R - rt * kRows);
-  if (wave_active) {
-    const uint32_t slot = (uint32_t)blockIdx.x * kRows + wave * 32 + l32;
+  // Several splits hold keys of this row tile: this split's partial rows --
+  // unnormalized O, the max in the exp2 domain (-inf: no allowed key) and the sum.
+  if (!wave_active) return;
+  const int64_t slot = (int64_t)blockIdx.x * kRows + wave * 32 + l32;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        f32x4 t;
+    for (int rg = 0; rg < 4; ++rg) {
+      f32x4 t;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) t[e] = oacc[dt][4 * rg + e];
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, t), ro,
-                                               (slot * D + 32 * dt + 8 * rg + 4 * hi) * 4, 0, kDevScope);
-      }
-    if (hi == 0) {
-      const float m2 = m_run == -INFINITY ? -INFINITY : m_run * c2;
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, f32x2{m2, l_tot}), rml, slot * 8, 0,
-                                            kDevScope);
+      for (int e = 0; e < 4; ++e) t[e] = oacc[dt][4 * rg + e];
+      *(f32x4*)&a.part_o[slot * D + 32 * dt + 8 * rg + 4 * hi] = t;
     }
-  }
-  __asm__ volatile("" ::: "memory");
-  wait_vmem();  // the partial rows are stored
-  __shared__ int last;
-  __syncthreads();
-  const int group = blockIdx.x / a.splits;  // (batch row, kv head, row tile)
-  if (tid == 0)
-    last = __hip_atomic_fetch_add(&a.counters[group], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n_valid - 1;
-  __syncthreads();
-  if (!last) return;
-  merge_split_rows<D>(a, ro, rml, group, n_valid, b, hk, rt, rt_rows, wave, lane);
+  if (hi == 0) *(f32x2*)&a.part_ml[slot * 2] = f32x2{m_run == -INFINITY ? -INFINITY : m_run * c2, l_tot};
+}
+
+// Adds the partial rows of cache_attn_kernel's key splits, one wave per query row.
+// In the last split to arrive, four waves took the up to 128 rows of a tile in
+// turn, two round trips of device-coherent loads each: a chunk of 100 tokens on
+// 3000 cached ones (Hq 16, Hkv 4, D 128) 171 -> 27 us, of 512 on none 69 -> 29, 8 x
+// 100 on 100 to 3000 81 -> 49 (append, attention and merge together).
+template <int D>
+__device__ __forceinline__ void cache_merge_splits_body(const CacheArgs& a) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int R = a.S * a.G;
+  const int groups = (R + kWaves - 1) / kWaves;  // workgroups per (batch row, kv head)
+  const int row = blockIdx.x % groups * kWaves + wave;
+  const int pair = blockIdx.x / groups;
+  const int b = pair / a.Hkv, hk = pair - b * a.Hkv;
+  if (row >= R) return;
+  const int64_t crow = cache_row(a, b);
+  const int keys = crow >= 0 && crow < a.rows ? min(cache_len_of(a, b) + a.S, a.L) : 0;
+  const int n = row_split(a, keys).n;
+  if (n <= 1) return;  // written by its split
+  const int64_t unit0 = ((int64_t)pair * a.n_rt + row / kRows) * a.splits;
+  const int t = row / a.G;
+  merge_row<D>(a, n, lane, [&](int c) { return (int)((unit0 + c) * kRows + row % kRows); },
+               a.out + (int64_t)b * a.o_sb + (int64_t)t * a.o_st + (int64_t)(hk * a.G + row - t * a.G) * a.o_sh);
+}
+__global__ __launch_bounds__(kThreads) void cache_merge_splits_d128_kernel(const CacheArgs a) {
+  cache_merge_splits_body<128>(a);
+}
+__global__ __launch_bounds__(kThreads) void cache_merge_splits_d64_kernel(const CacheArgs a) {
+  cache_merge_splits_body<64>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -867,16 +880,9 @@ __global__ __launch_bounds__(kPairWaves * 64, 1) void cache_decode_pairs_d64_ker
 }
 
 // Output rows of the (batch row, kv head) pairs whose key tiles lie in several
-// shares: out = sum_c O_c 2^(m_c - M) / sum_c l_c 2^(m_c - M) over the parts c in
-// the order of the line; zeros for batch rows without keys (outside the cache).
-// One wave per row: lane c takes part c's (max, sum), and the O rows are read one
-// part per D / 4 lanes with kChunk loads in flight beside it, so up to 32 parts
-// (D 128) cost one memory round trip.
+// shares, one wave per row, from the parts in the order of the line.
 template <int D>
 __device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
-  constexpr int kLanes = D / 4;        // lanes per part row, four columns each
-  constexpr int kParts = 64 / kLanes;  // part rows per load
-  constexpr int kChunk = 16;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int R = a.S * a.G;
@@ -901,54 +907,9 @@ __device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
   const int g0 = before * a.Hkv + hk * units_b;  // the pair's units [g0, g0 + units_b) of the line
   const int w0 = g0 / per, n = units_b > 0 ? (g0 + units_b - 1) / per - w0 + 1 : 0;  // shares it lies in
   if (n <= 1 || rr >= R) return;  // written by its share
-  const int sub = lane / kLanes, col = lane % kLanes * 4;
-  float M = -INFINITY, lsum = 0.f;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};  // this lane's columns over the parts of its lane group
-  for (int c0 = 0; c0 < n; c0 += 64) {
-    const int c = c0 + lane, in_chunk = min(n - c0, 64);
-    const int row = part_slot(c == 0 ? g0 : (w0 + min(c, n - 1)) * per, per) * R + rr;
-    f32x2 ml = *(const f32x2*)&a.part_ml[2 * (int64_t)row];
-    f32x4 ov[kChunk];
-    auto load_rows = [&](int i0) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < kChunk; ++i)
-        ov[i] = *(const f32x4*)&a.part_o[(int64_t)__shfl(row, min(i0 + i * kParts + sub, in_chunk - 1), 64) * D + col];
-    };
-    load_rows(0);  // in flight beside the weights
-    if (c >= n) ml = f32x2{-INFINITY, 0.f};
-    float m = ml[0];
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    const float m_new = fmaxf(M, m);
-    const float alpha = M == -INFINITY ? 0.f : fast_exp2(M - m_new);
-    const float w = ml[0] == -INFINITY ? 0.f : fast_exp2(ml[0] - m_new);  // -inf: no allowed key in this part
-    float l = ml[1] * w;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) l += __shfl_xor(l, off, 64);
-    lsum = lsum * alpha + l;
-    acc *= alpha;
-    M = m_new;
-    for (int i0 = 0;;) {
-#pragma unroll
-      for (int i = 0; i < kChunk; ++i) {
-        const int src = i0 + i * kParts + sub;
-        const float wi = __shfl(w, min(src, 63), 64);
-        if (src < in_chunk && wi != 0.f) acc += ov[i] * wi;
-      }
-      i0 += kChunk * kParts;
-      if (i0 >= in_chunk) break;
-      load_rows(i0);
-    }
-  }
-#pragma unroll
-  for (int off = kLanes; off < 64; off <<= 1)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
-  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-  const int ti = rr / a.G;
-  if (sub == 0)
-    *(bf16x4*)&a.out[(int64_t)b * a.o_sb + (int64_t)ti * a.o_st + (int64_t)(hk * a.G + rr - ti * a.G) * a.o_sh + col] =
-        __builtin_convertvector(acc * inv, bf16x4);
+  const int t = rr / a.G;
+  merge_row<D>(a, n, lane, [&](int c) { return part_slot(c == 0 ? g0 : (w0 + c) * per, per) * R + rr; },
+               a.out + (int64_t)b * a.o_sb + (int64_t)t * a.o_st + (int64_t)(hk * a.G + rr - t * a.G) * a.o_sh);
 }
 __global__ __launch_bounds__(kThreads) void cache_merge_d128_kernel(const CacheArgs a) { cache_merge_body<128>(a); }
 __global__ __launch_bounds__(kThreads) void cache_merge_d64_kernel(const CacheArgs a) { cache_merge_body<64>(a); }
@@ -997,9 +958,8 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
   if (splits > kMaxSplits) splits = kMaxSplits;
   s.splits = (int)splits;
   s.units = s.groups * s.splits;
-  // partial O, then (max, sum) per unit row, then the arrival counters
-  s.workspace_bytes =
-      s.splits > 1 ? (size_t)s.units * kRows * ((size_t)p.head_dim + 2) * sizeof(float) + (size_t)s.groups * 4 : 0;
+  // partial O, then (max, sum) per unit row
+  s.workspace_bytes = s.splits > 1 ? (size_t)s.units * kRows * ((size_t)p.head_dim + 2) * sizeof(float) : 0;
   return s;
 }
 
@@ -1058,11 +1018,8 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
     return hipGetLastError();
   }
   a.part_ml = a.part_o + (size_t)sp.units * kRows * p.head_dim;
-  a.counters = (int*)(a.part_ml + (size_t)sp.units * kRows * 2);
-  a.n_counters = sp.splits > 1 ? (int)sp.groups : 0;
   if (sp.splits > 1 && p.workspace == nullptr) return hipErrorInvalidValue;
   const int64_t appends = (int64_t)a.B * a.S * a.Hkv * (a.D / 8);
-  // units > 0 implies appends > 0, so the counters are always cleared before use
   if (appends > 0) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || sp.units == 0) return e;
@@ -1070,6 +1027,14 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
     hipLaunchKernelGGL(cache_attn_kernel<128>, dim3((unsigned)sp.units), dim3(kThreads), 0, stream, a);
   else
     hipLaunchKernelGGL(cache_attn_kernel<64>, dim3((unsigned)sp.units), dim3(kThreads), 0, stream, a);
+  if (sp.splits > 1) {
+    const int64_t rows = (int64_t)a.S * a.G;
+    const dim3 merge((unsigned)((int64_t)a.B * a.Hkv * ((rows + kWaves - 1) / kWaves)));
+    if (p.head_dim == 128)
+      hipLaunchKernelGGL(cache_merge_splits_d128_kernel, merge, dim3(kThreads), 0, stream, a);
+    else
+      hipLaunchKernelGGL(cache_merge_splits_d64_kernel, merge, dim3(kThreads), 0, stream, a);
+  }
   return hipGetLastError();
 }
 

@@ -99,6 +99,20 @@ def test_prefill_mha_d64(device):
     _run(device, B=2, S=130, hq=4, hkv=4, d=64, L=400, lens=[5, 200], causal=True, seed=2)
 
 
+@pytest.mark.parametrize("S,hq,hkv,d,lens", [
+    (257, 6, 2, 128, [0, 64, 100, 443]),   # 3 heads a group: tokens across row tiles; chunks on and off a tile edge
+    (600, 4, 4, 64, [0, 1, 63, 100]),
+    (512, 16, 16, 64, [188, 0]),
+])
+def test_prefill_reads_the_new_rows_in_place(device, S, hq, hkv, d, lens):
+    """Enough row tiles that the key range is not split: no append launch, the keys of the chunk
+    come from k / v and each workgroup stores its own tokens' rows."""
+    B, L = 24, 700
+    lens = (lens * B)[:B]
+    _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=True, seed=S)
+    _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=False, seed=S + 1)
+
+
 def test_unsplit_launch(device):
     """Enough row tiles that the key range is not split (one workgroup per row tile)."""
     _run(device, B=4, S=1024, hq=16, hkv=4, d=128, L=1100, lens=[0, 3, 40, 76], causal=True, seed=3)
