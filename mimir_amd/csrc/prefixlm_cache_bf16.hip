@@ -11,7 +11,9 @@
 //                            equal share of all key tiles of the call
 //     cache_merge_kernel     adds the partial rows of the shares
 //   otherwise:
-//     cache_append_kernel    the scatter of k_new / v_new into the cache rows
+//     cache_append_kernel    the scatter of k_new / v_new into the cache rows, where
+//                            cache_attn_kernel does not do it (batch rows that may share
+//                            a cache row, or new rows of another token stride)
 //     cache_attn_kernel      one workgroup per (batch row, kv head, 128 query rows,
 //                            key split): the G query heads of a kv head share its
 //                            K / V tiles (rows are (token, head) pairs, token-major),
@@ -49,6 +51,7 @@ struct CacheArgs {
   float* part_o;   // [unit, kRows, D] unnormalized O of each split (splits > 1)
   float* part_ml;  // [unit, kRows, 2]: running max (exp2 domain) and sum
   int shares;      // decode: workgroups the key tiles of the call are dealt to
+  int append;      // prefill: the attention kernel appends the new rows itself
 };
 
 __device__ __forceinline__ int64_t load_index(const void* p, int i, int idx64) {
@@ -215,10 +218,50 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
   const bf16_t* kbase = a.ck + (row_in_cache ? crow : 0) * a.ck_sb + (int64_t)hk * a.ck_sh;
   const bf16_t* vbase = a.cv + (row_in_cache ? crow : 0) * a.cv_sb + (int64_t)hk * a.cv_sh;
   const TileLoader<D, kWaves> ldk(a.ck_st, wave, lane), ldv(a.cv_st, wave, lane);
-  if (kt0 < kt1) {
-    ldk.issue(kbase, kt0 * kKeys, kv, sK0);
-    ldv.issue(vbase, kt0 * kKeys, kv, sV0);
-  }
+  // With `append`, keys [new_lo, new_hi) come from the new rows, which are on their
+  // way into the cache: key j from new row j - pos.  A tile of new rows alone is copied
+  // like one of the cache, from another base; a tile that holds both takes an address
+  // per lane (at most two tiles of a row: with such copies for all tiles of new rows the
+  // launch took longer than the append launch it saves, 8 x 512 on 1536: 78 -> 89 us).
+  // 16 / 4 heads, head_dim 128, against the append launch: 8 x 512 on 1536 keys 81 ->
+  // 78 us, 8 x 100 on 100 to 3000 46 -> 42, 100 on 3000 27 -> 24.5; 8 x 1024 on 1536,
+  // 8 / 8 heads of 64, 68 -> 65.
+  const int64_t pos_raw = load_index(a.cache_lengths, b, a.idx64);
+  const int pos = pos_raw < -(int64_t)a.S ? -a.S : (pos_raw > a.L ? a.L : (int)pos_raw);
+  const int new_lo = a.append ? max(pos, 0) : 0x7fffffff, new_hi = min(pos + a.S, kv);
+  const bf16_t* knb = a.kn + (int64_t)b * a.kn_sb + (int64_t)hk * a.kn_sh;
+  const bf16_t* vnb = a.vn + (int64_t)b * a.vn_sb + (int64_t)hk * a.vn_sh;
+  // Both kinds in one tile: every lane takes its 16 bytes from the row's own place
+  // (keys past the last one repeat it; they are masked).
+  auto issue_mixed = [&](int kb, bf16_t* tk, bf16_t* tv) {
+    using Loader = TileLoader<D, kWaves>;
+#pragma unroll
+    for (int i = 0; i < Loader::kPerWave; ++i) {
+      if (i == Loader::kPerWave - 1 && !ldk.has_last) break;
+      const int u = ldk.lds[i] / 8 + lane;  // 16-byte unit of the tile
+      const int c = min(u % L::kRowUnits, L::kUnits - 1) * 8;
+      const int key = min(kb + L::unperm(u / L::kRowUnits), kv - 1);
+      const bool fresh = key >= new_lo && key < new_hi;
+      const bf16_t* ks = fresh ? knb + (int64_t)(key - pos) * a.kn_st : kbase + (int64_t)key * a.ck_st;
+      const bf16_t* vs = fresh ? vnb + (int64_t)(key - pos) * a.vn_st : vbase + (int64_t)key * a.cv_st;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(ks + c),
+                                       (__attribute__((address_space(3))) void*)(tk + ldk.lds[i]), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vs + c),
+                                       (__attribute__((address_space(3))) void*)(tv + ldk.lds[i]), 16, 0, 0);
+    }
+  };
+  auto issue = [&](int kt, bf16_t* tk, bf16_t* tv) __attribute__((always_inline)) {
+    const int kb = kt * kKeys;
+    const bool some = kb + kKeys > new_lo && kb < new_hi;
+    if (some && (kb < new_lo || new_hi < min(kb + kKeys, kv))) {
+      issue_mixed(kb, tk, tv);
+    } else {
+      const int key0 = some ? kb - pos : kb;
+      ldk.issue_at((some ? knb : kbase) + (int64_t)key0 * a.ck_st, rows_bytes32(kv - kb, (uint32_t)a.ck_st, D), tk);
+      ldv.issue_at((some ? vnb : vbase) + (int64_t)key0 * a.cv_st, rows_bytes32(kv - kb, (uint32_t)a.cv_st, D), tv);
+    }
+  };
+  if (kt0 < kt1) issue(kt0, sK0, sV0);
 
   // Q^T B-operand fragments: lane holds row `row`, d = 16*ks + 8*hi .. +7 (0 for rows >= R).
   bf16x8 qf[KS];
@@ -306,21 +349,30 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
       }
   };
 
+  // The new tokens whose first row lies in this row tile go into the cache here (no
+  // workgroup reads these cache rows).
+  if (a.append && split == 0 && row_in_cache) {
+    constexpr int kUnits = D / 8;
+    const int first = max((rt * kRows + a.G - 1) / a.G, -pos);
+    const int last = min(((rt + 1) * kRows + a.G - 1) / a.G, min(a.S, a.L - pos));
+    for (int t = first + tid / kUnits; t < last; t += kThreads / kUnits) {
+      const int c = tid % kUnits * 8;
+      *(bf16x8*)&a.ck[crow * a.ck_sb + (int64_t)(pos + t) * a.ck_st + (int64_t)hk * a.ck_sh + c] =
+          *(const bf16x8*)&knb[(int64_t)t * a.kn_st + c];
+      *(bf16x8*)&a.cv[crow * a.cv_sb + (int64_t)(pos + t) * a.cv_st + (int64_t)hk * a.cv_sh + c] =
+          *(const bf16x8*)&vnb[(int64_t)t * a.vn_st + c];
+    }
+  }
+
   for (int kt = kt0; kt < kt1; kt += 2) {
     wait_vmem();
     __syncthreads();
-    if (kt + 1 < kt1) {
-      ldk.issue(kbase, (kt + 1) * kKeys, kv, sK1);
-      ldv.issue(vbase, (kt + 1) * kKeys, kv, sV1);
-    }
+    if (kt + 1 < kt1) issue(kt + 1, sK1, sV1);
     compute(kt, sK0, sV0);
     if (kt + 1 >= kt1) break;
     wait_vmem();
     __syncthreads();
-    if (kt + 2 < kt1) {
-      ldk.issue(kbase, (kt + 2) * kKeys, kv, sK0);
-      ldv.issue(vbase, (kt + 2) * kKeys, kv, sV0);
-    }
+    if (kt + 2 < kt1) issue(kt + 2, sK0, sV0);
     compute(kt + 1, sK1, sV1);
   }
 
@@ -965,7 +1017,7 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
 
 hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t stream) {
   const CacheSplit sp = cache_split(p);
-  CacheArgs a;
+  CacheArgs a = {};
   a.q = (const bf16_t*)p.q;
   a.kn = (const bf16_t*)p.k_new;
   a.vn = (const bf16_t*)p.v_new;
@@ -1019,8 +1071,10 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   }
   a.part_ml = a.part_o + (size_t)sp.units * kRows * p.head_dim;
   if (sp.splits > 1 && p.workspace == nullptr) return hipErrorInvalidValue;
+  // every batch row has a cache row of its own, and one set of copy offsets serves both
+  a.append = a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st;
   const int64_t appends = (int64_t)a.B * a.S * a.Hkv * (a.D / 8);
-  if (appends > 0) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);
+  if (appends > 0 && !a.append) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || sp.units == 0) return e;
   if (p.head_dim == 128)

@@ -113,6 +113,43 @@ def test_prefill_reads_the_new_rows_in_place(device, S, hq, hkv, d, lens):
     _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=False, seed=S + 1)
 
 
+@pytest.mark.parametrize("S,hq,hkv,d,lens", [
+    (33, 4, 4, 128, [0, 31, 1000]),      # one row tile per head, the chunk inside the last key split
+    (129, 8, 2, 128, [63, 64, 1367]),    # 516 rows: five row tiles, the last of four rows
+    (200, 2, 2, 64, [1296, 5, 127]),     # up to the end of the cache
+])
+def test_prefill_reads_the_new_rows_in_place_split_keys(device, S, hq, hkv, d, lens):
+    """The same with the key range split: the chunk's keys lie in one or several splits."""
+    for causal in (True, False):
+        _run(device, B=3, S=S, hq=hq, hkv=hkv, d=d, L=1496, lens=lens, causal=causal, seed=S)
+
+
+@pytest.mark.parametrize("S", [1, 40])
+def test_lengths_outside_the_cache(device, S):
+    """Without validation, new rows at positions outside the cache are dropped, and the row attends
+    the min(max(length, 0) + S, cache_len) first keys."""
+    gen = torch.Generator().manual_seed(S)
+    L, d, lens = 100, 64, [-1, -30, 90, 100, 150]
+    B = len(lens)
+    q, k, v = (torch.randn(B, S, 2, d, generator=gen).to(BF16) for _ in range(3))
+    ck, cv = (torch.randn(B, L, 2, d, generator=gen).to(BF16) for _ in range(2))
+    cache = Cache(ck.to(device), cv.to(device))
+    out = attention_with_cache(q.to(device), k.to(device), v.to(device), cache, torch.tensor(lens, device=device), True)
+    torch.cuda.synchronize()
+    for b, n in enumerate(lens):
+        for i in range(S):
+            if 0 <= n + i < L:
+                ck[b, n + i], cv[b, n + i] = k[b, i], v[b, i]
+        start = min(max(n, 0), L)
+        keys = min(start + S, L)
+        for i in range(S):
+            end = min(start + i + 1, keys)
+            p = torch.softmax(torch.einsum("hd,khd->hk", q[b, i].float(), ck[b, :end].float()) / d ** 0.5, dim=1)
+            ref = torch.einsum("hk,khd->hd", p, cv[b, :end].float())
+            assert (out[b, i].float().cpu() - ref).abs().max().item() <= 2e-2, (b, i)
+    assert torch.equal(cache.keys.cpu(), ck) and torch.equal(cache.values.cpu(), cv)
+
+
 def test_unsplit_launch(device):
     """Enough row tiles that the key range is not split (one workgroup per row tile)."""
     _run(device, B=4, S=1024, hq=16, hkv=4, d=128, L=1100, lens=[0, 3, 40, 76], causal=True, seed=3)
