@@ -994,10 +994,14 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
     if (s.pairs) {  // one workgroup per pair
       s.units = s.groups;
     } else {
-      // two shares of the line per CU, or one per unit if there cannot be as many;
-      // two part slots per share: partial O, then (max, sum) rows
-      const int64_t most = s.groups * ((tiles + kShareUnit - 1) / kShareUnit), two = 2 * (int64_t)device_cu_count();
-      s.units = most < two ? most : two;
+      // Two shares of the line per CU (head_dim 64: three, which its LDS allows and its
+      // copies of half the bytes need), or one per unit if there cannot be as many; two part
+      // slots per share: partial O, then (max, sum) rows.  Three against two, 8 / 8 heads of
+      // 64: 32 rows of 100 to 3200 keys 32.5 -> 27.8 us, 8 of 1000 to 3100 15.1 -> 13.3, 64 of
+      // 0 to 3780 57.0 -> 54.1; 64 of 512 to 7440 106 -> 111, 8 / 2 heads 29.6 -> 30.8.
+      const int64_t most = s.groups * ((tiles + kShareUnit - 1) / kShareUnit),
+                    shares = (p.head_dim == 64 ? 3 : 2) * (int64_t)device_cu_count();
+      s.units = most < shares ? most : shares;
       s.workspace_bytes = (size_t)s.units * 2 * (size_t)R * ((size_t)p.head_dim + 2) * sizeof(float);
     }
     s.splits = 1;
