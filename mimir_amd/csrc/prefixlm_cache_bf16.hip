@@ -51,6 +51,7 @@ struct CacheArgs {
   float* part_o;   // [unit, kRows, D] unnormalized O of each split (splits > 1)
   float* part_ml;  // [unit, kRows, 2]: running max (exp2 domain) and sum
   int shares;      // decode: workgroups the key tiles of the call are dealt to
+  int cus;         // CUs of the device
   int append;      // prefill: the attention kernel appends the new rows itself
 };
 
@@ -179,8 +180,15 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
   int u = blockIdx.x;
   const int split = u % a.splits;
   u /= a.splits;
-  const int rt = u % a.n_rt;
+  int rt = u % a.n_rt;
   u /= a.n_rt;
+  // Later row tiles of a causal chunk see more keys.  Workgroups b and b + (CUs) share a
+  // CU, and with the row tiles in the same order in every pair they were the same row
+  // tile of two pairs (n_rt a power of two): some CUs got two long ones.  Every other
+  // CU-sized run of pairs takes its row tiles in reverse: 8 x 512 on 1536 keys 76.8 ->
+  // 74.4 us, 8 x 512 on none 28.6 -> 25.2, 8 x 1024 on none 74.3 -> 68.0 (16 / 4 heads,
+  // head_dim 128), 8 x 1024 on 1536 64 -> 59 (8 / 8 heads of 64); split ranges unchanged.
+  if (u * a.n_rt * a.splits / a.cus % 2 == 1) rt = a.n_rt - 1 - rt;
   const int hk = u % a.Hkv;
   const int b = u / a.Hkv;
 
@@ -396,7 +404,7 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
   // Several splits hold keys of this row tile: this split's partial rows --
   // unnormalized O, the max in the exp2 domain (-inf: no allowed key) and the sum.
   if (!wave_active) return;
-  const int64_t slot = (int64_t)blockIdx.x * kRows + wave * 32 + l32;
+  const int64_t slot = (((int64_t)u * a.n_rt + rt) * a.splits + split) * kRows + wave * 32 + l32;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -1076,6 +1084,7 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   a.part_ml = a.part_o + (size_t)sp.units * kRows * p.head_dim;
   if (sp.splits > 1 && p.workspace == nullptr) return hipErrorInvalidValue;
   // every batch row has a cache row of its own, and one set of copy offsets serves both
+  a.cus = device_cu_count();
   a.append = a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st;
   const int64_t appends = (int64_t)a.B * a.S * a.Hkv * (a.D / 8);
   if (appends > 0 && !a.append) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);
