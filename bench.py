@@ -404,7 +404,7 @@ def cache_bench(torch, dev, args) -> int:
             entry["graph_gbs"] = round((cache_bytes + io_bytes) / (gms * 1e-3) / 1e9, 1)
         res[name] = entry
     res["value"] = res["decode"]["gbs"]
-    res["roofline"] = {"kernel": "cache_append_kernel + cache_attn_kernel<128> (decode step)", "bound": "hbm",
+    res["roofline"] = {"kernel": "cache_decode_d128_kernel + cache_merge_d128_kernel (decode step)", "bound": "hbm",
                        "achieved": res["decode"]["gbs"], "peak": HBM_GBS, "unit": "GB/s",
                        "frac": res["decode"]["hbm_frac"]}
     print(json.dumps(res), flush=True)
