@@ -474,7 +474,7 @@ __global__ __launch_bounds__(kThreads) void cache_merge_splits_d64_kernel(const 
 // Measured against an append kernel, one workgroup of four waves per (pair, equal
 // split) and a counted merge in it (Hq 16, Hkv 4, D 128): 64 rows of 512 to 8000 keys
 // 138 -> 119 us (5.0 TB/s), 32 rows of 100 to 4000 41 -> 33, one row of 8000 24 -> 15;
-// 8 rows of 1000 to 3600 18.2 -> 17.7, of which the two launches and their chains of
+// 8 rows of 1000 to 3600 18.2 -> 17.9, of which the two launches and their chains of
 // round trips (lengths, tiles, parts) are 9.
 // ---------------------------------------------------------------------------
 constexpr int kDecKeys = 32;  // keys per wave tile
