@@ -6,14 +6,13 @@
 // (and j <= cache_lengths[b] + i when causal).  The reference materializes the
 // repeated K/V heads and a [B, S, max_kv_len] mask for SDPA; here:
 //
+//   cache_append_kernel      the scatter of k_new / v_new into the cache rows, first,
+//                            where the attention kernels do not do it themselves
 //   decode (at most 32 query rows per kv head, e.g. S = 1):
 //     cache_decode_*_kernel  appends the new rows and attends, each workgroup an
 //                            equal share of all key tiles of the call
 //     cache_merge_kernel     adds the partial rows of the shares
 //   otherwise:
-//     cache_append_kernel    the scatter of k_new / v_new into the cache rows, where
-//                            cache_attn_kernel does not do it (batch rows that may share
-//                            a cache row, or new rows of another token stride)
 //     cache_attn_kernel      one workgroup per (batch row, kv head, 128 query rows,
 //                            key split): the G query heads of a kv head share its
 //                            K / V tiles (rows are (token, head) pairs, token-major),
@@ -21,6 +20,7 @@
 //                            and O^T += V^T P^T on bf16 MFMA with an online softmax
 //                            (the forward kernel's arithmetic)
 //     cache_merge_splits_*   with several splits: adds their partial rows
+#include "prefixlm_cache_layout.h"
 #include "prefixlm_common.h"
 
 namespace mimir {
@@ -52,7 +52,7 @@ struct CacheArgs {
   float* part_ml;  // [unit, kRows, 2]: running max (exp2 domain) and sum
   int shares;      // decode: workgroups the key tiles of the call are dealt to
   int cus;         // CUs of the device
-  int append;      // prefill: the attention kernel appends the new rows itself
+  int append;      // the attention kernel appends the new rows itself
 };
 
 __device__ __forceinline__ int64_t load_index(const void* p, int i, int idx64) {
@@ -754,6 +754,8 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
     for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const bf16x8*)&qrow[16 * ks];
     if (n_my > 0) issue(t0 + wave, mk0, mv0);
     if (n_my > 1) issue(t0 + wave + kDecWaves, mk1, mv1);
+    new_lo = new_hi = 0;  // appended by a launch of its own: the copies hold them
+    if (!a.append) return;
     new_lo = pos_b;
     new_hi = pos_b + a.S;
     for_others([&](int, int p) {
@@ -1061,9 +1063,20 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   a.splits = sp.splits;
   a.scale_log2 = p.softmax_scale * kLog2e;
   a.part_o = (float*)p.workspace;
+  // Where the attention kernels append the new rows themselves, no workgroup reads them
+  // from the cache, which asks for cache rows that share no memory: a batch row's new
+  // rows are then seen through its own cache row alone.  (Shared, e.g. a cache expanded
+  // over the batch, every batch row sees all new rows, as after appending all of them.)
+  // Decode finds the batch rows on one cache row by their indices; prefill does not, and
+  // needs one set of copy offsets for the new rows and the cache.
+  a.append = cache_rows_distinct(p) &&
+             (sp.decode || (a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st));
+  const int64_t appends = (int64_t)a.B * a.S * a.Hkv * (a.D / 8);
+  if ((sp.decode ? !sp.pairs : sp.splits > 1) && p.workspace == nullptr) return hipErrorInvalidValue;
+  if (appends > 0 && !a.append) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || sp.units == 0) return e;
   if (sp.decode) {
-    if (sp.units == 0) return hipSuccess;
-    if (!sp.pairs && p.workspace == nullptr) return hipErrorInvalidValue;
     const int64_t rows = (int64_t)a.S * a.G;
     a.shares = (int)sp.units;
     a.part_ml = a.part_o + (size_t)sp.units * 2 * rows * p.head_dim;
@@ -1086,14 +1099,7 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
     return hipGetLastError();
   }
   a.part_ml = a.part_o + (size_t)sp.units * kRows * p.head_dim;
-  if (sp.splits > 1 && p.workspace == nullptr) return hipErrorInvalidValue;
-  // every batch row has a cache row of its own, and one set of copy offsets serves both
   a.cus = device_cu_count();
-  a.append = a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st;
-  const int64_t appends = (int64_t)a.B * a.S * a.Hkv * (a.D / 8);
-  if (appends > 0 && !a.append) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || sp.units == 0) return e;
   if (p.head_dim == 128)
     hipLaunchKernelGGL(cache_attn_kernel<128>, dim3((unsigned)sp.units), dim3(kThreads), 0, stream, a);
   else

@@ -84,6 +84,49 @@ def test_decode_rows_sharing_a_cache_row(device):
          seed=32)  # one workgroup per pair
 
 
+@pytest.mark.parametrize("d,S,lens", [
+    (128, 1, [10, 63, 64, 40]),       # one workgroup per pair
+    (128, 2, [700, 2, 704, 702]),     # equal shares
+    (64, 8, [100, 92, 1990, 84]),
+    (128, 40, [0, 120, 40, 80]),      # prefill, one key split
+    (64, 100, [1500, 1300, 1400, 0]), # and several
+])
+@pytest.mark.parametrize("form", ["expanded", "windows", "one tensor"])
+def test_cache_rows_that_share_memory(device, d, S, lens, form):
+    """Every batch row sees all new rows that lie among its keys, as after appending all of them
+    first: batch rows on the same positions, overlapping windows, one tensor for keys and values."""
+    gen = torch.Generator().manual_seed(d + S)
+    B, L, hq, hkv = len(lens), max(lens) + S + 5, 4, 2
+    q = torch.randn(B, S, hq, d, generator=gen).to(BF16)
+    k, v = (torch.randn(B, S, hkv, d, generator=gen).to(BF16) for _ in range(2))
+    step = {"expanded": 0, "windows": 3, "one tensor": 2 * L}[form]  # positions from one row to the next
+    flat = torch.randn(2, L + (B - 1) * step, hkv, d, generator=gen).to(BF16)
+
+    def view(x):  # [B, L, hkv, d], batch row b at position b * step
+        return x.as_strided((B, L, hkv, d), (step * hkv * d, hkv * d, d, 1), x.storage_offset())
+
+    if form == "windows":  # new rows at positions of their own
+        lens = [n - 3 * b if n >= 3 * b else n for b, n in enumerate(lens)]
+        spans = sorted((n + b * step, n + b * step + S) for b, n in enumerate(lens))
+        assert all(e <= s for (_, e), (s, _) in zip(spans, spans[1:])), spans
+    kf, vf = (flat[0].clone(), flat[0 if form == "one tensor" else 1].clone())
+    if form == "one tensor":
+        vf = kf
+    for b, n in enumerate(lens):
+        kf[b * step + n:b * step + n + S] = k[b]
+        vf[b * step + n:b * step + n + S] = v[b]
+    dev = flat.to(device)
+    cache = Cache(view(dev[0]), view(dev[0 if form == "one tensor" else 1]))
+    out = attention_with_cache(q.to(device), k.to(device), v.to(device), cache, torch.tensor(lens, device=device), True)
+    torch.cuda.synchronize()
+    for b, n in enumerate(lens):
+        for i in range(S):
+            ks, vs = (x[b * step:b * step + n + i + 1].float().repeat_interleave(hq // hkv, 1) for x in (kf, vf))
+            p = torch.softmax(torch.einsum("hd,khd->hk", q[b, i].float(), ks) / d ** 0.5, dim=1)
+            assert (out[b, i].float().cpu() - torch.einsum("hk,khd->hd", p, vs)).abs().max().item() <= 2e-2, (b, i)
+    assert torch.equal(dev[0].cpu(), kf) and torch.equal(dev[0 if form == "one tensor" else 1].cpu(), vf)
+
+
 def test_decode_uneven_rows(device):
     """Rows whose key ranges split into different numbers of parts (1 key to the whole cache)."""
     _run(device, B=8, S=1, hq=16, hkv=4, d=128, L=4096, lens=[0, 63, 64, 65, 1000, 4095, 2048, 129],
