@@ -11,8 +11,10 @@
 //
 // Every function here serves only well-formed calls: anything else (another device
 // or dtype, a layout the kernels cannot read in place, metadata to convert, a failed
-// allocation or launch) returns None, and the caller takes the general path in
-// Python, which converts, falls back or raises.
+// allocation, arguments that the C ABI refuses) returns None, and the caller takes the
+// general path in Python, which converts, falls back or raises.  An error of the launch
+// itself raises here: kernels of the call may have run, and the general path would run
+// them again (an in-place RoPE twice).
 #include <Python.h>
 #include <dlfcn.h>
 
@@ -35,9 +37,12 @@ struct Library {
   decltype(&mimir_prefixlm_rope) rope = nullptr;
   decltype(&mimir_prefixlm_cache_attn) cache_attn = nullptr;
   decltype(&mimir_prefixlm_cache_attn_workspace_bytes) cache_workspace = nullptr;
+  decltype(&mimir_prefixlm_last_error) last_error = nullptr;
+  c10::DeviceType device = c10::DeviceType::CUDA;  // of the tensors it takes
 } lib;
 
 struct Fallback {};  // thrown where the general path takes over
+struct Raised {};    // thrown with the Python error set
 void need(bool ok) {
   if (!ok) throw Fallback();
 }
@@ -46,6 +51,7 @@ const at::Tensor& tensor(PyObject* o) {
   need(THPVariable_CheckExact(o));
   return THPVariable_Unpack(o);
 }
+bool on_device(const at::Tensor& t) { return t.device().type() == lib.device; }
 bool is_none(PyObject* o) { return o == Py_None; }
 int32_t int32(PyObject* o) {  // an int, or a one-element int64 CPU tensor (the reference's scalars)
   int64_t x;
@@ -106,7 +112,11 @@ void launch(int (*entry)(const P*, void*), const P& p, void* s) {
   Py_BEGIN_ALLOW_THREADS;
   status = entry(&p, s);
   Py_END_ALLOW_THREADS;
-  need(status == MIMIR_OK);
+  if (status == MIMIR_ERR_HIP) {
+    PyErr_SetString(PyExc_RuntimeError, lib.last_error());
+    throw Raised();
+  }
+  need(status == MIMIR_OK);  // else refused, nothing launched
 }
 
 // The checks and fields the forward and the backward share.
@@ -115,7 +125,7 @@ struct Geometry {
   int dtype;
 };
 Geometry geometry(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
-  need(q.is_cuda() && q.dim() == 3 && k.dim() == 3 && v.dim() == 3);
+  need(on_device(q) && q.dim() == 3 && k.dim() == 3 && v.dim() == 3);
   const Geometry g{q.size(0), q.size(1), k.size(1), q.size(2),
                    q.scalar_type() == at::kBFloat16 ? MIMIR_DTYPE_BFLOAT16 : MIMIR_DTYPE_FLOAT32};
   need(q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kFloat);
@@ -145,6 +155,8 @@ PyObject* guarded(Py_ssize_t given, Py_ssize_t wanted, F&& body) {
   }
   try {
     if (PyObject* out = body()) return out;
+  } catch (const Raised&) {
+    return nullptr;
   } catch (const Fallback&) {
   } catch (const std::exception&) {  // e.g. out of memory: the general path raises it
   }
@@ -278,7 +290,7 @@ PyObject* py_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 6, [&]() -> PyObject* {
     const at::Tensor &x = tensor(a[0]), &cos = tensor(a[1]), &sin = tensor(a[2]);
-    need(x.is_cuda() && x.dim() == 3 && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat));
+    need(on_device(x) && x.dim() == 3 && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat));
     in_place(x, x);
     const int64_t T = x.size(0), d = x.size(2);
     need(T <= 0x7fffffff && x.size(1) > 0);
@@ -314,7 +326,7 @@ PyObject* py_cache_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded(n, 11, [&]() -> PyObject* {
     const at::Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]), &ck = tensor(a[3]), &cv = tensor(a[4]);
     const at::Tensor& lens = tensor(a[5]);
-    need(q.is_cuda() && q.scalar_type() == at::kBFloat16 && q.dim() == 4 && k.dim() == 4 && v.dim() == 4 &&
+    need(on_device(q) && q.scalar_type() == at::kBFloat16 && q.dim() == 4 && k.dim() == 4 && v.dim() == 4 &&
          ck.dim() == 4 && cv.dim() == 4);
     const int64_t B = q.size(0), S = q.size(1), hq = q.size(2), d = q.size(3), hkv = k.size(2), L = ck.size(1);
     need(B > 0 && S > 0 && hq > 0 && hkv > 0 && hq % hkv == 0 && L > 0 && B <= 0x7fffffff && S <= 0x7fffffff &&
@@ -353,10 +365,16 @@ PyObject* py_cache_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// bind(path): the entry points of the (already loaded) C-ABI library.
-PyObject* py_bind(PyObject*, PyObject* path) {
-  const char* file = PyUnicode_AsUTF8(path);
-  if (file == nullptr) return nullptr;
+// bind(path, device="cuda"): the entry points of the (already loaded) C-ABI library, and
+// the type of device whose tensors it takes.
+PyObject* py_bind(PyObject*, PyObject* args) {
+  const char *file, *device = "cuda";
+  if (!PyArg_ParseTuple(args, "s|s", &file, &device)) return nullptr;
+  try {
+    lib.device = c10::Device(device).type();
+  } catch (const std::exception&) {
+    return PyErr_Format(PyExc_ValueError, "device %s", device);
+  }
   void* h = dlopen(file, RTLD_NOW | RTLD_LOCAL);
   if (h == nullptr) return PyErr_Format(PyExc_ImportError, "%s", dlerror());
   bool ok = true;
@@ -373,12 +391,13 @@ PyObject* py_bind(PyObject*, PyObject* path) {
   get(lib.rope, "mimir_prefixlm_rope");
   get(lib.cache_attn, "mimir_prefixlm_cache_attn");
   get(lib.cache_workspace, "mimir_prefixlm_cache_attn_workspace_bytes");
+  get(lib.last_error, "mimir_prefixlm_last_error");
   if (!ok) return PyErr_Format(PyExc_ImportError, "%s lacks an entry point", file);
   Py_RETURN_NONE;
 }
 
 PyMethodDef methods[] = {
-    {"bind", py_bind, METH_O, nullptr},
+    {"bind", py_bind, METH_VARARGS, nullptr},
     {"fwd", (PyCFunction)(void*)py_fwd, METH_FASTCALL, nullptr},
     {"bwd", (PyCFunction)(void*)py_bwd, METH_FASTCALL, nullptr},
     {"rope", (PyCFunction)(void*)py_rope, METH_FASTCALL, nullptr},
