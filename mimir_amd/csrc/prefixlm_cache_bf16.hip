@@ -479,6 +479,7 @@ __global__ __launch_bounds__(kThreads) void cache_merge_splits_d64_kernel(const 
 // ---------------------------------------------------------------------------
 constexpr int kDecKeys = 32;  // keys per wave tile
 constexpr int kDecRows = 32;  // query rows of the decode kernel (one wave's columns)
+constexpr float kRefRange = 30.f;  // how far (log2) a tile's reference may lie below the row's maximum
 // Shares of the line: two waves and two workgroups per CU, whose starts and ends
 // overlap; a unit of the line is both stages of every wave.
 constexpr int kShareWaves = 2;
@@ -765,7 +766,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   };
 
   f32x16 oacc[DT];
-  float m_run, l_run;
+  float m_run, m_top, l_run;  // the sums' reference and the row's maximum so far (scores), the sum
   auto compute = [&](int t, const bf16_t* sK, const bf16_t* sV) {
     const int kb = t * kDecKeys;
     f32x16 st = f32x16{};
@@ -783,21 +784,21 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[r]);
     mx = xor32_max(mx);
-    // Rescaled whenever the maximum grows, not lazily as in the forward kernel: under a
-    // fresh maximum the largest probability is 1 and its bf16 rounding exact, which a
-    // wave's few tiles show.  Error against 64 bits, lazily and so: 8 rows of 1000 to
-    // 3600 keys 2.3e-3 / 2.10e-3, 64 of 500 to 8000 2.3e-3 / 2.19e-3, one of 700 2.2e-3 /
-    // 2.05e-3; time 17.5 / 17.9 us, 118.8 / 119.4, 10.8 / 11.0.
-    const float m_cand = fmaxf(m_run, mx);
-    const bool grow = m_cand > m_run;
-    if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-      const float m_new = grow ? m_cand : m_run;
-      const float alpha = m_new == -INFINITY ? 1.f : fast_exp2((m_run - m_new) * c2);
-      l_run *= alpha;
+    // Every tile's probabilities are taken under the tile's own maximum (but not more than
+    // 2^30 below the row's so far, which bounds the sums): its largest probability is then 1
+    // and exact in bf16.  Rescaled only when the row's maximum grew, what P's rounding cost
+    // a tile depended on the tiles before it in its share, and so on the split: finer equal
+    // splits, one tile per wave for a few rows, were more exact there.  Error against 64
+    // bits, under the growing maximum / so: one row of 700 keys 2.07e-3 / 2.03e-3, 8 rows of
+    // 1000 to 3600 2.09e-3 / 2.02e-3, 64 of 100 to 3000 2.12e-3 / 2.02e-3; time 11.9 / 11.5
+    // us, 17.1 / 16.7, and 64 rows of 500 to 8000 120.3 / 119.8.
+    m_top = fmaxf(m_top, mx);
+    const float m_new = fmaxf(mx, m_top - kRefRange / c2);
+    const float alpha = m_run == -INFINITY ? 1.f : fast_exp2((m_run - m_new) * c2);
+    l_run *= alpha;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
-      m_run = m_new;
-    }
+    for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
+    m_run = m_new;
     const float mb = m_run == -INFINITY ? 0.f : m_run * c2;
     float lsum = 0.f;
 #pragma unroll
@@ -828,7 +829,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   for (;;) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x16{};
-    m_run = -INFINITY;
+    m_run = m_top = -INFINITY;
     l_run = 0.f;
     // Each wave waits only for its own copies: tile i has landed once at most the
     // copies of tile i + 1 are outstanding.

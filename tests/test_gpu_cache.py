@@ -75,6 +75,42 @@ def test_decode_work_split(device, B, S, hq, hkv, d, L, seed):
          rows=torch.randperm(B, generator=gen).tolist(), seed=seed)
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(16, 4, 128), (8, 8, 64)])
+def test_decode_does_not_depend_on_the_split(device, hq, hkv, d):
+    """One row alone (a tile or two per wave) and the same row 64 times over (whole pairs per
+    workgroup, or shares of many tiles per wave) round P alike, so they differ by fp32 sums
+    alone: 1e-6, which moves about one bf16 result in a thousand by 2^-8 of itself (1e-4 in
+    all).  Under maxima that depend on the split, P rounds elsewhere: 1e-3 and more."""
+    gen = torch.Generator(device=device).manual_seed(3)
+    mk = lambda *s: torch.randn(*s, generator=gen, device=device).to(BF16)
+    for L, n in ((1024, 700), (4096, 2500)):
+        q, k, v = mk(1, 1, hq, d), mk(1, 1, hkv, d), mk(1, 1, hkv, d)
+        keys, values = mk(1, L, hkv, d), mk(1, L, hkv, d)
+        one = attention_with_cache(q, k, v, Cache(keys.clone(), values.clone()), torch.tensor([n], device=device), True)
+        many = [t.repeat(64, 1, 1, 1) for t in (q, k, v, keys, values)]
+        out = attention_with_cache(*many[:3], Cache(*many[3:]), torch.tensor([n] * 64, device=device), True)
+        err = (out.float() - one.float()).norm() / (one.float().norm() * 8)
+        print(f"[split] hq={hq} d={d} L={L} n={n} err={err:.3g}", flush=True)
+        assert err <= 4e-4
+
+
+def test_decode_reference_of_a_low_tile(device):
+    """Key tiles whose scores lie far below (and far above) those of the tiles before them."""
+    B, L, d = 2, 512, 128
+    gen = torch.Generator().manual_seed(4)
+    q = torch.randn(B, 1, 2, d, generator=gen)
+    scale = torch.tensor([40.0, 1e-3, 40.0, 0.1] * 4).repeat_interleave(L // 16)[None, :, None, None]
+    keys = (q.mean(2, keepdim=True) * scale + torch.randn(B, L, 2, d, generator=gen) * 1e-2).to(BF16)
+    values = torch.randn(B, L, 2, d, generator=gen).to(BF16)
+    q, k, v = q.to(BF16), keys[:, :1].clone(), values[:, :1].clone()
+    lens = torch.tensor([L - 1, 100])
+    ref = LO.attention_with_cache(q, k, v, keys.clone(), values.clone(), lens, True)
+    out = attention_with_cache(q.to(device), k.to(device), v.to(device), Cache(keys.to(device), values.to(device)),
+                               lens.to(device), True)
+    torch.cuda.synchronize()
+    assert (out.float().cpu() - ref.float()).abs().max().item() <= 2e-2
+
+
 def test_decode_rows_sharing_a_cache_row(device):
     """Batch rows on one cache row attend each other's new keys, as after appending all of them
     first: consecutive tokens of a sequence fed as separate batch rows, and one far behind."""
