@@ -587,11 +587,16 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   __shared__ __attribute__((aligned(16))) bf16_t sV0[kDecWaves * T::kElems];
   __shared__ __attribute__((aligned(16))) bf16_t sK1[kDecWaves * T::kElems];
   __shared__ __attribute__((aligned(16))) bf16_t sV1[kDecWaves * T::kElems];
-  __shared__ __attribute__((aligned(16))) float sMl[kDecWaves][kDecRows][2];  // per wave and row: max (exp2), sum
-  // the waves' partial O, kMergeRows rows at a time (two workgroups share the
-  // CU's 160 KiB); a padded row keeps the rows in distinct banks
-  constexpr int kMergeRows = D == 128 ? 4 : 8;
-  __shared__ __attribute__((aligned(16))) float sO[kDecWaves][kMergeRows][D + 4];
+  // The merge's area per wave, in the second stages, which are free between a segment's
+  // last tile and the second of the next: partial O [kDecRows][kPitch] (the padding keeps
+  // the rows in distinct banks), then per row the reference (exp2 domain) and the sum.
+  // (In an area of its own, four rows at a time, since two workgroups share the CU's LDS,
+  // a segment of 32 query rows took eight passes between barriers: 64 rows of 100 to 3900
+  // keys, 32 query rows a head, 87.5 -> 68.1 us, 32 of 100 to 3000, 8 / 8 heads of 64, 41.6 -> 33.6; 8
+  // rows of 500 to 3000 24.2 -> 18.5, with 4 query rows a head 16.7 -> 15.9.)
+  constexpr int kPitch = D + 4;
+  constexpr int kArea = kDecRows * (kPitch + 2);
+  static_assert(kArea * 4 <= 2 * T::kElems * 2, "two waves' K (or V) stages hold a wave's area");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -724,7 +729,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
                                                voffv[i], 0, 0, 0);
   };
   // Makes the segment at u0 (lane j of the line) the current one: its Q rows and
-  // this wave's first two tiles are requested.
+  // this wave's first tile are requested; its second tile's stages may still be in use.
   auto begin = [&]() __attribute__((always_inline)) {
     const CacheArgs& c = cold_args();
     b = line.first + j;
@@ -754,7 +759,6 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const bf16x8*)&qrow[16 * ks];
     if (n_my > 0) issue(t0 + wave, mk0, mv0);
-    if (n_my > 1) issue(t0 + wave + kDecWaves, mk1, mv1);
     new_lo = new_hi = 0;  // appended by a launch of its own: the copies hold them
     if (!a.append) return;
     new_lo = pos_b;
@@ -826,6 +830,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   };
 
   begin();
+  if (n_my > 1) issue(t0 + wave + kDecWaves, mk1, mv1);
   for (;;) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x16{};
@@ -857,9 +862,9 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
       }
     }
 
-    // The next segment's copies go out before this one's merge (this wave's reads
-    // of its stages are done; the merge has LDS of its own), so that a share of
-    // several short segments does not pay a memory round trip for each.
+    // The next segment's first copies go out before this one's merge (this wave's
+    // reads of its stages are done; the merge uses the second ones), so that a share
+    // of several short segments does not pay a memory round trip for each.
     const int cur_b = b, cur_hk = hk;
     const bool cur_whole = whole;
     const int64_t slot = (int64_t)part_slot(u0, per) * R;
@@ -873,61 +878,61 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
       }
       begin();
     }
-    // Merge the waves' partial rows through LDS, kMergeRows at a time.
+    // Merge the waves' partial rows through LDS.
     const float l_tot = xor32_sum(l_run);
-    if (hi == 0) {
-      sMl[wave][l32][0] = m_run == -INFINITY ? -INFINITY : m_run * c2;
-      sMl[wave][l32][1] = l_tot;
-    }
-    constexpr int cpl = D / 64;
-    for (int r0 = 0; r0 < R; r0 += kMergeRows) {
-      if (l32 >= r0 && l32 < r0 + kMergeRows) {
-        float* po = sO[wave][l32 - r0];
+    auto area = [&](int w) __attribute__((always_inline)) {  // of wave w
+      return (float*)(w < kDecWaves / 2 ? sK1 : sV1) + w % (kDecWaves / 2) * kArea;
+    };
+    auto row_ml = [&](int w, int row) __attribute__((always_inline)) {
+      return (f32x2*)(area(w) + kDecRows * kPitch) + row;
+    };
+    lds_barrier();  // every wave is done with its second stage
+    if (l32 < R) {
+      if (hi == 0) *row_ml(wave, l32) = f32x2{m_run == -INFINITY ? -INFINITY : m_run * c2, l_tot};
+      float* po = area(wave) + l32 * kPitch;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
-            f32x4 tv;
+        for (int rg = 0; rg < 4; ++rg) {
+          f32x4 tv;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) tv[e] = oacc[dt][4 * rg + e];
-            *(f32x4*)&po[32 * dt + 8 * rg + 4 * hi] = tv;
-          }
-      }
-      lds_barrier();
-      for (int rr = r0 + wave; rr < min(R, r0 + kMergeRows); rr += kDecWaves) {  // D / 64 columns per lane
-        float M = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < kDecWaves; ++w) M = fmaxf(M, sMl[w][rr][0]);
-        float lsum = 0.f;
-        float acc[cpl] = {};
-        if (M != -INFINITY) {
-#pragma unroll
-          for (int w = 0; w < kDecWaves; ++w) {
-            const float m = sMl[w][rr][0];
-            const float wt = m == -INFINITY ? 0.f : fast_exp2(m - M);
-            lsum += sMl[w][rr][1] * wt;
-#pragma unroll
-            for (int e = 0; e < cpl; ++e) acc[e] += sO[w][rr - r0][lane * cpl + e] * wt;
-          }
+          for (int e = 0; e < 4; ++e) tv[e] = oacc[dt][4 * rg + e];
+          *(f32x4*)&po[32 * dt + 8 * rg + 4 * hi] = tv;
         }
-        const CacheArgs& c = cold_args();
-        if (cur_whole) {
-          const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-          const int ti_r = rr / a.G;
-          const int h_r = cur_hk * a.G + (rr - ti_r * a.G);
-          bf16_t* orow = c.out + (int64_t)cur_b * c.o_sb + (int64_t)ti_r * c.o_st + (int64_t)h_r * c.o_sh + lane * cpl;
-#pragma unroll
-          for (int e = 0; e < cpl; ++e) orow[e] = (bf16_t)(acc[e] * inv);
-        } else {
-          float* prow = c.part_o + (slot + rr) * D + lane * cpl;
-#pragma unroll
-          for (int e = 0; e < cpl; ++e) prow[e] = acc[e];
-          if (lane == 0) *(f32x2*)&c.part_ml[(slot + rr) * 2] = f32x2{M, lsum};
-        }
-      }
-      if (!more && r0 + kMergeRows >= R) return;
-      lds_barrier();  // the merge area is written again
     }
+    lds_barrier();
+    constexpr int kLanes = D / 4;        // lanes per row, four columns each
+    constexpr int kRowsAt = 64 / kLanes; // rows a wave takes at a time
+    const int dcol = lane % kLanes * 4;
+    const CacheArgs& c = cold_args();
+    for (int r0 = wave * kRowsAt; r0 < R; r0 += kDecWaves * kRowsAt) {
+      const int rr = min(r0 + lane / kLanes, R - 1);  // past the last row: that row again
+      float M = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < kDecWaves; ++w) M = fmaxf(M, (*row_ml(w, rr))[0]);
+      float lsum = 0.f;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kDecWaves; ++w) {
+        const f32x2 ml = *row_ml(w, rr);
+        const float wt = ml[0] == -INFINITY ? 0.f : fast_exp2(ml[0] - M);
+        lsum += ml[1] * wt;
+        acc += *(const f32x4*)&area(w)[rr * kPitch + dcol] * wt;
+      }
+      if (cur_whole) {
+        const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+        const int ti_r = rr / a.G;
+        const int h_r = cur_hk * a.G + (rr - ti_r * a.G);
+        bf16_t* orow = c.out + (int64_t)cur_b * c.o_sb + (int64_t)ti_r * c.o_st + (int64_t)h_r * c.o_sh;
+        *(bf16x4*)&orow[dcol] = __builtin_convertvector(acc * inv, bf16x4);
+      } else {
+        *(f32x4*)&c.part_o[(slot + rr) * D + dcol] = acc;
+        if (dcol == 0) *(f32x2*)&c.part_ml[(slot + rr) * 2] = f32x2{M, lsum};
+      }
+    }
+    if (!more) return;
+    lds_barrier();  // the merge's area is the second stages again
+    if (n_my > 1) issue(t0 + wave + kDecWaves, mk1, mv1);
   }
 }
 

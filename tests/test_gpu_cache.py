@@ -64,6 +64,9 @@ def test_short_chunks_around_the_decode_kernel(device, S, causal):
     (3, 1, 4, 4, 128, 9000, 4),     # equal shares: pairs over many shares
     (70, 1, 4, 1, 64, 3000, 5),     # shares over several pairs, batch rows past the first 64
     (5, 8, 4, 1, 128, 700, 6),      # 32 query rows merged over parts
+    (6, 17, 2, 2, 64, 900, 7),      # 17 query rows, several pairs per share
+    (40, 3, 10, 2, 128, 300, 8),    # 15 query rows, one workgroup per pair
+    (33, 32, 3, 3, 64, 260, 9),
 ])
 def test_decode_work_split(device, B, S, hq, hkv, d, L, seed):
     """One workgroup per pair, and the line of key tiles dealt to equal shares: ragged lengths
