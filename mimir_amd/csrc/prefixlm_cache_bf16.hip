@@ -484,10 +484,10 @@ constexpr float kRefRange = 30.f;  // how far (log2) a tile's reference may lie 
 // overlap; a unit of the line is both stages of every wave.
 constexpr int kShareWaves = 2;
 constexpr int kShareUnit = 2 * kShareWaves;
-// One workgroup per pair: four waves, one workgroup per CU, a unit is all tiles of a
-// pair, so every pair is whole and nothing is left to merge.
+// One workgroup per pair: four waves, one workgroup per CU; every pair is whole,
+// nothing is left to merge, and only the pair's own batch row is looked up (1024 rows of
+// 10 to 200 keys, 4 kv heads: 205 us with the line of all of them, 93 so).
 constexpr int kPairWaves = 4;
-constexpr int kPairUnit = 1 << 24;
 
 template <int D>
 struct DecTile {
@@ -525,9 +525,8 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
   return x;
 }
 
-// The line of key tiles, in units of kUnit tiles, as one wave sees it: 64 batch
+// The line of key tiles, in units of kShareUnit tiles, as one wave sees it: 64 batch
 // rows at a time, one per lane.
-template <int kUnit>
 struct TileLine {
   int first;  // batch row of lane 0
   int pos;    // position of the lane's batch row: cache_lengths clamped to [-S, L] (new row i goes to pos + i)
@@ -535,21 +534,63 @@ struct TileLine {
   int keys;   // keys it attends: cached and new ones inside the cache
   int units;  // units per kv head
   int incl;   // units per kv head of all batch rows up to this one
-  __device__ __forceinline__ void load(const CacheArgs& a, int first_, int before, int lane) {
-    first = first_;
+  struct Raw {
+    int64_t length, row;
+  };
+  static __device__ __forceinline__ Raw fetch(const CacheArgs& a, int first, int lane) {
     const int b = first + lane;
-    row = -1;
-    pos = keys = 0;
-    if (b < a.B) {
-      const int64_t n = load_index(a.cache_lengths, b, a.idx64), r = cache_row(a, b);
-      pos = n < -(int64_t)a.S ? -a.S : (n > a.L ? a.L : (int)n);
-      row = r >= 0 && r < a.rows ? (int)r : -1;
-      keys = row >= 0 ? min(max(pos, 0) + a.S, a.L) : 0;
-    }
-    units = ((keys + kDecKeys - 1) / kDecKeys + kUnit - 1) / kUnit;
+    Raw r = {0, -1};
+    if (b < a.B) r = {load_index(a.cache_lengths, b, a.idx64), cache_row(a, b)};
+    return r;
+  }
+  __device__ __forceinline__ void set(const CacheArgs& a, Raw r, int first_, int before) {
+    first = first_;
+    pos = r.length < -(int64_t)a.S ? -a.S : (r.length > a.L ? a.L : (int)r.length);
+    row = r.row >= 0 && r.row < a.rows ? (int)r.row : -1;
+    keys = row >= 0 ? min(max(pos, 0) + a.S, a.L) : 0;
+    units = ((keys + kDecKeys - 1) / kDecKeys + kShareUnit - 1) / kShareUnit;
     incl = before + wave_inclusive_sum(units);
   }
+  __device__ __forceinline__ void load(const CacheArgs& a, int first_, int before, int lane) {
+    set(a, fetch(a, first_, lane), first_, before);
+  }
   __device__ __forceinline__ int end() const { return __builtin_amdgcn_readlane(incl, 63); }
+};
+
+// The line of a batch of more than 64 rows (at most kLineRows): lane c holds the units
+// per kv head of batch rows 64 c .. 64 c + 63, and of all up to the last of them.  The
+// loads of four chunks are in flight together, and each workgroup then loads the one
+// chunk that it needs.  (Chunk after chunk, once for the total and once more up to its
+// own, a round trip each: 512 rows of 0 to 300 keys in 4096 positions, 4 kv heads, 64.3
+// us, so 59.8.)  Past kLineRows there is a workgroup per pair, which needs no line: 1000
+// rows of 0 to 300 keys, one kv head, 47.6 us with the line chunk after chunk, 38.5 so,
+// 30.1 with pairs; 512 of 0 to 2000, 4 kv heads, 212 with the line, 222 with pairs.
+constexpr int kLineRows = 512;
+struct LineChunks {
+  int units, incl;
+  template <typename F>
+  __device__ __forceinline__ void scan(const CacheArgs& a, int lane, F&& each) {
+    constexpr int kAhead = 4;
+    units = 0;
+    for (int c0 = 0; 64 * c0 < a.B; c0 += kAhead) {
+      TileLine::Raw raw[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) raw[i] = TileLine::fetch(a, 64 * (c0 + i), lane);
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        TileLine line;
+        line.set(a, raw[i], 64 * (c0 + i), 0);
+        each(line);
+        const int n = line.end();
+        if (lane == c0 + i) units = n;
+      }
+    }
+    incl = wave_inclusive_sum(units);
+  }
+  __device__ __forceinline__ int total() const { return __builtin_amdgcn_readlane(incl, 63); }
+  __device__ __forceinline__ int before(int c) const {
+    return __builtin_amdgcn_readlane(incl, c) - __builtin_amdgcn_readlane(units, c);
+  }
 };
 
 // Units per share for a line of `total` units.
@@ -559,24 +600,28 @@ __device__ __forceinline__ int share_of(const CacheArgs& a, int total) {
 // Part slot (of two per share) of the segment that starts at position u of the line.
 __device__ __forceinline__ int part_slot(int u, int per) { return 2 * (u / per) + (u % per != 0); }
 
-// Zero output for the batch rows without keys (outside the cache) among the
-// loaded ones, dealt to the workgroups.
-template <int D, int kUnit>
-__device__ __forceinline__ void zero_keyless(const CacheArgs& a, const TileLine<kUnit>& line, int lane) {
-  uint64_t none = __builtin_amdgcn_ballot_w64(line.first + lane < a.B && line.keys == 0);
-  for (; none != 0; none &= none - 1) {
-    const int b = line.first + __builtin_ctzll(none);
-    if (b % (int)gridDim.x != (int)blockIdx.x) continue;
-    const int Hq = a.Hkv * a.G;
-    for (int i = threadIdx.x; i < a.S * Hq * (D / 8); i += blockDim.x) {
-      const int c = i % (D / 8), row = i / (D / 8);
-      *(bf16x8*)&a.out[(int64_t)b * a.o_sb + (int64_t)(row / Hq) * a.o_st + (int64_t)(row % Hq) * a.o_sh + c * 8] =
-          bf16x8{};
-    }
+// Zero output for `heads` heads from h0 on of batch row b.
+template <int D>
+__device__ __forceinline__ void zero_rows(const CacheArgs& a, int b, int h0, int heads) {
+  for (int i = threadIdx.x; i < a.S * heads * (D / 8); i += blockDim.x) {
+    const int c = i % (D / 8), row = i / (D / 8);
+    *(bf16x8*)&a.out[(int64_t)b * a.o_sb + (int64_t)(row / heads) * a.o_st + (int64_t)(h0 + row % heads) * a.o_sh +
+                     c * 8] = bf16x8{};
   }
 }
 
-template <int D, int kDecWaves, int kUnit>
+// The same for the batch rows without keys (outside the cache) among the loaded ones,
+// dealt to the workgroups.
+template <int D>
+__device__ __forceinline__ void zero_keyless(const CacheArgs& a, const TileLine& line, int lane) {
+  uint64_t none = __builtin_amdgcn_ballot_w64(line.first + lane < a.B && line.keys == 0);
+  for (; none != 0; none &= none - 1) {
+    const int b = line.first + __builtin_ctzll(none);
+    if (b % (int)gridDim.x == (int)blockIdx.x) zero_rows<D>(a, b, 0, a.Hkv * a.G);
+  }
+}
+
+template <int D, int kDecWaves, bool kPairs>
 __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   constexpr int DT = D / 32;
   constexpr int KS = D / 16;
@@ -604,24 +649,39 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   const int l32 = lane & 31;
   const int hi = lane >> 5;
 
-  // This share [u_begin, u_end) of the line, and the first batch row it touches:
-  // lane j of the loaded rows, its units at `base` on the line.
-  TileLine<kUnit> line;
-  line.load(a, 0, 0, lane);
-  zero_keyless<D>(a, line, lane);
-  int total = line.end();
-  for (int first = 64; first < a.B; first += 64) {
-    line.load(a, first, total, lane);
-    zero_keyless<D>(a, line, lane);
-    total = line.end();
+  // This share [u_begin, u_end) of the line, and the first batch row it touches: lane j
+  // of the loaded rows.  One workgroup per pair: its batch row, and no line.
+  TileLine line;
+  int j, u_begin = 0, u_end = 1, per = 1;
+  if constexpr (kPairs) {
+    const int pair_b = blockIdx.x / a.Hkv;
+    line.load(a, pair_b & ~63, 0, lane);
+    j = pair_b & 63;
+    if (__builtin_amdgcn_readlane(line.keys, j) == 0) {
+      zero_rows<D>(a, pair_b, blockIdx.x % a.Hkv * a.G, a.G);
+      return;
+    }
+  } else {
+    LineChunks chunks;
+    int total;
+    if (a.B <= 64) {
+      line.load(a, 0, 0, lane);
+      zero_keyless<D>(a, line, lane);
+      total = line.end();
+    } else {
+      chunks.scan(a, lane, [&](const TileLine& l) { zero_keyless<D>(a, l, lane); });
+      total = chunks.total();
+    }
+    per = share_of(a, total * a.Hkv);
+    u_begin = (int)blockIdx.x * per;
+    u_end = min(total * a.Hkv, u_begin + per);
+    if (u_begin >= u_end) return;
+    if (a.B > 64) {
+      const int c = __builtin_ctzll(__builtin_amdgcn_ballot_w64(chunks.incl * a.Hkv > u_begin));
+      line.load(a, 64 * c, chunks.before(c), lane);
+    }
+    j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl * a.Hkv > u_begin));
   }
-  const int per = share_of(a, total * a.Hkv);
-  const int u_begin = (int)blockIdx.x * per;
-  const int u_end = min(total * a.Hkv, u_begin + per);
-  if (u_begin >= u_end) return;
-  if (a.B > 64) line.load(a, 0, 0, lane);
-  while (line.end() * a.Hkv <= u_begin) line.load(a, line.first + 64, line.end(), lane);
-  int j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl * a.Hkv > u_begin));
 
   const int R = a.S * a.G;  // <= kDecRows
   const bool row_ok = l32 < R;
@@ -668,17 +728,14 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   bf16_t *kbase, *vbase;
   bf16x8 qf[KS];
 
-  // The other batch rows on the segment's cache row: f(batch row, its position).
+  // The other batch rows on the segment's cache row: f(batch row, its position).  With
+  // indices the call has at most 64 batch rows, all of them in the line.
   auto for_others = [&](auto&& f) __attribute__((always_inline)) {
     if (a.batch_indices == nullptr) return;
-    TileLine<kUnit> other = line;
-    for (int first = 0; first < a.B; first += 64) {
-      if (a.B > 64) other.load(a, first, 0, lane);
-      uint64_t same = __builtin_amdgcn_ballot_w64(other.row == crow && first + lane != b);
-      for (; same != 0; same &= same - 1) {
-        const int o = __builtin_ctzll(same);
-        f(first + o, __builtin_amdgcn_readlane(other.pos, o));
-      }
+    uint64_t same = __builtin_amdgcn_ballot_w64(line.row == crow && lane != b);
+    for (; same != 0; same &= same - 1) {
+      const int o = __builtin_ctzll(same);
+      f(o, __builtin_amdgcn_readlane(line.pos, o));
     }
   };
   // Overlay tile t's copy with the new rows (of batch row o, at position p on)
@@ -733,19 +790,27 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   auto begin = [&]() __attribute__((always_inline)) {
     const CacheArgs& c = cold_args();
     b = line.first + j;
-    const int units_b = __builtin_amdgcn_readlane(line.units, j);
-    const int base = (__builtin_amdgcn_readlane(line.incl, j) - units_b) * c.Hkv;
     kv = __builtin_amdgcn_readlane(line.keys, j);
     pos_b = __builtin_amdgcn_readlane(line.pos, j);
     crow = __builtin_amdgcn_readlane(line.row, j);
-    hk = (u0 - base) / units_b;
-    const int unit0 = (u0 - base) - hk * units_b;
-    const int unit1 = min(units_b, unit0 + u_end - u0);
-    whole = unit0 == 0 && unit1 == units_b;
-    u_next = u0 + unit1 - unit0;
-    u_row = base + units_b * c.Hkv;
-    t0 = unit0 * kUnit;
-    const int t_end = min((int64_t)unit1 * kUnit, (int64_t)(kv + kDecKeys - 1) / kDecKeys);
+    int t_end = (kv + kDecKeys - 1) / kDecKeys;
+    if constexpr (kPairs) {
+      hk = blockIdx.x - b * c.Hkv;
+      whole = true;
+      u_next = u_end;
+      t0 = 0;
+    } else {
+      const int units_b = __builtin_amdgcn_readlane(line.units, j);
+      const int base = (__builtin_amdgcn_readlane(line.incl, j) - units_b) * c.Hkv;
+      hk = (u0 - base) / units_b;
+      const int unit0 = (u0 - base) - hk * units_b;
+      const int unit1 = min(units_b, unit0 + u_end - u0);
+      whole = unit0 == 0 && unit1 == units_b;
+      u_next = u0 + unit1 - unit0;
+      u_row = base + units_b * c.Hkv;
+      t0 = unit0 * kShareUnit;
+      t_end = min(unit1 * kShareUnit, t_end);
+    }
     n_my = t0 + wave < t_end ? (t_end - t0 - wave + kDecWaves - 1) / kDecWaves : 0;  // this wave's tiles
     const int clen = max(pos_b, 0);
     kend_lane = row_ok ? (c.causal ? min(clen + ti + 1, kv) : kv) : 0;
@@ -939,16 +1004,16 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
 // One kernel per head_dim, by name: two instantiations of one kernel template
 // launched from the two branches below lost one host stub in this toolchain.
 __global__ __launch_bounds__(kShareWaves * 64, 1) void cache_decode_d128_kernel(const CacheArgs a) {
-  cache_decode_body<128, kShareWaves, kShareUnit>(a);
+  cache_decode_body<128, kShareWaves, false>(a);
 }
 __global__ __launch_bounds__(kShareWaves * 64, 1) void cache_decode_d64_kernel(const CacheArgs a) {
-  cache_decode_body<64, kShareWaves, kShareUnit>(a);
+  cache_decode_body<64, kShareWaves, false>(a);
 }
 __global__ __launch_bounds__(kPairWaves * 64, 1) void cache_decode_pairs_d128_kernel(const CacheArgs a) {
-  cache_decode_body<128, kPairWaves, kPairUnit>(a);
+  cache_decode_body<128, kPairWaves, true>(a);
 }
 __global__ __launch_bounds__(kPairWaves * 64, 1) void cache_decode_pairs_d64_kernel(const CacheArgs a) {
-  cache_decode_body<64, kPairWaves, kPairUnit>(a);
+  cache_decode_body<64, kPairWaves, true>(a);
 }
 
 // Output rows of the (batch row, kv head) pairs whose key tiles lie in several
@@ -962,19 +1027,19 @@ __device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
   const int rr = blockIdx.x % groups * kWaves + wave;
   const int hk = blockIdx.x / groups % a.Hkv;
   const int b = blockIdx.x / groups / a.Hkv;
-  TileLine<kShareUnit> line;
-  line.load(a, 0, 0, lane);
-  int total = line.end(), units_b = 0, before = 0;
-  for (int first = 0;;) {
-    if (b >= first && b < first + 64) {
-      units_b = __builtin_amdgcn_readlane(line.units, b - first);
-      before = __builtin_amdgcn_readlane(line.incl, b - first) - units_b;
-    }
-    first += 64;
-    if (first >= a.B) break;
-    line.load(a, first, total, lane);
+  TileLine line;
+  int total;
+  if (a.B <= 64) {
+    line.load(a, 0, 0, lane);
     total = line.end();
+  } else {
+    LineChunks chunks;
+    chunks.scan(a, lane, [](const TileLine&) {});
+    total = chunks.total();
+    line.load(a, b & ~63, chunks.before(b / 64), lane);
   }
+  const int units_b = __builtin_amdgcn_readlane(line.units, b & 63);
+  const int before = __builtin_amdgcn_readlane(line.incl, b & 63) - units_b;
   const int per = share_of(a, total * a.Hkv);
   const int g0 = before * a.Hkv + hk * units_b;  // the pair's units [g0, g0 + units_b) of the line
   const int w0 = g0 / per, n = units_b > 0 ? (g0 + units_b - 1) / per - w0 + 1 : 0;  // shares it lies in
@@ -1009,8 +1074,9 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
     // for any batch (two rounds of copies) up to 2048 for a pair per CU.  64 x 4
     // pairs (one launch against two, no merge): 100 to 1000 keys 25.5 -> 19.0 us, 100
     // to 2000 keys 37.5 / 37.9, 100 to 4000 keys 65 / 72 (the longest pair runs alone).
+    // And for a batch past kLineRows, where a share would look for its pairs too long.
     const int64_t pair_keys = 8 * s.groups;
-    s.pairs = max_kv <= (pair_keys < 256 ? 256 : (pair_keys < 2048 ? pair_keys : 2048));
+    s.pairs = p.batch > kLineRows || max_kv <= (pair_keys < 256 ? 256 : (pair_keys < 2048 ? pair_keys : 2048));
     if (s.pairs) {  // one workgroup per pair
       s.units = s.groups;
     } else {
@@ -1073,10 +1139,10 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   // from the cache, which asks for cache rows that share no memory: a batch row's new
   // rows are then seen through its own cache row alone.  (Shared, e.g. a cache expanded
   // over the batch, every batch row sees all new rows, as after appending all of them.)
-  // Decode finds the batch rows on one cache row by their indices; prefill does not, and
-  // needs one set of copy offsets for the new rows and the cache.
+  // Decode finds the batch rows on one cache row by their indices, up to 64 of them;
+  // prefill does not, and needs one set of copy offsets for the new rows and the cache.
   a.append = cache_rows_distinct(p) &&
-             (sp.decode || (a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st));
+             (sp.decode ? a.batch_indices == nullptr || a.B <= 64 : (a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st));
   const int64_t appends = (int64_t)a.B * a.S * a.Hkv * (a.D / 8);
   if ((sp.decode ? !sp.pairs : sp.splits > 1) && p.workspace == nullptr) return hipErrorInvalidValue;
   if (appends > 0 && !a.append) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);

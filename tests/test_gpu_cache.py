@@ -166,6 +166,54 @@ def test_cache_rows_that_share_memory(device, d, S, lens, form):
     assert torch.equal(dev[0].cpu(), kf) and torch.equal(dev[0 if form == "one tensor" else 1].cpu(), vf)
 
 
+@pytest.mark.parametrize("B,S,hq,hkv,d,L,rows", [
+    (65, 1, 2, 1, 64, 3000, None),        # shares: one batch row past the first 64
+    (130, 2, 4, 2, 128, 1300, None),      # three chunks of batch rows
+    (512, 1, 2, 1, 64, 1100, "distinct"), # as many as a share looks through; appended first
+    (513, 1, 2, 1, 64, 1100, None),       # a workgroup per pair from here on
+    (100, 1, 4, 2, 128, 300, "distinct"), # pairs, appended first
+    (200, 1, 4, 1, 64, 1500, "shared"),   # 200 batch rows on 90 cache rows
+    (70, 2, 2, 2, 128, 200, "shared"),
+])
+def test_decode_of_large_batches(device, B, S, hq, hkv, d, L, rows):
+    """More batch rows than a wave has lanes: ragged lengths among them 0 and the whole cache,
+    chosen cache rows, batch rows that share one (each at positions of its own)."""
+    gen = torch.Generator().manual_seed(B)
+    lens = torch.randint(0, L - S + 1, (B,), generator=gen).tolist()
+    lens[0], lens[-1] = 0, L - S
+    if rows is None:
+        _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=True, seed=B)
+    elif rows == "distinct":
+        _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=True, seed=B, cache_rows=B + 3,
+             rows=torch.randperm(B + 3, generator=gen)[:B].tolist())
+    else:
+        n = 90 if B > 90 else 40
+        lens = (torch.randperm(L // S - 1, generator=gen)[:B] * S).tolist()
+        _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=False, seed=B, cache_rows=n,
+             rows=[b % n for b in range(B)])
+
+
+@pytest.mark.parametrize("B,L", [(3, 200), (3, 2000), (100, 2000), (600, 100)])
+def test_decode_batch_rows_without_keys(device, B, L):
+    """Batch rows outside the cache get zeros, write nothing and take no part of the work."""
+    gen = torch.Generator().manual_seed(B)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(BF16)
+    q, k, v, keys, values = mk(B, 1, 4, 64), mk(B, 1, 2, 64), mk(B, 1, 2, 64), mk(B, L, 2, 64), mk(B, L, 2, 64)
+    rows = torch.randperm(B, generator=gen)
+    lens = torch.randint(0, L, (B,), generator=gen)
+    gone = torch.arange(B) % 3 == 1
+    ck, cv = keys.clone(), values.clone()
+    ref = torch.zeros_like(q)
+    ref[~gone] = LO.attention_with_cache(q[~gone], k[~gone], v[~gone], ck, cv, lens[~gone], True, rows[~gone])
+    rows[gone] = torch.where(torch.arange(int(gone.sum())) % 2 == 0, -1, B)
+    cache = Cache(keys.to(device), values.to(device))
+    out = attention_with_cache(q.to(device), k.to(device), v.to(device), cache, lens.to(device), True, rows.to(device))
+    torch.cuda.synchronize()
+    assert torch.count_nonzero(out[gone]) == 0
+    assert (out.float().cpu() - ref.float()).abs().max().item() <= 2e-2
+    assert torch.equal(cache.keys.cpu(), ck) and torch.equal(cache.values.cpu(), cv)
+
+
 def test_decode_uneven_rows(device):
     """Rows whose key ranges split into different numbers of parts (1 key to the whole cache)."""
     _run(device, B=8, S=1, hq=16, hkv=4, d=128, L=4096, lens=[0, 63, 64, 65, 1000, 4095, 2048, 129],
