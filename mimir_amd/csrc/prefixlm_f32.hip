@@ -11,8 +11,9 @@
 // A workgroup owns 32 rows (queries, or keys for dK / dV) of one head; its four
 // waves take the 32-row tiles of the other side in turn, each with accumulators
 // of its own that are added through LDS at the end.  Small fp32 batches (a few
-// thousand tokens) then still put two waves on every SIMD, and the tile loop
-// holds no barrier.  With the owned rows on the columns of every product, S^T =
+// thousand tokens) then still put two waves on every SIMD (one in the backward at
+// head_dim 96 and 128, whose operands take more than half of its registers), and
+// the tile loop holds no barrier.  With the owned rows on the columns of every product, S^T =
 // K Q^T (dK / dV: S = Q K^T) leaves the probabilities in registers exactly as
 // the B operand of the next product wants them: register r of lane half hi is
 // row 8 (r / 4) + 4 hi + r % 4, and one matrix step sums over the two rows that
@@ -29,15 +30,17 @@
 //    wave at head_dim 64, well under what L1 and L2 deliver.  Each operand is
 //    requested one product (D / 2 matrix steps, 2048 cycles at head_dim 64)
 //    before its use, which covers the latency without double buffers.
+//  * S and dP are added up from short chains of matrix steps (kScoreChain), which
+//    keeps their rounding at that of a row spread over lanes.
 //    Row ranges are enforced by the buffer resource of the tile: rows past the
 //    end read as zeros.
 //
 // Bound by the matrix unit and, on small batches, by the number of workgroups:
 // 4 x 512 tokens, 8 heads, head_dim 64 (1.2 GFLOP forward, 5.0 executed in the
-// backward): forward 86 -> 25 us (a workgroup's start-up and merge are a third
-// of it), dQ + dK / dV 310 -> 77 us against the vector-ALU kernels these
+// backward): forward 86 -> 27 us (a workgroup's start-up and merge are a third
+// of it), dQ + dK / dV 310 -> 78 us against the vector-ALU kernels these
 // replace; one sequence of 4096 tokens, same heads, forward + backward 3.20 ->
-// 0.68 ms.
+// 0.75 ms.
 #include "prefixlm_common.h"
 
 namespace {
@@ -110,8 +113,8 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
 
 // Keeps the instruction scheduler from moving the loads in front of it behind
 // the products (it otherwise sinks them to their use, which then waits for
-// memory: forward 26.5 -> 25.3 us).  Not in the backward, whose registers are
-// full (28 spilled with it, 85 -> 99 us).
+// memory: forward 26.5 -> 25.3 us), or from moving those behind a product in front
+// of it, where they would hold registers that the product needs (backward).
 __device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(0); }
 
 // Row of accumulator register r in lane half hi.
@@ -142,24 +145,30 @@ struct Tile {
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) x[c] = __builtin_bit_cast(f32x4, buf_load16(r, lane_off + 32 * c));
   }
-  // Column form: step s holds row acc_row(s, hi), columns kCols * (lane % 32) + 0 ..
-  __device__ __forceinline__ void cols(float (&x)[16][kCols], uint32_t lane_off, uint32_t row_bytes) const {
+  // Column form: step s holds row acc_row(s, hi), columns kCols * (lane % 32) + 0 .. : one
+  // resource per eight rows, so that four lane offsets serve all of them.
+  static __device__ __forceinline__ void cols(float (&x)[16][kCols], const float* base, int64_t stride, int row0,
+                                              int nrows, uint32_t lane_off, uint32_t row_bytes) {
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int off = (int)(lane_off + acc_row(s, 0) * row_bytes);
-      if constexpr (kCols == 1) {
-        x[s][0] = buf_load_f32(r, off);
-      } else if constexpr (kCols == 2) {
-        const f32x2 t = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-        x[s][0] = t[0]; x[s][1] = t[1];
-      } else if constexpr (kCols == 3) {
-        const auto t = __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0);
+    for (int g = 0; g < 4; ++g) {
+      const Tile t(base, stride, row0 + 8 * g, nrows);
 #pragma unroll
-        for (int e = 0; e < 3; ++e) x[s][e] = __uint_as_float(t[e]);
-      } else {
-        const f32x4 t = __builtin_bit_cast(f32x4, buf_load16(r, off));
+      for (int e = 0; e < 4; ++e) {
+        const int s = 4 * g + e, off = (int)(lane_off + e * row_bytes);
+        if constexpr (kCols == 1) {
+          x[s][0] = buf_load_f32(t.r, off);
+        } else if constexpr (kCols == 2) {
+          const f32x2 v = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(t.r, off, 0, 0));
+          x[s][0] = v[0]; x[s][1] = v[1];
+        } else if constexpr (kCols == 3) {
+          const auto v = __builtin_amdgcn_raw_buffer_load_b96(t.r, off, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[s][e] = t[e];
+          for (int c = 0; c < 3; ++c) x[s][c] = __uint_as_float(v[c]);
+        } else {
+          const f32x4 v = __builtin_bit_cast(f32x4, buf_load16(t.r, off));
+#pragma unroll
+          for (int c = 0; c < 4; ++c) x[s][c] = v[c];
+        }
       }
     }
   }
@@ -194,18 +203,57 @@ __device__ __forceinline__ void stage_owned(float* dst, const float* base, int64
   }
 }
 
-// X W^T for a streamed tile x in row form and the owned rows w in LDS: 32 x 32.
+// Matrix steps (two columns each) that S and dP add up in one chain before the chains
+// are added to one another.  A chain rounds after every product, so its error grows with
+// its length, and one over all of D was up to 1.8 times as far off as the short chains
+// and tree of a row spread over lanes (short documents, whose sums over keys are few).
+// S is formed alike in the forward and the backward: its error is then in the logsumexp
+// too, and the rows of P sum to 1.  The relative error against 64 bits of O, dQ, dK
+// (documents of 2 to 12 tokens; one chain / row over lanes / so), x 1e-7:
+//   D  32: 0.98 2.5 2.5 / 0.81 2.2 2.2 / 0.76 2.1 2.1    D  64: 1.2 3.0 3.0 / 0.85 2.3 2.5 / 0.80 2.2 2.3
+//   D  96: 1.4 3.6 3.6 / 0.91 2.7 2.8 / 0.85 2.7 2.7    D 128: 1.6 4.0 4.0 / 0.91 2.8 3.0 / 0.87 2.7 2.7
+// The additions and their waits for the products cost, with one chain / so: forward +
+// backward of 8192 tokens in documents of 2048, 8 heads, D 64 0.95 / 0.99 ms, of 4096, 16 / 4
+// heads, D 128 2.75 / 3.04 (15.8 on the vector ALUs); 4 x 512, 8 heads, D 64 unchanged.
 template <int D>
-__device__ __forceinline__ f32x16 product_rows(const f32x4 (&x)[D / 8], const float* w, int l32, int hi) {
-  f32x16 acc = f32x16{};
-  const float* row = w + l32 * Smem<D>::kStride + 4 * hi;
+constexpr int kScoreChain = D == 32 ? 2 : D == 128 ? 8 : 4;
+template <int D>
+constexpr int kDpChain = D == 32 ? 4 : D == 64 ? 8 : 16;
+
+// Steps [S0, S0 + N) of X W^T: chains of kChain steps, added as a tree.
+template <int D, int kChain, int S0, int N>
+__device__ __forceinline__ f32x16 product_tree(const f32x4 (&x)[D / 8], const float* row) {
+  if constexpr (N > kChain) {
+    const f32x16 left = product_tree<D, kChain, S0, N / 2>(x, row);
+    return left + product_tree<D, kChain, S0 + N / 2, N / 2>(x, row);
+  } else {
+    f32x16 acc = f32x16{};
 #pragma unroll
-  for (int c = 0; c < D / 8; ++c) {
-    const f32x4 b = *(const f32x4*)&row[8 * c];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc = mfma_f32(x[c][e], b[e], acc);
+    for (int s = S0; s < S0 + N; ++s) acc = mfma_f32(x[s / 4][s % 4], row[8 * (s / 4) + s % 4], acc);
+    return acc;
   }
-  return acc;
+}
+
+// X W^T for a streamed tile x in row form and the owned rows w in LDS: 32 x 32, in
+// trees of 16 steps added in turn.  Each sum is pinned where it is formed: the compiler
+// otherwise moves the additions to their use and holds all chains until then.
+template <int D, int kChain>
+__device__ __forceinline__ f32x16 product_rows(const f32x4 (&x)[D / 8], const float* w, int l32, int hi) {
+  const float* row = w + l32 * Smem<D>::kStride + 4 * hi;
+  f32x16 sum = product_tree<D, kChain, 0, 16>(x, row);
+  if constexpr (D > 32) {
+    sum += product_tree<D, kChain, 16, 16>(x, row);
+    __asm__ volatile("" : "+v"(sum));
+  }
+  if constexpr (D > 64) {
+    sum += product_tree<D, kChain, 32, 16>(x, row);
+    __asm__ volatile("" : "+v"(sum));
+  }
+  if constexpr (D > 96) {
+    sum += product_tree<D, kChain, 48, 16>(x, row);
+    __asm__ volatile("" : "+v"(sum));
+  }
+  return sum;
 }
 
 // acc[dt] += X^T P: X the streamed tile in column form, P [32 x 32] in accumulator
@@ -236,10 +284,10 @@ __device__ __forceinline__ void put_partial(float* dst, const f32x16 (&acc)[D / 
   }
 }
 
-// Sum of the four partials times `scale(row)` -> global rows row0 .. of [rows, D].
-template <int D, typename Scale>
+// finish(row, sum of the four partials) -> global rows row0 .. of [rows, D].
+template <int D, typename Finish>
 __device__ __forceinline__ void store_sum(const float* x, float* base, int64_t stride, int row0, int nrows,
-                                          Scale&& scale) {
+                                          Finish&& finish) {
   using S = Smem<D>;
   for (int i = threadIdx.x; i < kRows * (D / 4); i += kThreads) {
     const int row = i / (D / 4), c = i % (D / 4);
@@ -247,7 +295,7 @@ __device__ __forceinline__ void store_sum(const float* x, float* base, int64_t s
     f32x4 t = *(const f32x4*)&x[row * S::kStride + 4 * c];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) t += *(const f32x4*)&x[w * S::kTile + row * S::kStride + 4 * c];
-    *(f32x4*)&base[(int64_t)(row0 + row) * stride + 4 * c] = t * scale(row);
+    *(f32x4*)&base[(int64_t)(row0 + row) * stride + 4 * c] = finish(row, t);
   }
 }
 
@@ -292,9 +340,9 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(const F32Args a) {
   float m_run = -INFINITY, l_run = 0.f;
   for (; kt < n_tiles; kt += kWaves) {
     const int k0 = kt * kRows;
-    Tile<D>(vb, a.v_st, k0, g.n).cols(vx, vo.col, vo.row_bytes);
+    Tile<D>::cols(vx, vb, a.v_st, k0, g.n, vo.col, vo.row_bytes);
     pin();
-    f32x16 st = product_rows<D>(kx, sm.x, ln.l32, ln.hi);
+    f32x16 st = product_rows<D, kScoreChain<D>>(kx, sm.x, ln.l32, ln.hi);
     // the next tile's rows (none past the last: an empty range reads zeros)
     Tile<D>(kb, a.k_st, k0 + kWaves * kRows, kt + kWaves < n_tiles ? g.n : 0).rows(kx, ko.row);
     pin();
@@ -344,13 +392,13 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(const F32Args a) {
   }
   __syncthreads();
   if (threadIdx.x < kRows) {
-    sm.l[0][threadIdx.x] = 1.f / l_sum;
+    sm.l[0][threadIdx.x] = l_sum;
     if (m0 + (int)threadIdx.x < g.nq && a.lse != nullptr)
       a.lse[(int64_t)h * a.lse_sh + g.start + m0 + threadIdx.x] = M * a.scale + logf(l_sum);
   }
   __syncthreads();
   store_sum<D>(sm.x, a.o + (int64_t)g.start * a.o_st + (int64_t)h * a.o_sh, a.o_st, m0, g.nq,
-               [&](int row) { return sm.l[0][row]; });
+               [&](int row, f32x4 t) { return t / sm.l[0][row]; });  // not times 1 / l: one rounding less
 }
 
 // dQ of one (head, sequence, 32-query tile): dQ^T += K^T dS^T over the key tiles.
@@ -393,10 +441,12 @@ __device__ __forceinline__ void dq_body(const F32Args& a, Smem<D>& sm, int h, in
   for (; kt < n_tiles; kt += kWaves) {
     const int k0 = kt * kRows;
     const int n_next = kt + kWaves < n_tiles ? g.n : 0;
-    Tile<D>(kb, a.k_st, k0, g.n).cols(kc, ko.col, ko.row_bytes);
-    f32x16 st = product_rows<D>(kx, sq, ln.l32, ln.hi);
+    f32x16 st = product_rows<D, kScoreChain<D>>(kx, sq, ln.l32, ln.hi);
+    pin();
+    Tile<D>::cols(kc, kb, a.k_st, k0, g.n, ko.col, ko.row_bytes);
     Tile<D>(kb, a.k_st, k0 + kWaves * kRows, n_next).rows(kx, ko.row);
-    const f32x16 dp = product_rows<D>(vx, sdo, ln.l32, ln.hi);
+    const f32x16 dp = product_rows<D, kDpChain<D>>(vx, sdo, ln.l32, ln.hi);
+    pin();
     Tile<D>(vb, a.v_st, k0 + kWaves * kRows, n_next).rows(vx, vo.row);
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[r] = fast_exp2(__builtin_fmaf(st[r], a.scale_log2, -lse2));
@@ -414,7 +464,7 @@ __device__ __forceinline__ void dq_body(const F32Args& a, Smem<D>& sm, int h, in
   put_partial<D>(sm.x + ln.wave * Smem<D>::kTile, acc, a.scale, ln.l32, ln.hi);
   __syncthreads();
   store_sum<D>(sm.x, a.dq + (int64_t)g.start * a.dq_st + (int64_t)h * a.dq_sh, a.dq_st, m0, g.nq,
-               [](int) { return 1.f; });
+               [](int, f32x4 t) { return t; });
 }
 
 // dK and dV of one (kv head, sequence, 32-key tile): the waves take the (q head,
@@ -464,8 +514,12 @@ __device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk,
   for (int it = ln.wave; it < steps; it += kWaves) {
     const int q0 = (t0 + t) * kRows;
     const int h = hk * a.group + hh;
-    const Tile<D> qt = tile_of(qb, a.q_st, a.q_sh), ot = tile_of(ob, a.do_st, a.do_sh);
-    ot.cols(oc, oo.col, oo.row_bytes);
+    const float *const qh = qb + (int64_t)hh * a.q_sh, *const oh = ob + (int64_t)hh * a.do_sh;
+    t += kWaves;
+    wrap();
+    f32x16 p = product_rows<D, kScoreChain<D>>(qx, sk, ln.l32, ln.hi);
+    pin();
+    Tile<D>::cols(oc, oh, a.do_st, q0, g.nq, oo.col, oo.row_bytes);
     // Rows of the tile past the last query are read too (other rows, or the
     // workspace section behind the array) and masked below.
     const f32x4u* const lp = (const f32x4u*)(a.lse2 + (int64_t)h * a.T + g.start + q0 + 4 * ln.hi);
@@ -475,11 +529,9 @@ __device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk,
     for (int e = 0; e < 4; ++e) lse[e] = lp[2 * e];
 #pragma unroll
     for (int e = 0; e < 4; ++e) dlt[e] = dp[2 * e];
-    t += kWaves;
-    wrap();
-    f32x16 p = product_rows<D>(qx, sk, ln.l32, ln.hi);
-    qt.cols(qc, qo.col, qo.row_bytes);
-    f32x16 ds = product_rows<D>(ox, sv, ln.l32, ln.hi);
+    f32x16 ds = product_rows<D, kDpChain<D>>(ox, sv, ln.l32, ln.hi);
+    pin();
+    Tile<D>::cols(qc, qh, a.q_st, q0, g.nq, qo.col, qo.row_bytes);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       p[r] = fast_exp2(__builtin_fmaf(p[r], a.scale_log2, -lse[r >> 2][r & 3]));
@@ -504,12 +556,12 @@ __device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk,
   put_partial<D>(mine, dva, 1.f, ln.l32, ln.hi);
   __syncthreads();
   store_sum<D>(base, a.dv + (int64_t)g.start * a.dv_st + (int64_t)hk * a.dv_sh, a.dv_st, k0, g.n,
-               [](int) { return 1.f; });
+               [](int, f32x4 t) { return t; });
   __syncthreads();
   put_partial<D>(mine, dka, a.scale, ln.l32, ln.hi);
   __syncthreads();
   store_sum<D>(base, a.dk + (int64_t)g.start * a.dk_st + (int64_t)hk * a.dk_sh, a.dk_st, k0, g.n,
-               [](int) { return 1.f; });
+               [](int, f32x4 t) { return t; });
 }
 
 // dK / dV units, then dQ units, in one launch: independent work, and the lighter

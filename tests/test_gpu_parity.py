@@ -218,6 +218,30 @@ def test_f32_tile_edges(device, d, hq, hkv, causal):
         assert torch.equal(x.detach().cpu(), got[name]), name
 
 
+@pytest.mark.parametrize("d,o_bound,dq_bound", [(32, 9.0e-8, 2.3e-7), (64, 1.0e-7, 2.6e-7), (96, 1.1e-7, 3.1e-7),
+                                                (128, 1.15e-7, 3.2e-7)])
+def test_f32_error_on_short_documents(device, d, o_bound, dq_bound):
+    """Documents of 2 to 12 tokens, where the rounding of the dot products over head_dim shows
+    (relative 2-norm error against 64 bits, O and dQ).  The bounds lie half way, in ratio,
+    between what short chains added as a tree give (0.76, 0.80, 0.85, 0.87 and 2.1, 2.2, 2.7, 2.7 x
+    1e-7) and one chain over head_dim (0.98, 1.2, 1.4, 1.6 and 2.5, 3.0, 3.6, 4.0)."""
+    gen = torch.Generator().manual_seed(d)
+    lens = torch.randint(2, 13, (150,), generator=gen).tolist()
+    prefixes = [int(torch.randint(0, n + 1, (1,), generator=gen)) for n in lens]
+    err = {}
+    for seed in range(4):
+        case = make_case(lens, prefixes, 4, 2, d, seed=seed, dtype=torch.float32)
+        got = run_gpu(case, device)
+        q, k, v, dout = (x.double() for x in (case.q, case.k, case.v, case.dout))
+        ref = {"o": dense_forward(q, k, v, False, *case.oracle_args())}
+        ref["dq"] = dense_backward(q, k, v, ref["o"], dout, False, *case.oracle_args())[0]
+        for name, r in ref.items():
+            assert r.dtype == torch.float64
+            err[name] = err.get(name, 0.0) + float((got[name].double() - r).norm() / r.norm()) / 4
+    print(f"[f32 short] d={d} {err}", flush=True)
+    assert err["o"] <= o_bound and err["dq"] <= dq_bound
+
+
 @pytest.mark.parametrize("lead,tail", [(1, 0), (37, 300), (0, 2500)])
 @pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (32, torch.float32)], ids=["bf16", "fp32"])
 def test_padding_rows_before_and_after(device, lead, tail, d, dtype):
