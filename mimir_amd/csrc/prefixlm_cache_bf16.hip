@@ -9,8 +9,8 @@
 //   cache_append_kernel      the scatter of k_new / v_new into the cache rows, first,
 //                            where the attention kernels do not do it themselves
 //   decode (at most 32 query rows per kv head, e.g. S = 1):
-//     cache_decode_*_kernel  appends the new rows and attends, each workgroup an
-//                            equal share of all key tiles of the call
+//     cache_decode_*_kernel  appends the new rows and attends, the workgroups equal
+//                            shares of all key tiles of the call
 //     cache_merge_kernel     adds the partial rows of the shares
 //   otherwise:
 //     cache_attn_kernel      one workgroup per (batch row, kv head, 128 query rows,
@@ -50,7 +50,7 @@ struct CacheArgs {
   float scale_log2;
   float* part_o;   // [unit, kRows, D] unnormalized O of each split (splits > 1)
   float* part_ml;  // [unit, kRows, 2]: running max (exp2 domain) and sum
-  int shares;      // decode: workgroups the key tiles of the call are dealt to
+  int shares;      // decode: runs of key tiles, one workgroup per kv head each
   int cus;         // CUs of the device
   int append;      // the attention kernel appends the new rows itself
 };
@@ -451,20 +451,23 @@ __global__ __launch_bounds__(kThreads) void cache_merge_splits_d64_kernel(const 
 // ---------------------------------------------------------------------------
 // Decode: at most 32 query rows per kv head (R = S * G <= 32, e.g. S = 1); bound
 // by the read of the cache, and for a few rows by the chain of memory round
-// trips.  The 32-key tiles of all (batch row, kv head) pairs form one line,
-// batch rows outermost; every workgroup takes an equal share of it (at least
-// kMinShare tiles), so rows of very different lengths keep all CUs busy to the
-// end.  A share covers one or more segments (tiles of one pair).  The rows of a
+// trips.  The 32-key tiles of all batch rows form one line, in units of
+// kShareUnit, which is dealt evenly to shares (Shares), each of one workgroup per
+// kv head, so rows of very different lengths keep all CUs busy to the end.  A
+// share covers one or more segments (tiles of one batch row).  The query rows of a
 // segment fit one wave, so instead of sharing 64-key tiles behind workgroup
-// barriers, each of the four waves streams its own tiles of the segment through
-// two LDS stages of its own and waits only for its own copies: four independent
-// copy pipelines per workgroup, one workgroup per CU.  The waves' partial rows
-// are merged through LDS.  A pair inside one share is finished there; the parts
-// of the others go to the workspace and cache_merge_kernel adds them.  A second
-// kernel needs no arrival counters, whose clearing took a launch of its own, and
-// no device-coherent round trips: merging in the last share to arrive (flags with
-// a value of the call's own instead of counters) left one launch, but 12.5 us of
-// it instead of 7.4 + 4.4 for one row and 22.5 instead of 12.6 + 4.3 for eight.
+// barriers, each of the kShareWaves waves streams its own tiles of the segment
+// through two LDS stages of its own and waits only for its own copies: two
+// independent copy pipelines per workgroup, two workgroups per CU.  The waves'
+// partial rows are merged through LDS.  A (batch row, kv head) pair inside one
+// share is finished there; the parts of the others go to the workspace and
+// cache_merge_* adds them.  A second kernel needs no arrival counters, whose
+// clearing took a launch of its own, and no device-coherent round trips: merging in
+// the last share to arrive (flags with a value of the call's own instead of
+// counters) left one launch, but 12.5 us of it instead of 7.4 + 4.4 for one row and
+// 22.5 instead of 12.6 + 4.3 for eight.  Where pairs fill the chip about evenly
+// (cache_split) each takes one workgroup of kPairWaves waves instead, and nothing
+// is left to merge.
 //
 // The new rows are appended here too: the wave whose tile holds one stores it to
 // the cache and to its LDS copy of the tile.  Batch rows that share a cache row
@@ -473,8 +476,8 @@ __global__ __launch_bounds__(kThreads) void cache_merge_splits_d64_kernel(const 
 //
 // Measured against an append kernel, one workgroup of four waves per (pair, equal
 // split) and a counted merge in it (Hq 16, Hkv 4, D 128): 64 rows of 512 to 8000 keys
-// 138 -> 119 us (5.0 TB/s), 32 rows of 100 to 4000 41 -> 33, one row of 8000 24 -> 15;
-// 8 rows of 1000 to 3600 18.2 -> 17.9, of which the two launches and their chains of
+// 140 -> 117 us (5.1 TB/s), 32 rows of 100 to 4000 41 -> 33, one row of 8000 22 -> 14;
+// 8 rows of 1000 to 3600 17.4 -> 15.0, of which the two launches and their chains of
 // round trips (lengths, tiles, parts) are 9.
 // ---------------------------------------------------------------------------
 constexpr int kDecKeys = 32;  // keys per wave tile
@@ -525,8 +528,8 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
   return x;
 }
 
-// The line of key tiles, in units of kShareUnit tiles, as one wave sees it: 64 batch
-// rows at a time, one per lane.
+// The line of key tiles (of one kv head; they are alike), in units of kShareUnit, as
+// one wave sees it: 64 batch rows at a time, one per lane.
 struct TileLine {
   int first;  // batch row of lane 0
   int pos;    // position of the lane's batch row: cache_lengths clamped to [-S, L] (new row i goes to pos + i)
@@ -593,12 +596,28 @@ struct LineChunks {
   }
 };
 
-// Units per share for a line of `total` units.
-__device__ __forceinline__ int share_of(const CacheArgs& a, int total) {
-  return max(1, (total + a.shares - 1) / a.shares);
-}
-// Part slot (of two per share) of the segment that starts at position u of the line.
-__device__ __forceinline__ int part_slot(int u, int per) { return 2 * (u / per) + (u % per != 0); }
+// The line's units dealt to the shares: q each, and one more to the first r.  A share is
+// a run of the line for each kv head, one workgroup per head, so that the heads of a
+// batch row, whose keys are adjacent in memory, stream the same positions at the same
+// time.  (With the heads' lines one after another, a share somewhere in one of them, 128
+// bytes of each key at a time, 64 rows of 0 to 2500 keys, 8 / 8 heads of 64, took 43.7 us, 38.0
+// with a workgroup for each pair and key split, which starts the heads together; so
+// 34.7.  Of 0 to 3780 54.8 -> 54.5 and 59.7 -> 49.1, of equal length 2000 53.8 -> 45.4; 64 of 500
+// to 8000, 16 / 4 heads of 128, 119.4 -> 116.7.)  In whole units, the last shares empty, 24 rows
+// of 500 to 2500, 8 / 8 heads of 64, 22.7 us instead of 21.1, 64 of 500 to 8000 118.6 instead of
+// 116.7; but one row of 120000, 4 kv heads of 128, 51.5 instead of 53.0.
+struct Shares {
+  int q, r;
+  __device__ __forceinline__ Shares(const CacheArgs& a, int total) : q(total / a.shares), r(total - q * a.shares) {}
+  __device__ __forceinline__ int begin(int share) const { return share * q + min(share, r); }
+  // the share that unit u < total lies in
+  __device__ __forceinline__ int of(int u) const {
+    const int longer = r * (q + 1);  // units of the first r shares, all of them if q is 0
+    return u < longer ? u / (q + 1) : r + (u - longer) / q;
+  }
+};
+// Part slot (of two per share) of a segment: the one the share begins with, or a later one.
+__device__ __forceinline__ int part_slot(int share, bool first) { return 2 * share + !first; }
 
 // Zero output for `heads` heads from h0 on of batch row b.
 template <int D>
@@ -652,13 +671,13 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   // This share [u_begin, u_end) of the line, and the first batch row it touches: lane j
   // of the loaded rows.  One workgroup per pair: its batch row, and no line.
   TileLine line;
-  int j, u_begin = 0, u_end = 1, per = 1;
+  const int share = blockIdx.x / a.Hkv, hk = blockIdx.x - share * a.Hkv;  // share: the batch row, for pairs
+  int j, u_begin = 0, u_end = 1;
   if constexpr (kPairs) {
-    const int pair_b = blockIdx.x / a.Hkv;
-    line.load(a, pair_b & ~63, 0, lane);
-    j = pair_b & 63;
+    line.load(a, share & ~63, 0, lane);
+    j = share & 63;
     if (__builtin_amdgcn_readlane(line.keys, j) == 0) {
-      zero_rows<D>(a, pair_b, blockIdx.x % a.Hkv * a.G, a.G);
+      zero_rows<D>(a, share, hk * a.G, a.G);
       return;
     }
   } else {
@@ -672,15 +691,15 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
       chunks.scan(a, lane, [&](const TileLine& l) { zero_keyless<D>(a, l, lane); });
       total = chunks.total();
     }
-    per = share_of(a, total * a.Hkv);
-    u_begin = (int)blockIdx.x * per;
-    u_end = min(total * a.Hkv, u_begin + per);
+    const Shares shares(a, total);
+    u_begin = shares.begin(share);
+    u_end = shares.begin(share + 1);
     if (u_begin >= u_end) return;
     if (a.B > 64) {
-      const int c = __builtin_ctzll(__builtin_amdgcn_ballot_w64(chunks.incl * a.Hkv > u_begin));
+      const int c = __builtin_ctzll(__builtin_amdgcn_ballot_w64(chunks.incl > u_begin));
       line.load(a, 64 * c, chunks.before(c), lane);
     }
-    j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl * a.Hkv > u_begin));
+    j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl > u_begin));
   }
 
   const int R = a.S * a.G;  // <= kDecRows
@@ -722,7 +741,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   // first at position u0 of the line.
   const int ck_st = (int)a.ck_st, cv_st = (int)a.cv_st;  // a span check bounds them
   int u0 = u_begin;
-  int b, hk, kv, pos_b, crow, t0, n_my, kend_lane, kend_min, u_next, u_row;  // u_row: where the next batch row begins
+  int b, kv, pos_b, crow, t0, n_my, kend_lane, kend_min, u_next;
   bool whole;
   int new_lo, new_hi;  // positions [new_lo, new_hi) may hold new rows
   bf16_t *kbase, *vbase;
@@ -795,19 +814,15 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
     crow = __builtin_amdgcn_readlane(line.row, j);
     int t_end = (kv + kDecKeys - 1) / kDecKeys;
     if constexpr (kPairs) {
-      hk = blockIdx.x - b * c.Hkv;
       whole = true;
       u_next = u_end;
       t0 = 0;
     } else {
       const int units_b = __builtin_amdgcn_readlane(line.units, j);
-      const int base = (__builtin_amdgcn_readlane(line.incl, j) - units_b) * c.Hkv;
-      hk = (u0 - base) / units_b;
-      const int unit0 = (u0 - base) - hk * units_b;
+      const int unit0 = u0 - (__builtin_amdgcn_readlane(line.incl, j) - units_b);
       const int unit1 = min(units_b, unit0 + u_end - u0);
       whole = unit0 == 0 && unit1 == units_b;
       u_next = u0 + unit1 - unit0;
-      u_row = base + units_b * c.Hkv;
       t0 = unit0 * kShareUnit;
       t_end = min(unit1 * kShareUnit, t_end);
     }
@@ -930,17 +945,15 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
     // The next segment's first copies go out before this one's merge (this wave's
     // reads of its stages are done; the merge uses the second ones), so that a share
     // of several short segments does not pay a memory round trip for each.
-    const int cur_b = b, cur_hk = hk;
+    const int cur_b = b;
     const bool cur_whole = whole;
-    const int64_t slot = (int64_t)part_slot(u0, per) * R;
+    const int64_t slot = ((int64_t)part_slot(share, u0 == u_begin) * a.Hkv + hk) * R;
     const bool more = u_next < u_end;
     wait_lds();
     if (more) {
-      u0 = u_next;
-      if (u0 == u_row) {  // the next batch row with keys
-        while (line.end() * a.Hkv <= u0) line.load(a, line.first + 64, line.end(), lane);
-        j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl * a.Hkv > u0));
-      }
+      u0 = u_next;  // the next batch row with keys
+      while (line.end() <= u0) line.load(a, line.first + 64, line.end(), lane);
+      j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl > u0));
       begin();
     }
     // Merge the waves' partial rows through LDS.
@@ -987,7 +1000,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
       if (cur_whole) {
         const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
         const int ti_r = rr / a.G;
-        const int h_r = cur_hk * a.G + (rr - ti_r * a.G);
+        const int h_r = hk * a.G + (rr - ti_r * a.G);
         bf16_t* orow = c.out + (int64_t)cur_b * c.o_sb + (int64_t)ti_r * c.o_st + (int64_t)h_r * c.o_sh;
         *(bf16x4*)&orow[dcol] = __builtin_convertvector(acc * inv, bf16x4);
       } else {
@@ -1025,8 +1038,8 @@ __device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
   const int R = a.S * a.G;
   const int groups = (R + kWaves - 1) / kWaves;  // workgroups per pair
   const int rr = blockIdx.x % groups * kWaves + wave;
-  const int hk = blockIdx.x / groups % a.Hkv;
-  const int b = blockIdx.x / groups / a.Hkv;
+  const int pair = blockIdx.x / groups;
+  const int b = pair / a.Hkv, hk = pair - b * a.Hkv;
   TileLine line;
   int total;
   if (a.B <= 64) {
@@ -1040,12 +1053,13 @@ __device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
   }
   const int units_b = __builtin_amdgcn_readlane(line.units, b & 63);
   const int before = __builtin_amdgcn_readlane(line.incl, b & 63) - units_b;
-  const int per = share_of(a, total * a.Hkv);
-  const int g0 = before * a.Hkv + hk * units_b;  // the pair's units [g0, g0 + units_b) of the line
-  const int w0 = g0 / per, n = units_b > 0 ? (g0 + units_b - 1) / per - w0 + 1 : 0;  // shares it lies in
-  if (n <= 1 || rr >= R) return;  // written by its share
+  const Shares shares(a, total);
+  if (units_b == 0 || rr >= R) return;
+  const int w0 = shares.of(before), n = shares.of(before + units_b - 1) - w0 + 1;  // shares it lies in
+  if (n == 1) return;  // written by its share
+  const int slot0 = part_slot(w0, before == shares.begin(w0));
   const int t = rr / a.G;
-  merge_row<D>(a, n, lane, [&](int c) { return part_slot(c == 0 ? g0 : (w0 + c) * per, per) * R + rr; },
+  merge_row<D>(a, n, lane, [&](int c) { return ((c == 0 ? slot0 : part_slot(w0 + c, true)) * a.Hkv + hk) * R + rr; },
                a.out + (int64_t)b * a.o_sb + (int64_t)t * a.o_st + (int64_t)(hk * a.G + rr - t * a.G) * a.o_sh);
 }
 __global__ __launch_bounds__(kThreads) void cache_merge_d128_kernel(const CacheArgs a) { cache_merge_body<128>(a); }
@@ -1062,7 +1076,7 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
   CacheSplit s = {};
   const int G = p.num_kv_heads > 0 ? p.num_q_heads / p.num_kv_heads : 1;
   const int64_t R = (int64_t)p.seqlen * G;
-  s.decode = R <= kDecRows;  // the decode kernels: 32-key wave tiles, one workgroup per CU
+  s.decode = R <= kDecRows;  // the decode kernels: 32-key wave tiles
   s.n_rt = (int)((R + kRows - 1) / kRows);
   int max_kv = p.max_kv_len < p.cache_len ? p.max_kv_len : p.cache_len;
   if (max_kv < 1) max_kv = 1;
@@ -1080,14 +1094,14 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
     if (s.pairs) {  // one workgroup per pair
       s.units = s.groups;
     } else {
-      // Two shares of the line per CU (head_dim 64: three, which its LDS allows and its
-      // copies of half the bytes need), or one per unit if there cannot be as many; two part
-      // slots per share: partial O, then (max, sum) rows.  Three against two, 8 / 8 heads of
-      // 64: 32 rows of 100 to 3200 keys 32.5 -> 27.8 us, 8 of 1000 to 3100 15.1 -> 13.3, 64 of
-      // 0 to 3780 57.0 -> 54.1; 64 of 512 to 7440 106 -> 111, 8 / 2 heads 29.6 -> 30.8.
-      const int64_t most = s.groups * ((tiles + kShareUnit - 1) / kShareUnit),
-                    shares = (p.head_dim == 64 ? 3 : 2) * (int64_t)device_cu_count();
-      s.units = most < shares ? most : shares;
+      // Two workgroups per CU, or one per unit and kv head if there cannot be as many (head_dim
+      // 64: if those are at most four per CU, which its LDS allows: 16 rows of 10 to 4000 keys,
+      // 8 / 2 heads, 13.2 -> 11.8 us); two part slots each: partial O, then (max, sum) rows.
+      const int64_t cus = device_cu_count(), most = (int64_t)p.batch * ((tiles + kShareUnit - 1) / kShareUnit);
+      int64_t shares = 2 * cus / p.num_kv_heads;
+      if (shares < 1) shares = 1;
+      if (p.head_dim == 64 && most * p.num_kv_heads <= 4 * cus) shares = most;
+      s.units = p.num_kv_heads * (most < shares ? most : shares);
       s.workspace_bytes = (size_t)s.units * 2 * (size_t)R * ((size_t)p.head_dim + 2) * sizeof(float);
     }
     s.splits = 1;
@@ -1150,7 +1164,7 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   if (e != hipSuccess || sp.units == 0) return e;
   if (sp.decode) {
     const int64_t rows = (int64_t)a.S * a.G;
-    a.shares = (int)sp.units;
+    a.shares = (int)(sp.units / a.Hkv);
     a.part_ml = a.part_o + (size_t)sp.units * 2 * rows * p.head_dim;
     const dim3 grid((unsigned)sp.units);
     if (sp.pairs) {

@@ -214,7 +214,7 @@ __device__ __forceinline__ void stage_owned(float* dst, const float* base, int64
 //   D  96: 1.4 3.6 3.6 / 0.91 2.7 2.8 / 0.85 2.7 2.7    D 128: 1.6 4.0 4.0 / 0.91 2.8 3.0 / 0.87 2.7 2.7
 // The additions and their waits for the products cost, with one chain / so: forward +
 // backward of 8192 tokens in documents of 2048, 8 heads, D 64 0.95 / 0.99 ms, of 4096, 16 / 4
-// heads, D 128 2.75 / 3.04 (15.8 on the vector ALUs); 4 x 512, 8 heads, D 64 unchanged.
+// heads, D 128 2.75 / 2.96 (15.8 on the vector ALUs).
 template <int D>
 constexpr int kScoreChain = D == 32 ? 2 : D == 128 ? 8 : 4;
 template <int D>

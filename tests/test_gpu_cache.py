@@ -67,6 +67,10 @@ def test_short_chunks_around_the_decode_kernel(device, S, causal):
     (6, 17, 2, 2, 64, 900, 7),      # 17 query rows, several pairs per share
     (40, 3, 10, 2, 128, 300, 8),    # 15 query rows, one workgroup per pair
     (33, 32, 3, 3, 64, 260, 9),
+    (3, 1, 24, 24, 64, 1500, 10),   # a run of the line for each of 24 kv heads
+    (2, 1, 300, 300, 64, 600, 11),  # more kv heads than there are CUs: one run for each
+    (9, 1, 6, 3, 128, 2000, 12),    # 3 kv heads: their runs leave two workgroups out
+    (20, 1, 2, 2, 64, 2500, 13),    # head_dim 64: one unit for each run, or none
 ])
 def test_decode_work_split(device, B, S, hq, hkv, d, L, seed):
     """One workgroup per pair, and the line of key tiles dealt to equal shares: ragged lengths
