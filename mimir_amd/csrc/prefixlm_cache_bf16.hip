@@ -93,11 +93,10 @@ __global__ __launch_bounds__(256) void cache_append_kernel(const CacheArgs a) {
 // out = sum_c O_c 2^(m_c - M) / sum_c l_c 2^(m_c - M).  One wave: lane c takes part
 // c's (max, sum), and the O rows are read one part per D / 4 lanes with kChunk
 // loads in flight beside it, so up to 32 parts (D 128) cost one memory round trip.
-template <int D, typename Slot>
+template <int D, int kChunk = 16, typename Slot>
 __device__ __forceinline__ void merge_row(const CacheArgs& a, int n, int lane, Slot&& slot, bf16_t* orow) {
   constexpr int kLanes = D / 4;        // lanes per part row, four columns each
   constexpr int kParts = 64 / kLanes;  // part rows per load
-  constexpr int kChunk = 16;
   const int sub = lane / kLanes, col = lane % kLanes * 4;
   float M = -INFINITY, lsum = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};  // this lane's columns over the parts of its lane group
@@ -1031,7 +1030,7 @@ __global__ __launch_bounds__(kPairWaves * 64, 1) void cache_decode_pairs_d64_ker
 
 // Output rows of the (batch row, kv head) pairs whose key tiles lie in several
 // shares, one wave per row, from the parts in the order of the line.
-template <int D>
+template <int D, int kChunk>
 __device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1059,11 +1058,20 @@ __device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
   if (n == 1) return;  // written by its share
   const int slot0 = part_slot(w0, before == shares.begin(w0));
   const int t = rr / a.G;
-  merge_row<D>(a, n, lane, [&](int c) { return ((c == 0 ? slot0 : part_slot(w0 + c, true)) * a.Hkv + hk) * R + rr; },
+  merge_row<D, kChunk>(a, n, lane, [&](int c) { return ((c == 0 ? slot0 : part_slot(w0 + c, true)) * a.Hkv + hk) * R + rr; },
                a.out + (int64_t)b * a.o_sb + (int64_t)t * a.o_st + (int64_t)(hk * a.G + rr - t * a.G) * a.o_sh);
 }
-__global__ __launch_bounds__(kThreads) void cache_merge_d128_kernel(const CacheArgs a) { cache_merge_body<128>(a); }
-__global__ __launch_bounds__(kThreads) void cache_merge_d64_kernel(const CacheArgs a) { cache_merge_body<64>(a); }
+__global__ __launch_bounds__(kThreads) void cache_merge_d128_kernel(const CacheArgs a) { cache_merge_body<128, 16>(a); }
+__global__ __launch_bounds__(kThreads) void cache_merge_d64_kernel(const CacheArgs a) { cache_merge_body<64, 16>(a); }
+// For more than 16 query rows per kv head: many more waves than the chip holds, and few
+// parts for each; with fewer loads in flight (and registers) per wave twice as many fit
+// (256 pairs of 32 rows, head_dim 64: the two launches 32.4 -> 30.7 us).
+__global__ __launch_bounds__(kThreads, 8) void cache_merge_rows_d128_kernel(const CacheArgs a) {
+  cache_merge_body<128, 4>(a);
+}
+__global__ __launch_bounds__(kThreads, 8) void cache_merge_rows_d64_kernel(const CacheArgs a) {
+  cache_merge_body<64, 4>(a);
+}
 
 unsigned grid_for(int64_t items) {
   const int64_t blocks = (items + 255) / 256;
@@ -1088,9 +1096,12 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
     // for any batch (two rounds of copies) up to 2048 for a pair per CU.  64 x 4
     // pairs (one launch against two, no merge): 100 to 1000 keys 25.5 -> 19.0 us, 100
     // to 2000 keys 37.5 / 37.9, 100 to 4000 keys 65 / 72 (the longest pair runs alone).
-    // And for a batch past kLineRows, where a share would look for its pairs too long.
+    // And for a batch past kLineRows, where a share would look for its pairs too long, and
+    // for more than 16 query rows if the pairs fill the chip twice: then the parts of the
+    // cut pairs are much of what there is to move (64 rows of 100 to 3000 keys, 8 / 8 heads
+    // of 64, 32 query rows: 53 us, 62 dealt evenly, 57 with equal splits per pair).
     const int64_t pair_keys = 8 * s.groups;
-    s.pairs = p.batch > kLineRows || max_kv <= (pair_keys < 256 ? 256 : (pair_keys < 2048 ? pair_keys : 2048));
+    s.pairs = p.batch > kLineRows || (R > 16 && s.groups >= 2 * (int64_t)device_cu_count()) || max_kv <= (pair_keys < 256 ? 256 : (pair_keys < 2048 ? pair_keys : 2048));
     if (s.pairs) {  // one workgroup per pair
       s.units = s.groups;
     } else {
@@ -1177,10 +1188,12 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
     const dim3 merge((unsigned)(sp.groups * ((rows + kWaves - 1) / kWaves)));
     if (p.head_dim == 128) {
       hipLaunchKernelGGL(cache_decode_d128_kernel, grid, dim3(kShareWaves * 64), 0, stream, a);
-      hipLaunchKernelGGL(cache_merge_d128_kernel, merge, dim3(kThreads), 0, stream, a);
+      hipLaunchKernelGGL(rows > 16 ? cache_merge_rows_d128_kernel : cache_merge_d128_kernel, merge, dim3(kThreads), 0,
+                         stream, a);
     } else {
       hipLaunchKernelGGL(cache_decode_d64_kernel, grid, dim3(kShareWaves * 64), 0, stream, a);
-      hipLaunchKernelGGL(cache_merge_d64_kernel, merge, dim3(kThreads), 0, stream, a);
+      hipLaunchKernelGGL(rows > 16 ? cache_merge_rows_d64_kernel : cache_merge_d64_kernel, merge, dim3(kThreads), 0,
+                         stream, a);
     }
     return hipGetLastError();
   }

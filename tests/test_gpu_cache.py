@@ -71,6 +71,9 @@ def test_short_chunks_around_the_decode_kernel(device, S, causal):
     (2, 1, 300, 300, 64, 600, 11),  # more kv heads than there are CUs: one run for each
     (9, 1, 6, 3, 128, 2000, 12),    # 3 kv heads: their runs leave two workgroups out
     (20, 1, 2, 2, 64, 2500, 13),    # head_dim 64: one unit for each run, or none
+    (3, 9, 6, 3, 128, 2200, 14),    # 18 query rows: parts merged a few loads at a time, many of them
+    (1, 32, 1, 1, 64, 9000, 15),
+    (130, 20, 4, 4, 64, 600, 16),   # 20 query rows and a workgroup per pair
 ])
 def test_decode_work_split(device, B, S, hq, hkv, d, L, seed):
     """One workgroup per pair, and the line of key tiles dealt to equal shares: ragged lengths
