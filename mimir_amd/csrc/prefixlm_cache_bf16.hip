@@ -160,7 +160,19 @@ __device__ __forceinline__ RowSplit row_split(const CacheArgs& a, int keys) {
   return r;
 }
 
-template <int D>
+// Whether the batch rows (at most 64) hold about as many cached keys: none differs from the
+// first by more than an eighth of the chunk.
+__device__ __forceinline__ bool even_lengths(const CacheArgs& a) {
+  if (a.B > 64) return false;
+  const int n = cache_len_of(a, min((int)threadIdx.x & 63, a.B - 1));
+  const int64_t off = n - __builtin_amdgcn_readfirstlane(n);
+  return __builtin_amdgcn_ballot_w64(8 * (off < 0 ? -off : off) > a.S) == 0;
+}
+
+// kAppend: the kernel reads the chunk's keys in place and appends them; without it they
+// are in the cache already.  (One kernel for both: what the first needs, sixteen registers
+// among it, slowed the second by 1 to 2%.)
+template <int D, bool kAppend>
 __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs a) {
   constexpr int DT = D / 32;
   constexpr int KS = D / 16;
@@ -176,18 +188,29 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
   const int l32 = lane & 31;
   const int hi = lane >> 5;
 
-  int u = blockIdx.x;
-  const int split = u % a.splits;
-  u /= a.splits;
-  int rt = u % a.n_rt;
-  u /= a.n_rt;
-  // Later row tiles of a causal chunk see more keys.  Workgroups b and b + (CUs) share a
-  // CU, and with the row tiles in the same order in every pair they were the same row
-  // tile of two pairs (n_rt a power of two): some CUs got two long ones.  Every other
-  // CU-sized run of pairs takes its row tiles in reverse: 8 x 512 on 1536 keys 76.8 ->
-  // 74.4 us, 8 x 512 on none 28.6 -> 25.2, 8 x 1024 on none 74.3 -> 68.0 (16 / 4 heads,
-  // head_dim 128), 8 x 1024 on 1536 64 -> 59 (8 / 8 heads of 64); split ranges unchanged.
-  if (u * a.n_rt * a.splits / a.cus % 2 == 1) rt = a.n_rt - 1 - rt;
+  // Later row tiles of a causal chunk see more keys, and workgroups b and b + (CUs) share a
+  // CU.  Where the row tile decides (an unsplit chunk on rows of about the same length), the
+  // workgroups take them by rank, the latest first over all pairs, and every other CU-sized
+  // run backwards: a CU's two are then a long and a short one, and what is left over at the
+  // end is short.  Against the row tiles of a pair in a row: 8 x 512 on 1536 keys 76.0 -> 68.0
+  // us, 8 x 1024 on none 74.4 -> 56.4, 8 x 2048 on none 193 -> 142 (16 / 4 heads of 128), 12 x 700
+  // on none 31.0 -> 25.2, 8 x 1024 on 1536 66.7 -> 52 (8 / 8 heads of 64); on rows of 100 to 2200
+  // keys 8 x 300 would go from 98.9 to 107.  With the key range split, the runs of pairs alone
+  // alternate (33 on 300 keys 15.1 -> 13.7, 8 x 139 on 60 to 145 25.2 -> 23.6).  Unsplit, that
+  // alternation took the row tiles of some pairs the wrong way round: 12 x 700 on none 32.7.
+  int u = blockIdx.x, split = 0, rt;
+  if (a.splits == 1 && a.causal && even_lengths(a)) {
+    const int run = u / a.cus, pairs = gridDim.x / a.n_rt;
+    if (run % 2 == 1 && (run + 1) * a.cus <= (int)gridDim.x) u = (2 * run + 1) * a.cus - 1 - u;
+    rt = a.n_rt - 1 - u / pairs;
+    u %= pairs;
+  } else {
+    split = u % a.splits;
+    u /= a.splits;
+    rt = u % a.n_rt;
+    u /= a.n_rt;
+    if (a.splits > 1 && u * a.n_rt * a.splits / a.cus % 2 == 1) rt = a.n_rt - 1 - rt;
+  }
   const int hk = u % a.Hkv;
   const int b = u / a.Hkv;
 
@@ -233,9 +256,9 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
   // 16 / 4 heads, head_dim 128, against the append launch: 8 x 512 on 1536 keys 81 ->
   // 78 us, 8 x 100 on 100 to 3000 46 -> 42, 100 on 3000 27 -> 24.5; 8 x 1024 on 1536,
   // 8 / 8 heads of 64, 68 -> 65.
-  const int64_t pos_raw = load_index(a.cache_lengths, b, a.idx64);
+  const int64_t pos_raw = kAppend ? load_index(a.cache_lengths, b, a.idx64) : 0;
   const int pos = pos_raw < -(int64_t)a.S ? -a.S : (pos_raw > a.L ? a.L : (int)pos_raw);
-  const int new_lo = a.append ? max(pos, 0) : 0x7fffffff, new_hi = min(pos + a.S, kv);
+  const int new_lo = max(pos, 0), new_hi = min(pos + a.S, kv);
   const bf16_t* knb = a.kn + (int64_t)b * a.kn_sb + (int64_t)hk * a.kn_sh;
   const bf16_t* vnb = a.vn + (int64_t)b * a.vn_sb + (int64_t)hk * a.vn_sh;
   // Both kinds in one tile: every lane takes its 16 bytes from the row's own place
@@ -259,6 +282,11 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
   };
   auto issue = [&](int kt, bf16_t* tk, bf16_t* tv) __attribute__((always_inline)) {
     const int kb = kt * kKeys;
+    if constexpr (!kAppend) {
+      ldk.issue_at(kbase + (int64_t)kb * a.ck_st, rows_bytes32(kv - kb, (uint32_t)a.ck_st, D), tk);
+      ldv.issue_at(vbase + (int64_t)kb * a.cv_st, rows_bytes32(kv - kb, (uint32_t)a.cv_st, D), tv);
+      return;
+    }
     const bool some = kb + kKeys > new_lo && kb < new_hi;
     if (some && (kb < new_lo || new_hi < min(kb + kKeys, kv))) {
       issue_mixed(kb, tk, tv);
@@ -358,7 +386,7 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
 
   // The new tokens whose first row lies in this row tile go into the cache here (no
   // workgroup reads these cache rows).
-  if (a.append && split == 0 && row_in_cache) {
+  if (kAppend && split == 0 && row_in_cache) {
     constexpr int kUnits = D / 8;
     const int first = max((rt * kRows + a.G - 1) / a.G, -pos);
     const int last = min(((rt + 1) * kRows + a.G - 1) / a.G, min(a.S, a.L - pos));
@@ -415,6 +443,12 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
     }
   if (hi == 0) *(f32x2*)&a.part_ml[slot * 2] = f32x2{m_run == -INFINITY ? -INFINITY : m_run * c2, l_tot};
 }
+
+// By name: of several instantiations launched below, this toolchain drops host stubs.
+template __global__ void cache_attn_kernel<128, true>(const CacheArgs);
+template __global__ void cache_attn_kernel<128, false>(const CacheArgs);
+template __global__ void cache_attn_kernel<64, true>(const CacheArgs);
+template __global__ void cache_attn_kernel<64, false>(const CacheArgs);
 
 // Adds the partial rows of cache_attn_kernel's key splits, one wave per query row.
 // In the last split to arrive, four waves took the up to 128 rows of a tile in
@@ -1199,10 +1233,15 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   }
   a.part_ml = a.part_o + (size_t)sp.units * kRows * p.head_dim;
   a.cus = device_cu_count();
-  if (p.head_dim == 128)
-    hipLaunchKernelGGL(cache_attn_kernel<128>, dim3((unsigned)sp.units), dim3(kThreads), 0, stream, a);
+  const dim3 grid((unsigned)sp.units);
+  if (p.head_dim == 128 && a.append)
+    hipLaunchKernelGGL((cache_attn_kernel<128, true>), grid, dim3(kThreads), 0, stream, a);
+  else if (p.head_dim == 128)
+    hipLaunchKernelGGL((cache_attn_kernel<128, false>), grid, dim3(kThreads), 0, stream, a);
+  else if (a.append)
+    hipLaunchKernelGGL((cache_attn_kernel<64, true>), grid, dim3(kThreads), 0, stream, a);
   else
-    hipLaunchKernelGGL(cache_attn_kernel<64>, dim3((unsigned)sp.units), dim3(kThreads), 0, stream, a);
+    hipLaunchKernelGGL((cache_attn_kernel<64, false>), grid, dim3(kThreads), 0, stream, a);
   if (sp.splits > 1) {
     const int64_t rows = (int64_t)a.S * a.G;
     const dim3 merge((unsigned)((int64_t)a.B * a.Hkv * ((rows + kWaves - 1) / kWaves)));

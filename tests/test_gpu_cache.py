@@ -68,7 +68,7 @@ def test_short_chunks_around_the_decode_kernel(device, S, causal):
     (40, 3, 10, 2, 128, 300, 8),    # 15 query rows, one workgroup per pair
     (33, 32, 3, 3, 64, 260, 9),
     (3, 1, 24, 24, 64, 1500, 10),   # a run of the line for each of 24 kv heads
-    (2, 1, 300, 300, 64, 600, 11),  # more kv heads than there are CUs: one run for each
+    (2, 1, 300, 300, 64, 2100, 11), # more kv heads than there are CUs: one run for each
     (9, 1, 6, 3, 128, 2000, 12),    # 3 kv heads: their runs leave two workgroups out
     (20, 1, 2, 2, 64, 2500, 13),    # head_dim 64: one unit for each run, or none
     (3, 9, 6, 3, 128, 2200, 14),    # 18 query rows: parts merged a few loads at a time, many of them
@@ -248,6 +248,20 @@ def test_prefill_reads_the_new_rows_in_place(device, S, hq, hkv, d, lens):
     lens = (lens * B)[:B]
     _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=True, seed=S)
     _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=L, lens=lens, causal=False, seed=S + 1)
+
+
+@pytest.mark.parametrize("B,S,hq,hkv,d,lens", [
+    (24, 700, 4, 4, 64, [0, 87]),         # 576 row tiles: more than two to a CU, about equal lengths
+    (24, 700, 4, 4, 64, [0, 88]),         # lengths too far apart for the order by rank
+    (33, 520, 6, 6, 64, [11, 0, 65]),     # 990: an odd run of CUs cut short
+    (13, 300, 32, 8, 128, [100]),         # 1040, grouped heads: 1200 rows in ten row tiles
+    (70, 200, 2, 2, 64, [50]),            # more batch rows than lanes
+])
+def test_prefill_order_of_the_row_tiles(device, B, S, hq, hkv, d, lens):
+    """Unsplit chunks on rows of about equal length are dealt by rank, others as they come."""
+    lens = (lens * B)[:B]
+    for causal, rows in ((True, None), (True, list(range(B))[::-1]), (False, None)):
+        _run(device, B=B, S=S, hq=hq, hkv=hkv, d=d, L=max(lens) + S, lens=lens, causal=causal, rows=rows, seed=B)
 
 
 @pytest.mark.parametrize("S,hq,hkv,d,lens", [
