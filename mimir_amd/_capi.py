@@ -13,7 +13,9 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sys
 import threading
+import warnings
 from pathlib import Path
 
 # MIMIR_PREFIXLM_LIB overrides the in-tree library (e.g. to A/B two builds).
@@ -199,28 +201,59 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+class _GeneralPath:
+    """In place of the native host calls: serves none, so that every call takes the general path."""
+
+    @staticmethod
+    def fwd(*args):
+        return None
+
+    bwd = rope = cache_attn = fwd
+
+
+def _load_host():
+    """The module of the native host calls, or None (with a warning) if there is none that fits."""
+    import torch
+
+    if not HOST_PATH.exists():
+        why = f"{HOST_PATH} is not built"
+    else:
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("_host_calls", str(HOST_PATH))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host_calls", loader))
+            loader.exec_module(module)
+            # compiled against the C++ interfaces of one torch and one Python
+            here = f"torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]}"
+            if module.built_for == here:
+                return module
+            why = f"{HOST_PATH} is built for {module.built_for}, not {here}"
+        except (ImportError, AttributeError) as e:
+            why = f"{HOST_PATH} does not load: {e}"
+    warnings.warn(f"mimir_amd: {why}; calls take the general path (10 to 30 us more host time each). "
+                  "Build it with `python -m mimir_amd.build`", RuntimeWarning, stacklevel=3)
+    return None
+
+
 _host = None
 
 
 def host():
-    """The native host calls (csrc/host_calls.cpp), bound to the library; ImportError if not built.
+    """The native host calls (csrc/host_calls.cpp), bound to the library.
 
     ``fwd`` / ``bwd`` / ``rope`` / ``cache_attn`` check, allocate and launch a
-    well-formed call and return None for any other, which then takes the general path."""
+    well-formed call and return None for any other, which then takes the general path.
+    Where the module is not built, or built for another torch or Python, they serve
+    no call.  ImportError if the library itself is not built."""
     global _host
     if _host is not None:
         return _host
     load()
     with _lock:
         if _host is None:
-            if not HOST_PATH.exists():
-                raise ImportError(f"mimir_amd prefix-LM attention requires {HOST_PATH}; "
-                                  "build it with `python -m mimir_amd.build`")
-            loader = importlib.machinery.ExtensionFileLoader("_host_calls", str(HOST_PATH))
-            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_host_calls", loader))
-            loader.exec_module(module)
-            module.bind(str(LIB_PATH))
-            _host = module
+            module = _load_host()
+            if module is not None:
+                module.bind(str(LIB_PATH))
+            _host = module or _GeneralPath
     return _host
 
 

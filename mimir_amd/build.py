@@ -4,8 +4,9 @@ Every HIP source under ``mimir_amd/csrc`` is compiled with hipcc for
 ``--offload-arch=gfx950`` and linked into ``mimir_amd/_lib/libmimir_prefixlm.so``.
 No torch extension machinery is involved: the library exports only the
 ``extern "C"`` entry points declared in ``include/mimir_prefixlm.h`` and is loaded
-with ctypes.  ``csrc/host_calls.cpp`` (no device code; torch's C++ headers) becomes
-``mimir_amd/_lib/_host_calls.so``, the Python module that makes the common calls.  Run ``python -m mimir_amd.build`` (or ``__graft_entry__.build()``).
+with ctypes.  ``csrc/host_calls.cpp`` (no device code; g++ and torch's C++ headers) becomes
+``mimir_amd/_lib/_host_calls.so``, the Python module that makes the common calls; the package
+works without it.  Run ``python -m mimir_amd.build`` (or ``__graft_entry__.build()``).
 """
 
 from __future__ import annotations
@@ -79,7 +80,10 @@ def _compile(src: Path, obj: Path) -> None:
 
 
 def _build_host() -> None:
-    """Compile the native host calls against the running Python and torch."""
+    """Compile the native host calls against the running Python and torch.
+
+    They only shorten calls that the general path in Python makes as well, so a
+    machine without a C++ compiler or Python's headers still gets the library."""
     import sysconfig
 
     import torch
@@ -87,14 +91,21 @@ def _build_host() -> None:
 
     libs = Path(torch.__file__).resolve().parent / "lib"
     tmp = HOST_PATH.with_suffix(".so.tmp")
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *(x for p in include_paths() for x in ("-isystem", p)), f"-I{sysconfig.get_paths()['include']}",
-           str(HOST_SOURCE), "-o", str(tmp), f"-L{libs}", f"-Wl,-rpath,{libs}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"compiling {HOST_SOURCE.name} failed:\n{res.stderr}")
-    os.replace(tmp, HOST_PATH)
+    args = ["-O2", "-std=c++17", "-fPIC", "-shared",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DMIMIR_BUILT_FOR="torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]}"',
+            *(x for p in include_paths() for x in ("-isystem", p)), f"-I{sysconfig.get_paths()['include']}",
+            str(HOST_SOURCE), "-o", str(tmp), f"-L{libs}", f"-Wl,-rpath,{libs}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    try:
+        res = subprocess.run([os.environ.get("CXX", "g++"), *args], capture_output=True, text=True)
+        error = res.stderr if res.returncode != 0 else ""
+    except OSError as e:
+        error = str(e)
+    if error:
+        HOST_PATH.unlink(missing_ok=True)  # not one of other sources
+        print(f"warning: {HOST_SOURCE.name} was not compiled, calls will take the general path:\n{error}", file=sys.stderr)
+    else:
+        os.replace(tmp, HOST_PATH)
 
 
 def build(verbose: bool = True) -> Path:

@@ -408,4 +408,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_calls() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host_calls() {
+  PyObject* m = PyModule_Create(&module);
+  if (m != nullptr) PyModule_AddStringConstant(m, "built_for", MIMIR_BUILT_FOR);
+  return m;
+}

@@ -109,3 +109,37 @@ def test_tensors_of_another_device_take_the_general_path(bound):
     ctypes.c_int.in_dll(stub, "stub_status").value = _capi.OK
     x, cos = torch.zeros(5, 2, 64, device="meta"), torch.zeros(5, 64, device="meta")
     assert host.rope(x, cos, cos, False, None, 0) is None
+
+
+@pytest.mark.parametrize("form", ["missing", "another torch", "not a module"])
+def test_without_the_native_calls_the_general_path_runs(monkeypatch, tmp_path, form):
+    monkeypatch.setattr(_capi, "_host", None)
+    if form == "missing":
+        monkeypatch.setattr(_capi, "HOST_PATH", tmp_path / "_host_calls.so")
+    elif form == "another torch":
+        monkeypatch.setattr(torch, "__version__", "1.0")
+    else:
+        (tmp_path / "_host_calls.so").write_bytes(b"no shared object")
+        monkeypatch.setattr(_capi, "HOST_PATH", tmp_path / "_host_calls.so")
+    with pytest.warns(RuntimeWarning, match="general path"):
+        host = _capi.host()
+    assert host.fwd(1) is host.bwd(1) is host.rope(1) is host.cache_attn(1) is None
+    assert _capi.host() is host  # and without another warning
+
+
+def test_the_built_module_fits(monkeypatch):
+    if not _capi.HOST_PATH.exists():
+        pytest.skip("the native host calls are not built")
+    monkeypatch.setattr(_capi, "_host", None)
+    assert _capi.host() is not _capi._GeneralPath
+
+
+def test_build_without_a_compiler_keeps_the_library(monkeypatch, tmp_path, capsys):
+    from mimir_amd import build
+
+    stale = tmp_path / "_host_calls.so"
+    stale.write_bytes(b"of other sources")
+    monkeypatch.setattr(build, "HOST_PATH", stale)
+    monkeypatch.setenv("CXX", str(tmp_path / "no_such_compiler"))
+    build._build_host()
+    assert not stale.exists() and "general path" in capsys.readouterr().err
