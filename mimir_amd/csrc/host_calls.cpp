@@ -41,47 +41,52 @@ struct Library {
   c10::DeviceType device = c10::DeviceType::CUDA;  // of the tensors it takes
 } lib;
 
-struct Fallback {};  // thrown where the general path takes over
-struct Raised {};    // thrown with the Python error set
-void need(bool ok) {
-  if (!ok) throw Fallback();
-}
+// Where the general path takes over, a function returns nullptr without an error set: found
+// out in 0.3 us (a C++ exception for it made it 1 to 2 us).
+#define NEED(ok) \
+  do {           \
+    if (!(ok)) return nullptr; \
+  } while (0)
 
-const at::Tensor& tensor(PyObject* o) {
-  need(THPVariable_CheckExact(o));
-  return THPVariable_Unpack(o);
-}
+const at::Tensor* tensor(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+#define TENSOR(name, o)                       \
+  const at::Tensor* const name##_ = tensor(o); \
+  NEED(name##_ != nullptr);                   \
+  const at::Tensor& name = *name##_
 bool on_device(const at::Tensor& t) { return t.device().type() == lib.device; }
 bool is_none(PyObject* o) { return o == Py_None; }
-int32_t int32(PyObject* o) {  // an int, or a one-element int64 CPU tensor (the reference's scalars)
+bool int32(PyObject* o, int32_t& out) {  // an int, or a one-element int64 CPU tensor (the reference's scalars)
   int64_t x;
   if (PyLong_CheckExact(o)) {
     x = PyLong_AsLongLong(o);
   } else {
-    const at::Tensor& t = tensor(o);
-    need(t.device().is_cpu() && t.scalar_type() == at::kLong && t.numel() == 1);
-    x = *t.const_data_ptr<int64_t>();
+    const at::Tensor* t = tensor(o);
+    if (t == nullptr || !t->device().is_cpu() || t->scalar_type() != at::kLong || t->numel() != 1) return false;
+    x = *t->const_data_ptr<int64_t>();
   }
-  need(x >= 0 && x <= 0x7fffffff);
-  return (int32_t)x;
+  out = (int32_t)x;
+  return x >= 0 && x <= 0x7fffffff;
 }
 bool truth(PyObject* o) { return PyObject_IsTrue(o) == 1; }
 void* stream(PyObject* o) { return PyLong_AsVoidPtr(o); }
 
 // A [.., heads, head_dim] operand the kernels read or write in place: unit stride on
 // head_dim, 16-byte aligned rows that do not overlap.
-void in_place(const at::Tensor& t, const at::Tensor& like) {
+bool in_place(const at::Tensor& t, const at::Tensor& like) {
   const int64_t vec = 16 / (int64_t)t.element_size(), d = t.dim();
-  need(t.device() == like.device() && t.scalar_type() == like.scalar_type() && t.has_storage());
-  need(t.stride(d - 1) == 1 && t.stride(d - 3) >= t.size(d - 1) && (uintptr_t)t.const_data_ptr() % 16 == 0);
-  for (int64_t i = 0; i < d - 1; ++i) need(t.stride(i) % vec == 0);
+  if (t.device() != like.device() || t.scalar_type() != like.scalar_type() || !t.has_storage()) return false;
+  if (t.stride(d - 1) != 1 || t.stride(d - 3) < t.size(d - 1) || (uintptr_t)t.const_data_ptr() % 16 != 0) return false;
+  for (int64_t i = 0; i < d - 1; ++i)
+    if (t.stride(i) % vec != 0) return false;
+  return true;
 }
-void shaped(const at::Tensor& t, int64_t a, int64_t b, int64_t c) {
-  need(t.dim() == 3 && t.size(0) == a && t.size(1) == b && t.size(2) == c);
+bool shaped(const at::Tensor& t, int64_t a, int64_t b, int64_t c) {
+  return t.dim() == 3 && t.size(0) == a && t.size(1) == b && t.size(2) == c;
 }
+// A metadata operand's data, nullptr where it has to be converted or is too short.
 const int32_t* metadata(PyObject* o, int64_t n, const at::Tensor& like) {
-  const at::Tensor& t = tensor(o);
-  need(t.dim() == 1 && t.size(0) >= n && t.scalar_type() == at::kInt && t.device() == like.device() && t.is_contiguous());
+  TENSOR(t, o);
+  NEED(t.dim() == 1 && t.size(0) >= n && t.scalar_type() == at::kInt && t.device() == like.device() && t.is_contiguous());
   return t.const_data_ptr<int32_t>();
 }
 
@@ -89,7 +94,8 @@ at::Tensor empty(at::IntArrayRef shape, const at::Tensor& like, at::ScalarType t
   return at::empty(shape, at::TensorOptions().dtype(type).device(like.device()));
 }
 
-// Workspaces come from the caller's torch.empty (float32): it raises where there is no room.
+// Workspaces come from the caller's torch.empty (float32): it raises where there is no
+// room, and the result is then undefined here.
 at::Tensor workspace(PyObject* torch_empty, size_t bytes, PyObject* like) {
   const size_t n = bytes / 4 < 4 ? 4 : bytes / 4;
   PyObject* device = PyObject_GetAttrString(like, "device");
@@ -98,25 +104,25 @@ at::Tensor workspace(PyObject* torch_empty, size_t bytes, PyObject* like) {
   PyObject* t = args && kw ? PyObject_Call(torch_empty, args, kw) : nullptr;
   Py_XDECREF(args);
   Py_XDECREF(kw);
-  need(t != nullptr);
-  need(THPVariable_Check(t));
-  at::Tensor out = THPVariable_Unpack(t);
-  Py_DECREF(t);
+  at::Tensor out;
+  if (t != nullptr && THPVariable_Check(t)) out = THPVariable_Unpack(t);
+  Py_XDECREF(t);
   return out;
 }
 
+// Whether the call was launched; after a HIP error `raised` and the Python error are set.
 template <typename P>
-void launch(int (*entry)(const P*, void*), const P& p, void* s) {
-  need(PyErr_Occurred() == nullptr);  // an argument did not convert
+bool launch(int (*entry)(const P*, void*), const P& p, void* s, bool& raised) {
+  if (PyErr_Occurred() != nullptr) return false;  // an argument did not convert
   int status;
   Py_BEGIN_ALLOW_THREADS;
   status = entry(&p, s);
   Py_END_ALLOW_THREADS;
   if (status == MIMIR_ERR_HIP) {
     PyErr_SetString(PyExc_RuntimeError, lib.last_error());
-    throw Raised();
+    raised = true;
   }
-  need(status == MIMIR_OK);  // else refused, nothing launched
+  return status == MIMIR_OK;  // other failures are refusals: nothing launched
 }
 
 // The checks and fields the forward and the backward share.
@@ -124,18 +130,13 @@ struct Geometry {
   int64_t T, hq, hkv, d;
   int dtype;
 };
-Geometry geometry(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
-  need(on_device(q) && q.dim() == 3 && k.dim() == 3 && v.dim() == 3);
-  const Geometry g{q.size(0), q.size(1), k.size(1), q.size(2),
-                   q.scalar_type() == at::kBFloat16 ? MIMIR_DTYPE_BFLOAT16 : MIMIR_DTYPE_FLOAT32};
-  need(q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kFloat);
-  need(g.T > 0 && g.T <= 0x7fffffff && g.hq > 0 && g.hkv > 0 && g.hq % g.hkv == 0 && g.d > 0);
-  shaped(k, g.T, g.hkv, g.d);
-  shaped(v, g.T, g.hkv, g.d);
-  in_place(q, q);
-  in_place(k, q);
-  in_place(v, q);
-  return g;
+bool geometry(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, Geometry& g) {
+  if (!on_device(q) || q.dim() != 3 || k.dim() != 3 || v.dim() != 3) return false;
+  if (q.scalar_type() != at::kBFloat16 && q.scalar_type() != at::kFloat) return false;
+  g = {q.size(0), q.size(1), k.size(1), q.size(2),
+       q.scalar_type() == at::kBFloat16 ? MIMIR_DTYPE_BFLOAT16 : MIMIR_DTYPE_FLOAT32};
+  return g.T > 0 && g.T <= 0x7fffffff && g.hq > 0 && g.hkv > 0 && g.hq % g.hkv == 0 && g.d > 0 &&
+         shaped(k, g.T, g.hkv, g.d) && shaped(v, g.T, g.hkv, g.d) && in_place(q, q) && in_place(k, q) && in_place(v, q);
 }
 
 #define STRIDES(p, name, t) (p).name##_stride_token = (t).stride(0), (p).name##_stride_head = (t).stride(1)
@@ -153,13 +154,13 @@ PyObject* guarded(Py_ssize_t given, Py_ssize_t wanted, F&& body) {
     PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", wanted, given);
     return nullptr;
   }
+  PyObject* out = nullptr;
+  bool raised = false;
   try {
-    if (PyObject* out = body()) return out;
-  } catch (const Raised&) {
-    return nullptr;
-  } catch (const Fallback&) {
+    out = body(raised);
   } catch (const std::exception&) {  // e.g. out of memory: the general path raises it
   }
+  if (out != nullptr || raised) return out;
   PyErr_Clear();
   Py_RETURN_NONE;
 }
@@ -168,19 +169,22 @@ PyObject* guarded(Py_ssize_t given, Py_ssize_t wanted, F&& body) {
 //     softmax_scale, split_mode, key_chunks, want_lo, gate, gated_out, torch_empty, stream)
 //   -> (out, lse, out_lo, split_flag)
 PyObject* py_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  return guarded(n, 18, [&]() -> PyObject* {
-    const at::Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]);
-    const Geometry g = geometry(q, k, v);
+  return guarded(n, 18, [&](bool& raised) -> PyObject* {
+    TENSOR(q, a[0]);
+    TENSOR(k, a[1]);
+    TENSOR(v, a[2]);
+    Geometry g;
+    NEED(geometry(q, k, v, g));
     MimirPrefixLMFwdParams p = {};
     p.is_causal = truth(a[3]);
-    p.total_seqlen = int32(a[7]);
-    p.numseqs = int32(a[8]);
-    p.max_seqlen_all = int32(a[9]);
+    NEED(int32(a[7], p.total_seqlen));
+    NEED(int32(a[8], p.numseqs));
+    NEED(int32(a[9], p.max_seqlen_all));
     p.softmax_scale = (float)PyFloat_AsDouble(a[10]);
-    p.split_mode = int32(a[11]);
-    p.prefix_lens = metadata(a[4], p.numseqs, q);
-    p.causal_lens = metadata(a[5], p.numseqs, q);
-    p.cu_seqlens = metadata(a[6], p.numseqs + 1, q);
+    NEED(int32(a[11], p.split_mode));
+    NEED((p.prefix_lens = metadata(a[4], p.numseqs, q)) != nullptr);
+    NEED((p.causal_lens = metadata(a[5], p.numseqs, q)) != nullptr);
+    NEED((p.cu_seqlens = metadata(a[6], p.numseqs + 1, q)) != nullptr);
     p.total_tokens = (int32_t)g.T, p.num_q_heads = (int32_t)g.hq, p.num_kv_heads = (int32_t)g.hkv;
     p.head_dim = (int32_t)g.d, p.dtype = g.dtype;
     const bool bf16 = g.dtype == MIMIR_DTYPE_BFLOAT16;
@@ -194,19 +198,21 @@ PyObject* py_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (lo.numel() > 0) p.out_lo = lo.mutable_data_ptr(), STRIDES(p, out_lo, lo);
     if (bf16) p.split_flag = (int32_t*)flag.mutable_data_ptr();
     if (!is_none(a[14])) {
-      const at::Tensor &gate = tensor(a[14]), &gated = tensor(a[15]);
-      shaped(gate, g.T, g.hq, g.d);
-      shaped(gated, g.T, g.hq, g.d);
-      in_place(gate, q);
-      in_place(gated, q);
+      TENSOR(gate, a[14]);
+      TENSOR(gated, a[15]);
+      NEED(shaped(gate, g.T, g.hq, g.d));
+      NEED(shaped(gated, g.T, g.hq, g.d));
+      NEED(in_place(gate, q));
+      NEED(in_place(gated, q));
       p.gate = gate.const_data_ptr(), p.gated_out = gated.mutable_data_ptr();
       STRIDES(p, gate, gate), STRIDES(p, gated_out, gated);
     }
     p.workspace_bytes = truth(a[12]) ? lib.fwd_workspace_size(&p)
                                      : lib.fwd_workspace_bytes(p.total_tokens, p.numseqs, p.max_seqlen_all);
     at::Tensor ws = workspace(a[16], p.workspace_bytes, a[0]);
+    NEED(ws.defined());
     p.workspace = ws.mutable_data_ptr();
-    launch(lib.fwd, p, stream(a[17]));
+    NEED(launch(lib.fwd, p, stream(a[17]), raised));
     return wrap({out, lse, lo, flag});
   });
 }
@@ -217,26 +223,33 @@ PyObject* py_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // grads: None, or (dgate, dq, dk, dv) views to write.  A score-gradient region above
 // region_limit needs the general path's look at the free memory.
 PyObject* py_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  return guarded(n, 24, [&]() -> PyObject* {
-    const at::Tensor &dout = tensor(a[0]), &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]);
-    const at::Tensor &out = tensor(a[4]), &lse = tensor(a[5]), &lo = tensor(a[6]), &flag = tensor(a[7]);
-    const Geometry g = geometry(q, k, v);
-    shaped(dout, g.T, g.hq, g.d);
-    shaped(out, g.T, g.hq, g.d);
-    in_place(dout, q);
-    in_place(out, q);
-    need(lse.dim() == 2 && lse.size(0) == g.hq && lse.size(1) == g.T && lse.scalar_type() == at::kFloat &&
+  return guarded(n, 24, [&](bool& raised) -> PyObject* {
+    TENSOR(dout, a[0]);
+    TENSOR(q, a[1]);
+    TENSOR(k, a[2]);
+    TENSOR(v, a[3]);
+    TENSOR(out, a[4]);
+    TENSOR(lse, a[5]);
+    TENSOR(lo, a[6]);
+    TENSOR(flag, a[7]);
+    Geometry g;
+    NEED(geometry(q, k, v, g));
+    NEED(shaped(dout, g.T, g.hq, g.d));
+    NEED(shaped(out, g.T, g.hq, g.d));
+    NEED(in_place(dout, q));
+    NEED(in_place(out, q));
+    NEED(lse.dim() == 2 && lse.size(0) == g.hq && lse.size(1) == g.T && lse.scalar_type() == at::kFloat &&
          lse.device() == q.device() && lse.is_contiguous());
     MimirPrefixLMBwdParams p = {};
     p.is_causal = truth(a[8]);
-    p.total_seqlen = int32(a[12]);
-    p.numseqs = int32(a[13]);
-    p.max_seqlen_all = int32(a[14]);
+    NEED(int32(a[12], p.total_seqlen));
+    NEED(int32(a[13], p.numseqs));
+    NEED(int32(a[14], p.max_seqlen_all));
     p.softmax_scale = (float)PyFloat_AsDouble(a[15]);
-    p.split_mode = int32(a[16]);
-    p.prefix_lens = metadata(a[9], p.numseqs, q);
-    p.causal_lens = metadata(a[10], p.numseqs, q);
-    p.cu_seqlens = metadata(a[11], p.numseqs + 1, q);
+    NEED(int32(a[16], p.split_mode));
+    NEED((p.prefix_lens = metadata(a[9], p.numseqs, q)) != nullptr);
+    NEED((p.causal_lens = metadata(a[10], p.numseqs, q)) != nullptr);
+    NEED((p.cu_seqlens = metadata(a[11], p.numseqs + 1, q)) != nullptr);
     p.total_tokens = (int32_t)g.T, p.num_q_heads = (int32_t)g.hq, p.num_kv_heads = (int32_t)g.hkv;
     p.head_dim = (int32_t)g.d, p.dtype = g.dtype;
     at::Tensor dq, dk, dv;
@@ -245,18 +258,20 @@ PyObject* py_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
       dk = empty({g.T, g.hkv, g.d}, q, q.scalar_type());
       dv = empty({g.T, g.hkv, g.d}, q, q.scalar_type());
     } else {
-      need(PyTuple_Check(a[21]) && PyTuple_GET_SIZE(a[21]) == 4 && !is_none(a[20]));
-      const at::Tensor &gate = tensor(a[20]), &dgate = tensor(PyTuple_GET_ITEM(a[21], 0));
-      dq = tensor(PyTuple_GET_ITEM(a[21], 1));
-      dk = tensor(PyTuple_GET_ITEM(a[21], 2));
-      dv = tensor(PyTuple_GET_ITEM(a[21], 3));
-      shaped(gate, g.T, g.hq, g.d);
-      shaped(dgate, g.T, g.hq, g.d);
-      shaped(dq, g.T, g.hq, g.d);
-      shaped(dk, g.T, g.hkv, g.d);
-      shaped(dv, g.T, g.hkv, g.d);
+      NEED(PyTuple_Check(a[21]) && PyTuple_GET_SIZE(a[21]) == 4 && !is_none(a[20]));
+      TENSOR(gate, a[20]);
+      TENSOR(dgate, PyTuple_GET_ITEM(a[21], 0));
+      TENSOR(dq_view, PyTuple_GET_ITEM(a[21], 1));
+      TENSOR(dk_view, PyTuple_GET_ITEM(a[21], 2));
+      TENSOR(dv_view, PyTuple_GET_ITEM(a[21], 3));
+      dq = dq_view, dk = dk_view, dv = dv_view;
+      NEED(shaped(gate, g.T, g.hq, g.d));
+      NEED(shaped(dgate, g.T, g.hq, g.d));
+      NEED(shaped(dq, g.T, g.hq, g.d));
+      NEED(shaped(dk, g.T, g.hkv, g.d));
+      NEED(shaped(dv, g.T, g.hkv, g.d));
       for (const at::Tensor* t : {&gate, &dgate, (const at::Tensor*)&dq, (const at::Tensor*)&dk, (const at::Tensor*)&dv})
-        in_place(*t, q);
+        NEED(in_place(*t, q));
       p.gate = gate.const_data_ptr(), p.dgate = dgate.mutable_data_ptr();
       STRIDES(p, gate, gate), STRIDES(p, dgate, dgate);
     }
@@ -267,44 +282,48 @@ PyObject* py_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
     STRIDES(p, dq, dq), STRIDES(p, dk, dk), STRIDES(p, dv, dv);
     p.lse_stride_head = g.T;
     if (lo.numel() > 0) {
-      shaped(lo, g.T, g.hq, g.d);
-      in_place(lo, q);
+      NEED(shaped(lo, g.T, g.hq, g.d));
+      NEED(in_place(lo, q));
       p.out_lo = lo.const_data_ptr(), STRIDES(p, out_lo, lo);
     }
     if (flag.numel() > 0) {
-      need(flag.scalar_type() == at::kInt && flag.device() == q.device());
+      NEED(flag.scalar_type() == at::kInt && flag.device() == q.device());
       p.split_flag = flag.const_data_ptr<int32_t>();
     }
     p.dq_key_chunks = truth(a[17]);
     p.dscore_limit_bytes = (size_t)PyLong_AsUnsignedLongLong(a[18]);
-    if (p.dscore_limit_bytes > 0) need(lib.bwd_dscore_bytes(&p) <= (size_t)PyLong_AsUnsignedLongLong(a[19]));
+    if (p.dscore_limit_bytes > 0) NEED(lib.bwd_dscore_bytes(&p) <= (size_t)PyLong_AsUnsignedLongLong(a[19]));
     p.workspace_bytes = lib.bwd_workspace_size(&p);
     at::Tensor ws = workspace(a[22], p.workspace_bytes, a[1]);
+    NEED(ws.defined());
     p.workspace = ws.mutable_data_ptr();
-    launch(lib.bwd, p, stream(a[23]));
+    NEED(launch(lib.bwd, p, stream(a[23]), raised));
     return wrap({dq, dk, dv});
   });
 }
 
 // rope(x, cos, sin, inverse, out_or_None, stream) -> out
 PyObject* py_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  return guarded(n, 6, [&]() -> PyObject* {
-    const at::Tensor &x = tensor(a[0]), &cos = tensor(a[1]), &sin = tensor(a[2]);
-    need(on_device(x) && x.dim() == 3 && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat));
-    in_place(x, x);
+  return guarded(n, 6, [&](bool& raised) -> PyObject* {
+    TENSOR(x, a[0]);
+    TENSOR(cos, a[1]);
+    TENSOR(sin, a[2]);
+    NEED(on_device(x) && x.dim() == 3 && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat));
+    NEED(in_place(x, x));
     const int64_t T = x.size(0), d = x.size(2);
-    need(T <= 0x7fffffff && x.size(1) > 0);
+    NEED(T <= 0x7fffffff && x.size(1) > 0);
     for (const at::Tensor* t : {&cos, &sin})
-      need(t->dim() == 2 && t->size(0) == T && t->size(1) == d && t->scalar_type() == at::kFloat &&
+      NEED(t->dim() == 2 && t->size(0) == T && t->size(1) == d && t->scalar_type() == at::kFloat &&
            t->device() == x.device() && t->stride(1) == 1 && t->stride(0) == cos.stride(0) && t->stride(0) % 4 == 0 &&
            (uintptr_t)t->const_data_ptr() % 16 == 0);
     at::Tensor out;
     if (is_none(a[4])) {
       out = empty({T, x.size(1), d}, x, x.scalar_type());
     } else {
-      out = tensor(a[4]);
-      shaped(out, T, x.size(1), d);
-      in_place(out, x);
+      TENSOR(out_view, a[4]);
+      out = out_view;
+      NEED(shaped(out, T, x.size(1), d));
+      NEED(in_place(out, x));
     }
     MimirRopeParams p = {};
     p.x = x.const_data_ptr(), p.y = out.mutable_data_ptr();
@@ -315,7 +334,7 @@ PyObject* py_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
     p.total_tokens = (int32_t)T, p.num_heads = (int32_t)x.size(1), p.head_dim = (int32_t)d;
     p.dtype = x.scalar_type() == at::kBFloat16 ? MIMIR_DTYPE_BFLOAT16 : MIMIR_DTYPE_FLOAT32;
     p.inverse = truth(a[3]);
-    launch(lib.rope, p, stream(a[5]));
+    NEED(launch(lib.rope, p, stream(a[5]), raised));
     return THPVariable_Wrap(out);
   });
 }
@@ -323,26 +342,30 @@ PyObject* py_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // cache_attn(query, key, value, cache_keys, cache_values, cache_lengths, causal, batch_indices, softmax_scale,
 //            torch_empty, stream) -> out
 PyObject* py_cache_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  return guarded(n, 11, [&]() -> PyObject* {
-    const at::Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]), &ck = tensor(a[3]), &cv = tensor(a[4]);
-    const at::Tensor& lens = tensor(a[5]);
-    need(on_device(q) && q.scalar_type() == at::kBFloat16 && q.dim() == 4 && k.dim() == 4 && v.dim() == 4 &&
+  return guarded(n, 11, [&](bool& raised) -> PyObject* {
+    TENSOR(q, a[0]);
+    TENSOR(k, a[1]);
+    TENSOR(v, a[2]);
+    TENSOR(ck, a[3]);
+    TENSOR(cv, a[4]);
+    TENSOR(lens, a[5]);
+    NEED(on_device(q) && q.scalar_type() == at::kBFloat16 && q.dim() == 4 && k.dim() == 4 && v.dim() == 4 &&
          ck.dim() == 4 && cv.dim() == 4);
     const int64_t B = q.size(0), S = q.size(1), hq = q.size(2), d = q.size(3), hkv = k.size(2), L = ck.size(1);
-    need(B > 0 && S > 0 && hq > 0 && hkv > 0 && hq % hkv == 0 && L > 0 && B <= 0x7fffffff && S <= 0x7fffffff &&
+    NEED(B > 0 && S > 0 && hq > 0 && hkv > 0 && hq % hkv == 0 && L > 0 && B <= 0x7fffffff && S <= 0x7fffffff &&
          L <= 0x7fffffff && ck.size(0) <= 0x7fffffff);
-    for (const at::Tensor* t : {&k, &v}) need(t->size(0) == B && t->size(1) == S && t->size(2) == hkv && t->size(3) == d);
-    for (const at::Tensor* t : {&ck, &cv}) need(t->size(2) == hkv && t->size(3) == d && t->sizes() == ck.sizes());
-    for (const at::Tensor* t : {&q, &k, &v, &ck, &cv}) in_place(*t, q);
+    for (const at::Tensor* t : {&k, &v}) NEED(t->size(0) == B && t->size(1) == S && t->size(2) == hkv && t->size(3) == d);
+    for (const at::Tensor* t : {&ck, &cv}) NEED(t->size(2) == hkv && t->size(3) == d && t->sizes() == ck.sizes());
+    for (const at::Tensor* t : {&q, &k, &v, &ck, &cv}) NEED(in_place(*t, q));
     MimirCacheAttnParams p = {};
     for (PyObject* o : {a[5], a[7]}) {
       if (is_none(o)) continue;
-      const at::Tensor& t = tensor(o);
-      need(t.dim() == 1 && t.size(0) == B && t.device() == q.device() && t.is_contiguous() &&
+      TENSOR(t, o);
+      NEED(t.dim() == 1 && t.size(0) == B && t.device() == q.device() && t.is_contiguous() &&
            t.scalar_type() == lens.scalar_type() && (t.scalar_type() == at::kLong || t.scalar_type() == at::kInt));
     }
     p.cache_lengths = lens.const_data_ptr();
-    if (!is_none(a[7])) p.batch_indices = tensor(a[7]).const_data_ptr();
+    if (!is_none(a[7])) p.batch_indices = tensor(a[7])->const_data_ptr();
     p.index_int64 = lens.scalar_type() == at::kLong;
     at::Tensor out = empty({B, S, hq, d}, q, at::kBFloat16);
     p.q = q.const_data_ptr(), p.k_new = k.const_data_ptr(), p.v_new = v.const_data_ptr();
@@ -358,9 +381,10 @@ PyObject* py_cache_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::Tensor ws;
     if (p.workspace_bytes > 0) {
       ws = workspace(a[9], p.workspace_bytes, a[0]);
+      NEED(ws.defined());
       p.workspace = ws.mutable_data_ptr();
     }
-    launch(lib.cache_attn, p, stream(a[10]));
+    NEED(launch(lib.cache_attn, p, stream(a[10]), raised));
     return THPVariable_Wrap(out);
   });
 }
