@@ -275,6 +275,81 @@ def test_prefill_reads_the_new_rows_in_place_split_keys(device, S, hq, hkv, d, l
         _run(device, B=3, S=S, hq=hq, hkv=hkv, d=d, L=1496, lens=lens, causal=causal, seed=S)
 
 
+def _prefill(device, B, S, hq, hkv, d, L, lens, rows, cache_rows, causal, strided, seed):
+    """A chunk against the oracle, with q / k / v contiguous or slices of one projection (``strided``
+    names them), into cache rows ``rows``; batch rows outside the cache (-1, cache_rows) get zeros."""
+    gen = torch.Generator().manual_seed(seed)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(BF16)
+    heads = dict(q=hq, k=hkv, v=hkv)
+    fused = mk(B, S, hq + 2 * hkv, d)
+    parts = dict(zip("qkv", fused.split((hq, hkv, hkv), dim=2)))
+    ck, cv = mk(cache_rows, L, hkv, d), mk(cache_rows, L, hkv, d)
+    cache = Cache(ck.to(device), cv.to(device))
+    dev = dict(zip("qkv", fused.to(device).split((hq, hkv, hkv), dim=2)))
+    args = [dev[n] if n in strided else dev[n].contiguous() for n in "qkv"]
+    assert all((a.stride(1) != heads[n] * d) == (n in strided) for n, a in zip("qkv", args))
+    rows_t = None if rows is None else torch.tensor(rows)
+    out = attention_with_cache(*args, cache, torch.tensor(lens, device=device), causal,
+                               None if rows is None else rows_t.to(device))
+    torch.cuda.synchronize()
+    inside = torch.ones(B, dtype=torch.bool) if rows is None else (rows_t >= 0) & (rows_t < cache_rows)
+    ref = torch.zeros(B, S, hq, d, dtype=BF16)
+    ref[inside] = LO.attention_with_cache(*(parts[n][inside] for n in "qkv"), ck, cv, torch.tensor(lens)[inside], causal,
+                                          None if rows is None else rows_t[inside])
+    assert (out.float().cpu() - ref.float()).abs().max().item() <= 2e-2
+    assert torch.count_nonzero(out[~inside]) == 0
+    assert torch.equal(cache.keys.cpu(), ck) and torch.equal(cache.values.cpu(), cv)
+
+
+# Sizes with the key range split (few row tiles) and not (24 batch rows).
+@pytest.mark.parametrize("B,S,hq,hkv,d,L", [(4, 50, 8, 2, 128, 900), (4, 130, 2, 2, 64, 900), (24, 300, 8, 4, 128, 420),
+                                            (24, 600, 4, 4, 64, 700)])
+@pytest.mark.parametrize("form", ["shuffled", "outside", "shared"])
+def test_prefill_into_chosen_cache_rows(device, B, S, hq, hkv, d, L, form):
+    """batch_indices: the new rows are appended by a launch of their own.  Shuffled rows of a larger
+    cache; one of them outside it; several batch rows on a cache row, each at positions of its own,
+    which then see each other's new rows."""
+    gen = torch.Generator().manual_seed(B + S)
+    lens = torch.randint(0, L - S + 1, (B,), generator=gen).tolist()
+    rows = torch.randperm(B + 3, generator=gen)[:B].tolist()
+    n, causal = B + 3, True
+    if form == "outside":
+        rows[1], rows[-1] = -1, n
+    elif form == "shared":
+        per = L // S  # batch rows on one cache row
+        n, causal = -(-B // per), False
+        rows, lens = [b // per for b in range(B)], [b % per * S for b in range(B)]
+    _prefill(device, B, S, hq, hkv, d, L, lens, rows, n, causal, "", seed=S)
+
+
+@pytest.mark.parametrize("B,S,hq,hkv,d,L", [(3, 60, 8, 2, 128, 900), (24, 300, 8, 4, 128, 420), (4, 200, 4, 4, 64, 500)])
+@pytest.mark.parametrize("strided", ["v", "k", "kv", "qkv"])
+def test_prefill_from_the_projection(device, B, S, hq, hkv, d, L, strided):
+    """k or v (or both) as slices of the fused projection, whose token stride is not the cache's:
+    appended by a launch of their own also where only one of the strides differs."""
+    gen = torch.Generator().manual_seed(S)
+    lens = torch.randint(0, L - S + 1, (B,), generator=gen).tolist()
+    for causal in (True, False):
+        _prefill(device, B, S, hq, hkv, d, L, lens, None, B, causal, strided, seed=S)
+
+
+def test_prefill_with_the_strides_of_a_wider_cache(device):
+    """New rows whose token stride is the cache's although neither is dense: slices of wider buffers."""
+    B, S, hq, hkv, d, L = 3, 70, 4, 2, 64, 300
+    gen = torch.Generator().manual_seed(8)
+    mk = lambda *s: torch.randn(*s, generator=gen).to(BF16)
+    q, kw, vw, ckw, cvw = mk(B, S, hq, d), mk(B, S, 5, d), mk(B, S, 5, d), mk(B, L, 5, d), mk(B, L, 5, d)
+    ck, cv = ckw[:, :, 1:3], cvw[:, :, 2:4]
+    dev = [t.to(device) for t in (q, kw, vw, ckw, cvw)]
+    lens = torch.tensor([0, 100, 230])
+    out = attention_with_cache(dev[0], dev[1][:, :, :2], dev[2][:, :, 3:], Cache(dev[3][:, :, 1:3], dev[4][:, :, 2:4]),
+                               lens.to(device), True)
+    torch.cuda.synchronize()
+    ref = LO.attention_with_cache(q, kw[:, :, :2], vw[:, :, 3:], ck, cv, lens, True)
+    assert (out.float().cpu() - ref.float()).abs().max().item() <= 2e-2
+    assert torch.equal(dev[3].cpu(), ckw) and torch.equal(dev[4].cpu(), cvw)
+
+
 @pytest.mark.parametrize("S", [1, 40])
 def test_lengths_outside_the_cache(device, S):
     """Without validation, new rows at positions outside the cache are dropped, and the row attends
