@@ -174,10 +174,12 @@ def working_kernels(d: int, elem: int, handoff: bool) -> dict:
 
     One bf16 kernel serves both split modes (the device-side decision picks the
     body inside it).  ``handoff``: the dK/dV kernel stores dS and dq_ds_kernel
-    reads it.
+    reads it.  The float32 backward is one kernel: its dK/dV and dQ workgroups
+    share a launch in a step, and have one each where the stages are timed.
     """
     if elem == 4:
-        return {"fwd": f"fwd_f32_kernel<{d}>", "dkdv": f"dkdv_f32_kernel<{d}>", "dq": f"dq_f32_kernel<{d}>"}
+        bwd = f"bwd_f32_kernel<{d}>"
+        return {"fwd": f"fwd_f32_kernel<{d}>", "dkdv": f"{bwd} (dK/dV workgroups)", "dq": f"{bwd} (dQ workgroups)"}
     if d == 128:
         dkdv = "dkdv_pair_ds_kernel" if handoff else "dkdv_pair_kernel"
     else:
@@ -679,6 +681,8 @@ def main() -> int:
     res["dscore_handoff"] = handoff
     if elem == 2 and not fwd_only:
         res["split_active"] = split
+    if elem == 4 and not fwd_only:
+        res["stage_note"] = "dkdv and dq, timed one after the other, share one launch in a step"
     if handoff:
         # the dQ kernel is then HBM-bound: it streams every stored dS block once
         # (plus K once and the dQ rows)
