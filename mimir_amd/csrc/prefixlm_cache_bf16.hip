@@ -883,6 +883,8 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   };
 
   f32x16 oacc[DT];
+  // In scores, and finite (a scale below 1e-37): a tile without keys for a row keeps a reference.
+  const float ref_range = fminf(kRefRange / c2, 3e38f);
   float m_run, m_top, l_run;  // the sums' reference and the row's maximum so far (scores), the sum
   auto compute = [&](int t, const bf16_t* sK, const bf16_t* sV) {
     const int kb = t * kDecKeys;
@@ -910,7 +912,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
     // 1000 to 3600 2.09e-3 / 2.02e-3, 64 of 100 to 3000 2.12e-3 / 2.02e-3; time 11.9 / 11.5
     // us, 17.1 / 16.7, and 64 rows of 500 to 8000 120.3 / 119.8.
     m_top = fmaxf(m_top, mx);
-    const float m_new = fmaxf(mx, m_top - kRefRange / c2);
+    const float m_new = fmaxf(mx, m_top - ref_range);
     const float alpha = m_run == -INFINITY ? 1.f : fast_exp2((m_run - m_new) * c2);
     l_run *= alpha;
 #pragma unroll

@@ -121,6 +121,20 @@ def test_decode_reference_of_a_low_tile(device):
     assert (out.float().cpu() - ref.float()).abs().max().item() <= 2e-2
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("scale", [1e-38, 1e-30])
+def test_decode_with_a_tiny_scale(device, d, scale):
+    """Every score is 0: the mean of the values, also for a token that a later tile holds no key for."""
+    B, S, L, n = 1, 2, 4096, 63  # token 0 ends with tile 1, token 1 is alone in tile 2
+    gen = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(B, S, 2, d, generator=gen).to(BF16).to(device) for _ in range(3))
+    cache = Cache(*(torch.randn(B, L, 2, d, generator=gen).to(BF16).to(device) for _ in range(2)))
+    out = attention_with_cache(q, k, v, cache, torch.tensor([n], device=device), True, softmax_scale=scale)
+    ref = torch.stack([cache.values[0, :n + 1 + i].double().mean(0) for i in range(S)])
+    # every probability is 1: what is left is the rounding of the output
+    assert (out[0].double() - ref).abs().max().item() <= 2.0**-8 * ref.abs().max().item()
+
+
 def test_decode_rows_sharing_a_cache_row(device):
     """Batch rows on one cache row attend each other's new keys, as after appending all of them
     first: consecutive tokens of a sequence fed as separate batch rows, and one far behind."""
