@@ -31,6 +31,7 @@ constexpr int kThreads = kWaves * 64;
 constexpr int kRows = kWaves * 32;  // query rows per workgroup
 constexpr int kKeys = 64;           // keys per tile
 constexpr int kMaxSplits = 64;      // key splits per row tile
+constexpr int kMaxAppend = 1024;    // new tokens that the prefill kernel appends itself
 
 struct CacheArgs {
   const bf16_t* q;
@@ -385,17 +386,29 @@ __global__ __launch_bounds__(kThreads, 2) void cache_attn_kernel(const CacheArgs
   };
 
   // The new tokens whose first row lies in this row tile go into the cache here (no
-  // workgroup reads these cache rows).
+  // workgroup reads these cache rows): with a kv head per q head all 128 rows are tokens,
+  // and one load after another held up the first tile (8 x 1024 on 150 to 2000 keys, 6 / 6
+  // heads of 128: 126.0 us, 121.6 with four in flight; 12 x 700 on none 87.6 -> 84.8).
   if (kAppend && split == 0 && row_in_cache) {
-    constexpr int kUnits = D / 8;
+    constexpr int kUnits = D / 8, kStep = kThreads / kUnits, kBatch = 4;
     const int first = max((rt * kRows + a.G - 1) / a.G, -pos);
     const int last = min(((rt + 1) * kRows + a.G - 1) / a.G, min(a.S, a.L - pos));
-    for (int t = first + tid / kUnits; t < last; t += kThreads / kUnits) {
-      const int c = tid % kUnits * 8;
-      *(bf16x8*)&a.ck[crow * a.ck_sb + (int64_t)(pos + t) * a.ck_st + (int64_t)hk * a.ck_sh + c] =
-          *(const bf16x8*)&knb[(int64_t)t * a.kn_st + c];
-      *(bf16x8*)&a.cv[crow * a.cv_sb + (int64_t)(pos + t) * a.cv_st + (int64_t)hk * a.cv_sh + c] =
-          *(const bf16x8*)&vnb[(int64_t)t * a.vn_st + c];
+    const int c = tid % kUnits * 8;
+    for (int t0 = first + tid / kUnits; t0 < last; t0 += kBatch * kStep) {
+      bf16x8 kx[kBatch], vx[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int t = min(t0 + i * kStep, last - 1);
+        kx[i] = *(const bf16x8*)&knb[(int64_t)t * a.kn_st + c];
+        vx[i] = *(const bf16x8*)&vnb[(int64_t)t * a.vn_st + c];
+      }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int t = t0 + i * kStep;
+        if (t >= last) break;
+        *(bf16x8*)&a.ck[crow * a.ck_sb + (int64_t)(pos + t) * a.ck_st + (int64_t)hk * a.ck_sh + c] = kx[i];
+        *(bf16x8*)&a.cv[crow * a.cv_sb + (int64_t)(pos + t) * a.cv_st + (int64_t)hk * a.cv_sh + c] = vx[i];
+      }
     }
   }
 
@@ -1202,8 +1215,13 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   // over the batch, every batch row sees all new rows, as after appending all of them.)
   // Decode finds the batch rows on one cache row by their indices, up to 64 of them;
   // prefill does not, and needs one set of copy offsets for the new rows and the cache.
+  // Longer chunks outweigh the launch that this saves: the kernel without it is 1 to 4%
+  // faster (append launch / in place, rows on 150 to 2000 keys: 8 x 2048, 6 / 6 heads of 128,
+  // 181 / 189 us, 8 / 8 of 64 137 / 143, 32 / 8 of 128 657 / 673; 4 x 1024, 8 / 8 of 64, 58.6 / 57.7,
+  // 16 / 4 of 128 90.0 / 88.1; 12 x 700 on none, 8 / 8 of 64, 26.8 / 20.5).
   a.append = cache_rows_distinct(p) &&
-             (sp.decode ? a.batch_indices == nullptr || a.B <= 64 : (a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st));
+             (sp.decode ? a.batch_indices == nullptr || a.B <= 64
+                        : a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st && a.S <= kMaxAppend);
   const int64_t appends = (int64_t)a.B * a.S * a.Hkv * (a.D / 8);
   if ((sp.decode ? !sp.pairs : sp.splits > 1) && p.workspace == nullptr) return hipErrorInvalidValue;
   if (appends > 0 && !a.append) hipLaunchKernelGGL(cache_append_kernel, dim3(grid_for(appends)), dim3(256), 0, stream, a);

@@ -289,6 +289,14 @@ def test_prefill_reads_the_new_rows_in_place_split_keys(device, S, hq, hkv, d, l
         _run(device, B=3, S=S, hq=hq, hkv=hkv, d=d, L=1496, lens=lens, causal=causal, seed=S)
 
 
+@pytest.mark.parametrize("S", [1024, 1025])
+def test_prefill_around_the_longest_chunk_appended_in_place(device, S):
+    """The longest chunk whose rows the attention kernel appends, and the first that a launch of
+    its own does; a q head per kv head, so that a workgroup appends 128 tokens."""
+    for causal in (True, False):
+        _run(device, B=2, S=S, hq=2, hkv=2, d=128, L=1100, lens=[70, 0], causal=causal, seed=S)
+
+
 def _prefill(device, B, S, hq, hkv, d, L, lens, rows, cache_rows, causal, strided, seed):
     """A chunk against the oracle, with q / k / v contiguous or slices of one projection (``strided``
     names them), into cache rows ``rows``; batch rows outside the cache (-1, cache_rows) get zeros."""
