@@ -593,9 +593,13 @@ struct TileLine {
     return r;
   }
   __device__ __forceinline__ void set(const CacheArgs& a, Raw r, int first_, int before) {
+    place(a, r.length < -(int64_t)a.S ? -a.S : (r.length > a.L ? a.L : (int)r.length),
+          r.row >= 0 && r.row < a.rows ? (int)r.row : -1, first_, before);
+  }
+  __device__ __forceinline__ void place(const CacheArgs& a, int pos_, int row_, int first_, int before) {
     first = first_;
-    pos = r.length < -(int64_t)a.S ? -a.S : (r.length > a.L ? a.L : (int)r.length);
-    row = r.row >= 0 && r.row < a.rows ? (int)r.row : -1;
+    pos = pos_;
+    row = row_;
     keys = row >= 0 ? min(max(pos, 0) + a.S, a.L) : 0;
     units = ((keys + kDecKeys - 1) / kDecKeys + kShareUnit - 1) / kShareUnit;
     incl = before + wave_inclusive_sum(units);
@@ -607,38 +611,60 @@ struct TileLine {
 };
 
 // The line of a batch of more than 64 rows (at most kLineRows): lane c holds the units
-// per kv head of batch rows 64 c .. 64 c + 63, and of all up to the last of them.  The
-// loads of four chunks are in flight together, and each workgroup then loads the one
-// chunk that it needs.  (Chunk after chunk, once for the total and once more up to its
-// own, a round trip each: 512 rows of 0 to 300 keys in 4096 positions, 4 kv heads, 64.3
-// us, so 59.8.)  Past kLineRows there is a workgroup per pair, which needs no line: 1000
-// rows of 0 to 300 keys, one kv head, 47.6 us with the line chunk after chunk, 38.5 so,
-// 30.1 with pairs; 512 of 0 to 2000, 4 kv heads, 212 with the line, 222 with pairs.
-constexpr int kLineRows = 512;
+// per kv head of batch rows 64 c .. 64 c + 63, and of all up to the last of them; the rows
+// themselves stay in registers, 64 to a chunk.  All of them are loaded together, and with
+// indices the batch rows on one cache row are found without a look at memory, so that the
+// new rows need no launch of their own.  (Four chunks at a time and the needed one again,
+// new rows appended first with indices: 128 rows of 2000 keys, 8 / 2 heads of 64, 30.9 us, so
+// 30.3, with indices 34.6 -> 30.9; 300 of 0 to 100, 4 kv heads of 128, 26.2 -> 24.7 and 28.8 ->
+// 25.7.)  Past kLineRows there is a workgroup per pair, which needs no line: 1000 rows of 0 to
+// 300 keys, one kv head, 38.5 us with the line, 30.1 with pairs.
+constexpr int kLineChunks = 8;
+constexpr int kLineRows = 64 * kLineChunks;
 struct LineChunks {
   int units, incl;
+  int pos[kLineChunks], row[kLineChunks];
   template <typename F>
   __device__ __forceinline__ void scan(const CacheArgs& a, int lane, F&& each) {
-    constexpr int kAhead = 4;
+    TileLine::Raw raw[kLineChunks];
+#pragma unroll
+    for (int c = 0; c < kLineChunks; ++c) {
+      raw[c] = {0, -1};
+      if (64 * c < a.B) raw[c] = TileLine::fetch(a, 64 * c, lane);
+    }
     units = 0;
-    for (int c0 = 0; 64 * c0 < a.B; c0 += kAhead) {
-      TileLine::Raw raw[kAhead];
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) raw[i] = TileLine::fetch(a, 64 * (c0 + i), lane);
-#pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        TileLine line;
-        line.set(a, raw[i], 64 * (c0 + i), 0);
-        each(line);
-        const int n = line.end();
-        if (lane == c0 + i) units = n;
-      }
+    for (int c = 0; c < kLineChunks; ++c) {
+      pos[c] = 0, row[c] = -1;
+      if (64 * c >= a.B) continue;  // uniform
+      TileLine line;
+      line.set(a, raw[c], 64 * c, 0);
+      each(line);
+      pos[c] = line.pos, row[c] = line.row;
+      const int n = line.end();
+      if (lane == c) units = n;
     }
     incl = wave_inclusive_sum(units);
   }
   __device__ __forceinline__ int total() const { return __builtin_amdgcn_readlane(incl, 63); }
-  __device__ __forceinline__ int before(int c) const {
-    return __builtin_amdgcn_readlane(incl, c) - __builtin_amdgcn_readlane(units, c);
+  // Chunk c (uniform): its positions and cache rows, and its part of the line.
+  __device__ __forceinline__ void rows(int c, int& p, int& r) const {
+    p = pos[0], r = row[0];
+#pragma unroll
+    for (int i = 1; i < kLineChunks; ++i) p = c == i ? pos[i] : p, r = c == i ? row[i] : r;
+  }
+  // How many batch rows have cache row r.
+  __device__ __forceinline__ int on_row(const CacheArgs& a, int r) const {
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < kLineChunks; ++c)
+      if (64 * c < a.B) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(row[c] == r));
+    return n;
+  }
+  __device__ __forceinline__ void line(const CacheArgs& a, int c, TileLine& l) const {
+    int p, r;
+    rows(c, p, r);
+    l.place(a, p, r, 64 * c, __builtin_amdgcn_readlane(incl, c) - __builtin_amdgcn_readlane(units, c));
   }
 };
 
@@ -717,6 +743,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   // This share [u_begin, u_end) of the line, and the first batch row it touches: lane j
   // of the loaded rows.  One workgroup per pair: its batch row, and no line.
   TileLine line;
+  LineChunks chunks;  // of more than 64 batch rows, not for pairs
   const int share = blockIdx.x / a.Hkv, hk = blockIdx.x - share * a.Hkv;  // share: the batch row, for pairs
   int j, u_begin = 0, u_end = 1;
   if constexpr (kPairs) {
@@ -727,7 +754,6 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
       return;
     }
   } else {
-    LineChunks chunks;
     int total;
     if (a.B <= 64) {
       line.load(a, 0, 0, lane);
@@ -742,8 +768,7 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
     u_end = shares.begin(share + 1);
     if (u_begin >= u_end) return;
     if (a.B > 64) {
-      const int c = __builtin_ctzll(__builtin_amdgcn_ballot_w64(chunks.incl > u_begin));
-      line.load(a, 64 * c, chunks.before(c), lane);
+      chunks.line(a, __builtin_ctzll(__builtin_amdgcn_ballot_w64(chunks.incl > u_begin)), line);
     }
     j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl > u_begin));
   }
@@ -790,17 +815,22 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
   int b, kv, pos_b, crow, t0, n_my, kend_lane, kend_min, u_next;
   bool whole;
   int new_lo, new_hi;  // positions [new_lo, new_hi) may hold new rows
+  bool shared;         // other batch rows are on its cache row
   bf16_t *kbase, *vbase;
   bf16x8 qf[KS];
 
-  // The other batch rows on the segment's cache row: f(batch row, its position).  With
-  // indices the call has at most 64 batch rows, all of them in the line.
+  // The other batch rows on the segment's cache row: f(batch row, its position).  (Pairs:
+  // calls with indices have at most 64 batch rows here, all of them in the line.)
   auto for_others = [&](auto&& f) __attribute__((always_inline)) {
-    if (a.batch_indices == nullptr) return;
-    uint64_t same = __builtin_amdgcn_ballot_w64(line.row == crow && lane != b);
-    for (; same != 0; same &= same - 1) {
-      const int o = __builtin_ctzll(same);
-      f(o, __builtin_amdgcn_readlane(line.pos, o));
+    if (!shared) return;
+    for (int o0 = 0; o0 < a.B; o0 += 64) {
+      int pos = line.pos, row = line.row;
+      if (!kPairs && a.B > 64) chunks.rows(o0 / 64, pos, row);
+      uint64_t same = __builtin_amdgcn_ballot_w64(row == crow && o0 + lane != b);
+      for (; same != 0; same &= same - 1) {
+        const int o = __builtin_ctzll(same);
+        f(o0 + o, __builtin_amdgcn_readlane(pos, o));
+      }
     }
   };
   // Overlay tile t's copy with the new rows (of batch row o, at position p on)
@@ -889,6 +919,9 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
     if (!a.append) return;
     new_lo = pos_b;
     new_hi = pos_b + a.S;
+    shared = a.batch_indices != nullptr;
+    if (shared)
+      shared = (!kPairs && a.B > 64 ? chunks.on_row(a, crow) : __builtin_popcountll(__builtin_amdgcn_ballot_w64(line.row == crow))) > 1;
     for_others([&](int, int p) {
       new_lo = min(new_lo, p);
       new_hi = max(new_hi, p + a.S);
@@ -1000,7 +1033,8 @@ __device__ __forceinline__ void cache_decode_body(const CacheArgs& a) {
     wait_lds();
     if (more) {
       u0 = u_next;  // the next batch row with keys
-      while (line.end() <= u0) line.load(a, line.first + 64, line.end(), lane);
+      if constexpr (!kPairs)
+        while (line.end() <= u0) chunks.line(a, line.first / 64 + 1, line);
       j = __builtin_ctzll(__builtin_amdgcn_ballot_w64(line.incl > u0));
       begin();
     }
@@ -1097,7 +1131,7 @@ __device__ __forceinline__ void cache_merge_body(const CacheArgs& a) {
     LineChunks chunks;
     chunks.scan(a, lane, [](const TileLine&) {});
     total = chunks.total();
-    line.load(a, b & ~63, chunks.before(b / 64), lane);
+    chunks.line(a, b / 64, line);
   }
   const int units_b = __builtin_amdgcn_readlane(line.units, b & 63);
   const int before = __builtin_amdgcn_readlane(line.incl, b & 63) - units_b;
@@ -1213,14 +1247,15 @@ hipError_t launch_cache_attn_bf16(const MimirCacheAttnParams& p, hipStream_t str
   // from the cache, which asks for cache rows that share no memory: a batch row's new
   // rows are then seen through its own cache row alone.  (Shared, e.g. a cache expanded
   // over the batch, every batch row sees all new rows, as after appending all of them.)
-  // Decode finds the batch rows on one cache row by their indices, up to 64 of them;
+  // Decode finds the batch rows on one cache row by their indices (a workgroup per pair
+  // looks at up to 64 batch rows);
   // prefill does not, and needs one set of copy offsets for the new rows and the cache.
   // Longer chunks outweigh the launch that this saves: the kernel without it is 1 to 4%
   // faster (append launch / in place, rows on 150 to 2000 keys: 8 x 2048, 6 / 6 heads of 128,
   // 181 / 189 us, 8 / 8 of 64 137 / 143, 32 / 8 of 128 657 / 673; 4 x 1024, 8 / 8 of 64, 58.6 / 57.7,
   // 16 / 4 of 128 90.0 / 88.1; 12 x 700 on none, 8 / 8 of 64, 26.8 / 20.5).
   a.append = cache_rows_distinct(p) &&
-             (sp.decode ? a.batch_indices == nullptr || a.B <= 64
+             (sp.decode ? a.batch_indices == nullptr || a.B <= 64 || !sp.pairs
                         : a.batch_indices == nullptr && a.kn_st == a.ck_st && a.vn_st == a.cv_st && a.S <= kMaxAppend);
   const int64_t appends = (int64_t)a.B * a.S * a.Hkv * (a.D / 8);
   if ((sp.decode ? !sp.pairs : sp.splits > 1) && p.workspace == nullptr) return hipErrorInvalidValue;

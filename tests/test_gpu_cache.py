@@ -190,10 +190,13 @@ def test_cache_rows_that_share_memory(device, d, S, lens, form):
 @pytest.mark.parametrize("B,S,hq,hkv,d,L,rows", [
     (65, 1, 2, 1, 64, 3000, None),        # shares: one batch row past the first 64
     (130, 2, 4, 2, 128, 1300, None),      # three chunks of batch rows
-    (512, 1, 2, 1, 64, 1100, "distinct"), # as many as a share looks through; appended first
+    (512, 1, 2, 1, 64, 1100, "distinct"), # pairs: in a cache this short
+    (512, 1, 2, 1, 64, 2100, "distinct"), # as many as a share looks through
     (513, 1, 2, 1, 64, 1100, None),       # a workgroup per pair from here on
     (100, 1, 4, 2, 128, 300, "distinct"), # pairs, appended first
-    (200, 1, 4, 1, 64, 1500, "shared"),   # 200 batch rows on 90 cache rows
+    (200, 1, 4, 1, 64, 1500, "shared"),   # pairs: 200 batch rows on 90 cache rows
+    (200, 1, 4, 1, 64, 3000, "shared"),   # shares: batch rows of one cache row in several chunks
+    (130, 2, 4, 2, 128, 2600, "shared"),
     (70, 2, 2, 2, 128, 200, "shared"),
 ])
 def test_decode_of_large_batches(device, B, S, hq, hkv, d, L, rows):
