@@ -529,8 +529,8 @@ __global__ __launch_bounds__(kThreads) void cache_merge_splits_d64_kernel(const 
 constexpr int kDecKeys = 32;  // keys per wave tile
 constexpr int kDecRows = 32;  // query rows of the decode kernel (one wave's columns)
 constexpr float kRefRange = 30.f;  // how far (log2) a tile's reference may lie below the row's maximum
-// Shares of the line: two waves and two workgroups per CU, whose starts and ends
-// overlap; a unit of the line is both stages of every wave.
+// Shares of the line: two waves and two (or three, cache_split) workgroups per CU, whose
+// starts and ends overlap; a unit of the line is both stages of every wave.
 constexpr int kShareWaves = 2;
 constexpr int kShareUnit = 2 * kShareWaves;
 // One workgroup per pair: four waves, one workgroup per CU; every pair is whole,
@@ -1191,8 +1191,12 @@ CacheSplit cache_split(const MimirCacheAttnParams& p) {
       // Two workgroups per CU, or one per unit and kv head if there cannot be as many (head_dim
       // 64: if those are at most four per CU, which its LDS allows: 16 rows of 10 to 4000 keys,
       // 8 / 2 heads, 13.2 -> 11.8 us); two part slots each: partial O, then (max, sum) rows.
+      // Three at head_dim 64 with up to four kv heads, whose key rows of at most 512 bytes keep
+      // fewer bytes in flight (two / three: 8 / 2 heads, 252 rows of 2009 to 2068 keys 55.4 / 51.6
+      // us, 400 of 500 to 2000 57.8 / 53.6, 24 of 500 to 2400 13.3 / 11.4, 64 of 2000 19.0 / 20.0;
+      // 8 / 8 heads, 128 of 2000 110.6 / 124.1).
       const int64_t cus = device_cu_count(), most = (int64_t)p.batch * ((tiles + kShareUnit - 1) / kShareUnit);
-      int64_t shares = 2 * cus / p.num_kv_heads;
+      int64_t shares = (p.head_dim == 64 && p.num_kv_heads <= 4 ? 3 : 2) * cus / p.num_kv_heads;
       if (shares < 1) shares = 1;
       if (p.head_dim == 64 && most * p.num_kv_heads <= 4 * cus) shares = most;
       s.units = p.num_kv_heads * (most < shares ? most : shares);
