@@ -9,8 +9,8 @@
 // 391-476, dQ 967-1039, dK/dV 1245-1322), extended to GQA.
 //
 // A workgroup owns 32 rows (queries, or keys for dK / dV) of one head; its four
-// waves take the 32-row tiles of the other side in turn, each with accumulators
-// of its own that are added through LDS at the end.  Small fp32 batches (a few
+// waves (fewer for documents of up to two tiles) take the 32-row tiles of the other
+// side in turn, each with accumulators of its own that are added through LDS at the end.  Small fp32 batches (a few
 // thousand tokens) then still put two waves on every SIMD (one in the backward at
 // head_dim 96 and 128, whose operands take more than half of its registers), and
 // the tile loop holds no barrier.  With the owned rows on the columns of every product, S^T =
@@ -46,8 +46,8 @@
 namespace {
 using namespace mimir;
 
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * 64;
+constexpr int kMaxWaves = 4;         // waves of a workgroup: 1, 2 or 4 (waves_for)
+constexpr int kThreads = kMaxWaves * 64;
 constexpr int kRows = 32;            // rows per workgroup, and per streamed tile
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kDeltaRows = kThreads / 4;  // delta: 64 rows, 4 lanes per row
@@ -71,9 +71,12 @@ struct F32Args {
   int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh, do_st, do_sh;
   int64_t dq_st, dq_sh, dk_st, dk_sh, dv_st, dv_sh, lse_sh;
   int T, Hq, Hkv, group, total_seqlen, is_causal, num_tiles, numseqs;
+  int longer_than, up_to;  // serves the documents of more than / at most so many tokens
   int z0;  // backward: first role of the grid (0: dK / dV, 1 + g: dQ of q head g of the group)
   float scale, scale_log2;
 };
+
+__device__ __forceinline__ bool served(const F32Args& a, int n) { return n > a.longer_than && n <= a.up_to; }
 
 __device__ __forceinline__ float sum4(float x) {
   x += __shfl_xor(x, 1, 64);
@@ -120,14 +123,14 @@ __device__ __forceinline__ void pin() { __builtin_amdgcn_sched_barrier(0); }
 // Row of accumulator register r in lane half hi.
 __device__ __forceinline__ constexpr int acc_row(int r, int hi) { return 8 * (r >> 2) + 4 * hi + (r & 3); }
 
-// LDS of a workgroup: up to two owned operands, later the partial sums of the
-// four waves.
-template <int D>
+// LDS of a workgroup of W waves: the owned operands, later the partial sums of the
+// waves.
+template <int D, int W, int kOwned = 2>
 struct Smem {
   static constexpr int kStride = D + 4;
   static constexpr int kTile = kRows * kStride;
-  float x[kWaves * kTile];
-  float m[kWaves][kRows], l[kWaves][kRows];
+  float x[(W > kOwned ? W : kOwned) * kTile];
+  float m[W][kRows], l[W][kRows];
 };
 
 // One streamed 32-row tile of a [rows, D] fp32 matrix (row stride in elements).
@@ -186,9 +189,9 @@ struct LaneOff {
 };
 
 // The workgroup's 32 owned rows -> LDS; rows past nrows are zero.
-template <int D>
+template <int D, int W>
 __device__ __forceinline__ void stage_owned(float* dst, const float* base, int64_t stride, int row0, int nrows) {
-  constexpr int N = kRows * (D / 4) / kThreads;  // 16-byte units per thread
+  constexpr int kThreads = W * 64, N = kRows * (D / 4) / kThreads;  // 16-byte units per thread
   const Tile<D> t(base, stride, row0, nrows);
   i32x4 v[N];
 #pragma unroll
@@ -199,7 +202,7 @@ __device__ __forceinline__ void stage_owned(float* dst, const float* base, int64
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     const int i = threadIdx.x + j * kThreads, row = i / (D / 4), c = i % (D / 4);
-    *(i32x4*)&dst[row * Smem<D>::kStride + 4 * c] = v[j];
+    *(i32x4*)&dst[row * Smem<D, W>::kStride + 4 * c] = v[j];
   }
 }
 
@@ -239,7 +242,7 @@ __device__ __forceinline__ f32x16 product_tree(const f32x4 (&x)[D / 8], const fl
 // otherwise moves the additions to their use and holds all chains until then.
 template <int D, int kChain>
 __device__ __forceinline__ f32x16 product_rows(const f32x4 (&x)[D / 8], const float* w, int l32, int hi) {
-  const float* row = w + l32 * Smem<D>::kStride + 4 * hi;
+  const float* row = w + l32 * Smem<D, 1>::kStride + 4 * hi;
   f32x16 sum = product_tree<D, kChain, 0, 16>(x, row);
   if constexpr (D > 32) {
     sum += product_tree<D, kChain, 16, 16>(x, row);
@@ -270,7 +273,7 @@ __device__ __forceinline__ void product_cols(f32x16 (&acc)[D / 32], const float 
 template <int D>
 __device__ __forceinline__ void put_partial(float* dst, const f32x16 (&acc)[D / 32], float scale, int l32, int hi) {
   constexpr int C = D / 32;
-  float* row = dst + l32 * Smem<D>::kStride;
+  float* row = dst + l32 * Smem<D, 1>::kStride;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {  // registers 4 g .. + 3: columns C * (8 g + 4 hi) .. + 4 C
     float v[4 * C];
@@ -284,17 +287,17 @@ __device__ __forceinline__ void put_partial(float* dst, const f32x16 (&acc)[D / 
   }
 }
 
-// finish(row, sum of the four partials) -> global rows row0 .. of [rows, D].
-template <int D, typename Finish>
+// finish(row, sum of the waves' partials) -> global rows row0 .. of [rows, D].
+template <int D, int W, typename Finish>
 __device__ __forceinline__ void store_sum(const float* x, float* base, int64_t stride, int row0, int nrows,
                                           Finish&& finish) {
-  using S = Smem<D>;
-  for (int i = threadIdx.x; i < kRows * (D / 4); i += kThreads) {
+  using S = Smem<D, W>;
+  for (int i = threadIdx.x; i < kRows * (D / 4); i += W * 64) {
     const int row = i / (D / 4), c = i % (D / 4);
     if (row0 + row >= nrows) continue;
     f32x4 t = *(const f32x4*)&x[row * S::kStride + 4 * c];
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) t += *(const f32x4*)&x[w * S::kTile + row * S::kStride + 4 * c];
+    for (int w = 1; w < W; ++w) t += *(const f32x4*)&x[w * S::kTile + row * S::kStride + 4 * c];
     *(f32x4*)&base[(int64_t)(row0 + row) * stride + 4 * c] = finish(row, t);
   }
 }
@@ -308,16 +311,16 @@ struct Lanes {
   }
 };
 
-template <int D>
-__global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(const F32Args a) {
+template <int D, int W>
+__global__ __launch_bounds__(W * 64, 2) void fwd_f32_kernel(const F32Args a) {
   constexpr int C = D / 32;
-  __shared__ __attribute__((aligned(16))) Smem<D> sm;
+  __shared__ __attribute__((aligned(16))) Smem<D, W, 1> sm;
   const int h = blockIdx.x % a.Hq;
   const int s = blockIdx.x / a.Hq;
   const int tile = a.num_tiles - 1 - (int)blockIdx.y;  // heaviest first
   const SeqGeom g = load_seq<true>(a.cu_seqlens, a.prefix_lens, s, a.total_seqlen, a.is_causal, a.T);
   const int m0 = tile * kRows;
-  if (m0 >= g.nq) return;
+  if (m0 >= g.nq || !served(a, g.n)) return;
   const int hk = h / a.group;
   const Lanes ln;
   const int kend = kend_of(g.p, m0 + ln.l32);
@@ -331,20 +334,20 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(const F32Args a) {
   float vx[16][C];
   int kt = ln.wave;
   if (kt < n_tiles) Tile<D>(kb, a.k_st, kt * kRows, g.n).rows(kx, ko.row);
-  stage_owned<D>(sm.x, a.q + (int64_t)g.start * a.q_st + (int64_t)h * a.q_sh, a.q_st, m0, g.nq);
+  stage_owned<D, W>(sm.x, a.q + (int64_t)g.start * a.q_st + (int64_t)h * a.q_sh, a.q_st, m0, g.nq);
   __syncthreads();
 
   f32x16 acc[C];
 #pragma unroll
   for (int dt = 0; dt < C; ++dt) acc[dt] = f32x16{};
   float m_run = -INFINITY, l_run = 0.f;
-  for (; kt < n_tiles; kt += kWaves) {
+  for (; kt < n_tiles; kt += W) {
     const int k0 = kt * kRows;
     Tile<D>::cols(vx, vb, a.v_st, k0, g.n, vo.col, vo.row_bytes);
     pin();
     f32x16 st = product_rows<D, kScoreChain<D>>(kx, sm.x, ln.l32, ln.hi);
     // the next tile's rows (none past the last: an empty range reads zeros)
-    Tile<D>(kb, a.k_st, k0 + kWaves * kRows, kt + kWaves < n_tiles ? g.n : 0).rows(kx, ko.row);
+    Tile<D>(kb, a.k_st, k0 + W * kRows, kt + W < n_tiles ? g.n : 0).rows(kx, ko.row);
     pin();
     if (k0 + kRows > kend_min) {
       __asm__ volatile("");
@@ -381,12 +384,12 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(const F32Args a) {
   __syncthreads();  // also: every wave is done with the owned rows
   float M = sm.m[0][ln.l32];
 #pragma unroll
-  for (int w = 1; w < kWaves; ++w) M = fmaxf(M, sm.m[w][ln.l32]);
+  for (int w = 1; w < W; ++w) M = fmaxf(M, sm.m[w][ln.l32]);
   const float wt = m_run == -INFINITY ? 0.f : fast_exp2((m_run - M) * a.scale_log2);
-  put_partial<D>(sm.x + ln.wave * Smem<D>::kTile, acc, wt, ln.l32, ln.hi);
+  put_partial<D>(sm.x + ln.wave * Smem<D, W>::kTile, acc, wt, ln.l32, ln.hi);
   float l_sum = 0.f;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
+  for (int w = 0; w < W; ++w) {
     const float m = sm.m[w][ln.l32];
     l_sum += m == -INFINITY ? 0.f : sm.l[w][ln.l32] * fast_exp2((m - M) * a.scale_log2);
   }
@@ -397,17 +400,17 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_f32_kernel(const F32Args a) {
       a.lse[(int64_t)h * a.lse_sh + g.start + m0 + threadIdx.x] = M * a.scale + logf(l_sum);
   }
   __syncthreads();
-  store_sum<D>(sm.x, a.o + (int64_t)g.start * a.o_st + (int64_t)h * a.o_sh, a.o_st, m0, g.nq,
+  store_sum<D, W>(sm.x, a.o + (int64_t)g.start * a.o_st + (int64_t)h * a.o_sh, a.o_st, m0, g.nq,
                [&](int row, f32x4 t) { return t / sm.l[0][row]; });  // not times 1 / l: one rounding less
 }
 
 // dQ of one (head, sequence, 32-query tile): dQ^T += K^T dS^T over the key tiles.
-template <int D>
-__device__ __forceinline__ void dq_body(const F32Args& a, Smem<D>& sm, int h, int s, int tile) {
+template <int D, int W>
+__device__ __forceinline__ void dq_body(const F32Args& a, Smem<D, W>& sm, int h, int s, int tile) {
   constexpr int C = D / 32;
   const SeqGeom g = load_seq<true>(a.cu_seqlens, a.prefix_lens, s, a.total_seqlen, a.is_causal, a.T);
   const int m0 = tile * kRows;
-  if (m0 >= g.nq) return;
+  if (m0 >= g.nq || !served(a, g.n)) return;
   const int hk = h / a.group;
   const Lanes ln;
   const int qpos = m0 + ln.l32;
@@ -430,24 +433,24 @@ __device__ __forceinline__ void dq_body(const F32Args& a, Smem<D>& sm, int h, in
   const float lse2 = valid ? a.lse2[(int64_t)h * a.T + g.start + qpos] : 0.f;
   const float dlt = valid ? a.delta[(int64_t)h * a.T + g.start + qpos] : 0.f;
   float* const sq = sm.x;
-  float* const sdo = sm.x + Smem<D>::kTile;
-  stage_owned<D>(sq, a.q + (int64_t)g.start * a.q_st + (int64_t)h * a.q_sh, a.q_st, m0, g.nq);
-  stage_owned<D>(sdo, a.dout + (int64_t)g.start * a.do_st + (int64_t)h * a.do_sh, a.do_st, m0, g.nq);
+  float* const sdo = sm.x + Smem<D, W>::kTile;
+  stage_owned<D, W>(sq, a.q + (int64_t)g.start * a.q_st + (int64_t)h * a.q_sh, a.q_st, m0, g.nq);
+  stage_owned<D, W>(sdo, a.dout + (int64_t)g.start * a.do_st + (int64_t)h * a.do_sh, a.do_st, m0, g.nq);
   __syncthreads();
 
   f32x16 acc[C];
 #pragma unroll
   for (int dt = 0; dt < C; ++dt) acc[dt] = f32x16{};
-  for (; kt < n_tiles; kt += kWaves) {
+  for (; kt < n_tiles; kt += W) {
     const int k0 = kt * kRows;
-    const int n_next = kt + kWaves < n_tiles ? g.n : 0;
+    const int n_next = kt + W < n_tiles ? g.n : 0;
     f32x16 st = product_rows<D, kScoreChain<D>>(kx, sq, ln.l32, ln.hi);
     pin();
     Tile<D>::cols(kc, kb, a.k_st, k0, g.n, ko.col, ko.row_bytes);
-    Tile<D>(kb, a.k_st, k0 + kWaves * kRows, n_next).rows(kx, ko.row);
+    Tile<D>(kb, a.k_st, k0 + W * kRows, n_next).rows(kx, ko.row);
     const f32x16 dp = product_rows<D, kDpChain<D>>(vx, sdo, ln.l32, ln.hi);
     pin();
-    Tile<D>(vb, a.v_st, k0 + kWaves * kRows, n_next).rows(vx, vo.row);
+    Tile<D>(vb, a.v_st, k0 + W * kRows, n_next).rows(vx, vo.row);
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[r] = fast_exp2(__builtin_fmaf(st[r], a.scale_log2, -lse2));
     if (k0 + kRows > kend_min) {
@@ -461,20 +464,20 @@ __device__ __forceinline__ void dq_body(const F32Args& a, Smem<D>& sm, int h, in
     product_cols<D>(acc, kc, st);
   }
   __syncthreads();  // every wave is done with the owned rows
-  put_partial<D>(sm.x + ln.wave * Smem<D>::kTile, acc, a.scale, ln.l32, ln.hi);
+  put_partial<D>(sm.x + ln.wave * Smem<D, W>::kTile, acc, a.scale, ln.l32, ln.hi);
   __syncthreads();
-  store_sum<D>(sm.x, a.dq + (int64_t)g.start * a.dq_st + (int64_t)h * a.dq_sh, a.dq_st, m0, g.nq,
+  store_sum<D, W>(sm.x, a.dq + (int64_t)g.start * a.dq_st + (int64_t)h * a.dq_sh, a.dq_st, m0, g.nq,
                [](int, f32x4 t) { return t; });
 }
 
 // dK and dV of one (kv head, sequence, 32-key tile): the waves take the (q head,
 // 32-query tile) steps in turn; dV^T += dO^T P, dK^T += Q^T dS.
-template <int D>
-__device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk, int s, int tile) {
+template <int D, int W>
+__device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D, W>& sm, int hk, int s, int tile) {
   constexpr int C = D / 32;
   const SeqGeom g = load_seq<true>(a.cu_seqlens, a.prefix_lens, s, a.total_seqlen, a.is_causal, a.T);
   const int k0 = tile * kRows;
-  if (k0 >= g.n) return;
+  if (k0 >= g.n || !served(a, g.n)) return;
   const Lanes ln;
   const int kpos = k0 + ln.l32;
   const bool valid = kpos < g.n;
@@ -489,7 +492,7 @@ __device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk,
 
   f32x4 qx[Tile<D>::kChunks], ox[Tile<D>::kChunks];
   float qc[16][C], oc[16][C];
-  // this wave's step: q head `hh` of the group and query tile t0 + t; advanced by kWaves
+  // this wave's step: q head `hh` of the group and query tile t0 + t; advanced by W
   int hh = 0, t = ln.wave;
   auto wrap = [&]() __attribute__((always_inline)) {
     while (hh < a.group && t >= n_q) { t -= n_q; ++hh; }
@@ -503,19 +506,19 @@ __device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk,
     tile_of(ob, a.do_st, a.do_sh).rows(ox, oo.row);
   }
   float* const sk = sm.x;
-  float* const sv = sm.x + Smem<D>::kTile;
-  stage_owned<D>(sk, a.k + (int64_t)g.start * a.k_st + (int64_t)hk * a.k_sh, a.k_st, k0, g.n);
-  stage_owned<D>(sv, a.v + (int64_t)g.start * a.v_st + (int64_t)hk * a.v_sh, a.v_st, k0, g.n);
+  float* const sv = sm.x + Smem<D, W>::kTile;
+  stage_owned<D, W>(sk, a.k + (int64_t)g.start * a.k_st + (int64_t)hk * a.k_sh, a.k_st, k0, g.n);
+  stage_owned<D, W>(sv, a.v + (int64_t)g.start * a.v_st + (int64_t)hk * a.v_sh, a.v_st, k0, g.n);
   __syncthreads();
 
   f32x16 dka[C], dva[C];
 #pragma unroll
   for (int dt = 0; dt < C; ++dt) dka[dt] = dva[dt] = f32x16{};
-  for (int it = ln.wave; it < steps; it += kWaves) {
+  for (int it = ln.wave; it < steps; it += W) {
     const int q0 = (t0 + t) * kRows;
     const int h = hk * a.group + hh;
     const float *const qh = qb + (int64_t)hh * a.q_sh, *const oh = ob + (int64_t)hh * a.do_sh;
-    t += kWaves;
+    t += W;
     wrap();
     f32x16 p = product_rows<D, kScoreChain<D>>(qx, sk, ln.l32, ln.hi);
     pin();
@@ -551,16 +554,16 @@ __device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk,
     tile_of(ob, a.do_st, a.do_sh).rows(ox, oo.row);
   }
   const float* const base = sm.x;
-  float* const mine = sm.x + ln.wave * Smem<D>::kTile;
+  float* const mine = sm.x + ln.wave * Smem<D, W>::kTile;
   __syncthreads();  // every wave is done with the owned rows
   put_partial<D>(mine, dva, 1.f, ln.l32, ln.hi);
   __syncthreads();
-  store_sum<D>(base, a.dv + (int64_t)g.start * a.dv_st + (int64_t)hk * a.dv_sh, a.dv_st, k0, g.n,
+  store_sum<D, W>(base, a.dv + (int64_t)g.start * a.dv_st + (int64_t)hk * a.dv_sh, a.dv_st, k0, g.n,
                [](int, f32x4 t) { return t; });
   __syncthreads();
   put_partial<D>(mine, dka, a.scale, ln.l32, ln.hi);
   __syncthreads();
-  store_sum<D>(base, a.dk + (int64_t)g.start * a.dk_st + (int64_t)hk * a.dk_sh, a.dk_st, k0, g.n,
+  store_sum<D, W>(base, a.dk + (int64_t)g.start * a.dk_st + (int64_t)hk * a.dk_sh, a.dk_st, k0, g.n,
                [](int, f32x4 t) { return t; });
 }
 
@@ -573,16 +576,57 @@ __device__ __forceinline__ void dkdv_body(const F32Args& a, Smem<D>& sm, int hk,
 // engines, whether or not the next one has room, so the sequences rotate by one
 // per row of tiles: a long or prefix-heavy one then does not land on one engine
 // while the others idle (78 -> 76.7 us).
-template <int D>
-__global__ __launch_bounds__(kThreads, D <= 64 ? 2 : 1) void bwd_f32_kernel(const F32Args a) {
-  __shared__ __attribute__((aligned(16))) Smem<D> sm;
+template <int D, int W>
+__global__ __launch_bounds__(W * 64, D <= 64 ? 2 : 1) void bwd_f32_kernel(const F32Args a) {
+  __shared__ __attribute__((aligned(16))) Smem<D, W> sm;
   const int hk = blockIdx.x % a.Hkv, y = blockIdx.y;
   const int s = (int)(blockIdx.x / a.Hkv + y) % a.numseqs;
   const int z = blockIdx.z + a.z0;
   if (z == 0)
-    dkdv_body<D>(a, sm, hk, s, y);
+    dkdv_body<D, W>(a, sm, hk, s, y);
   else
-    dq_body<D>(a, sm, hk * a.group + z - 1, s, a.num_tiles - 1 - y);
+    dq_body<D, W>(a, sm, hk * a.group + z - 1, s, a.num_tiles - 1 - y);
+}
+
+// By name: of several instantiations launched from one place, this toolchain drops host stubs.
+#define F32_KERNELS(D, W)                                    \
+  template __global__ void fwd_f32_kernel<D, W>(const F32Args); \
+  template __global__ void bwd_f32_kernel<D, W>(const F32Args);
+#define F32_KERNELS_OF(D) F32_KERNELS(D, 1) F32_KERNELS(D, 2) F32_KERNELS(D, 4)
+F32_KERNELS_OF(32)
+F32_KERNELS_OF(64)
+F32_KERNELS_OF(96)
+F32_KERNELS_OF(128)
+
+// Waves of a workgroup whose waves take up to `steps` tiles in turn: no more than find one.
+// Idle ones keep other documents from the chip: a SIMD holds two waves, one in the backward at
+// head_dim 96 and 128.  Forward and backward, us, on the vector ALUs / four waves always / so:
+//   1641 documents of 1 to 4 tokens, 6 heads of 96:  121, 447 / 132, 774 / 58, 227
+//   395 documents of 5 to 16, 8 heads of 64:         36, 128 / 41, 111 / 23, 53
+//   83 documents of 33 to 64, 6 heads of 96:         37, 96 / 28, 101 / 22, 66
+// The results are the same bit for bit: an idle wave adds zeros.
+int waves_for(int64_t steps) { return steps <= 1 ? 1 : steps == 2 ? 2 : kMaxWaves; }
+
+// launch(tiles, waves) for the documents of a call, with a's bounds set to those it is to
+// serve: all of them, or, where most have one or two tiles but not the longest and they fill
+// the chip several times, the short ones in a launch of their own with the waves that they
+// need.  On the vector ALUs / one launch / two, us, with one document of 100 tokens among them:
+//   1596 of 1 to 4 tokens, 6 heads of 96:    124, 454 / 148, 821 / 80, 328
+//   386 of 5 to 16, 8 heads of 64:           39, 141 / 47, 127 / 33, 78
+//   498 of 30 to 34, 6 heads of 96:          87, 280 / 89, 415 / 70, 280
+// and 164 of 17 to 32, 8 heads of 64, the fewest that this line takes: 29, 104 / 26, 65 / 29, 60.
+template <typename Launch>
+void launch_documents(F32Args& a, int64_t heads_per_step, Launch&& launch) {
+  const int64_t mean = a.numseqs > 0 ? a.total_seqlen / a.numseqs : 0;
+  const int short_tiles = mean <= 16 ? 1 : 2;
+  const int short_waves = waves_for(short_tiles * heads_per_step), waves = waves_for(a.num_tiles * heads_per_step);
+  a.longer_than = 0, a.up_to = 0x7fffffff;
+  if (mean <= 40 && short_waves < waves && (int64_t)a.numseqs * a.Hq >= 4 * device_cu_count()) {
+    a.up_to = short_tiles * kRows;
+    launch(short_tiles, short_waves);
+    a.longer_than = a.up_to, a.up_to = 0x7fffffff;
+  }
+  launch(a.num_tiles, waves);
 }
 
 F32Args common_args(int T, int Hq, int Hkv, int total_seqlen, int is_causal, float scale,
@@ -615,8 +659,17 @@ hipError_t launch_fwd(const MimirPrefixLMFwdParams& p, hipStream_t stream) {
   a.num_tiles = (p.max_seqlen_all + kRows - 1) / kRows;
   a.numseqs = p.numseqs;
   if (a.num_tiles == 0 || p.numseqs == 0) return hipSuccess;
-  hipLaunchKernelGGL(fwd_f32_kernel<D>, dim3(p.num_q_heads * p.numseqs, a.num_tiles), dim3(kThreads), 0,
-                     stream, a);
+  launch_documents(a, 1, [&](int tiles, int waves) {
+    F32Args b = a;
+    b.num_tiles = tiles;
+    const dim3 grid(p.num_q_heads * p.numseqs, tiles), block(waves * 64);
+    if (waves == 1)
+      hipLaunchKernelGGL((fwd_f32_kernel<D, 1>), grid, block, 0, stream, b);
+    else if (waves == 2)
+      hipLaunchKernelGGL((fwd_f32_kernel<D, 2>), grid, block, 0, stream, b);
+    else
+      hipLaunchKernelGGL((fwd_f32_kernel<D, 4>), grid, block, 0, stream, b);
+  });
   return hipGetLastError();
 }
 
@@ -648,8 +701,17 @@ hipError_t launch_bwd(const MimirPrefixLMBwdParams& p, hipStream_t stream, int s
   a.z0 = stages & MIMIR_BWD_STAGE_DKDV ? 0 : 1;
   const int z1 = stages & MIMIR_BWD_STAGE_DQ ? 1 + a.group : 1;
   if (a.num_tiles > 0 && p.numseqs > 0 && z1 > a.z0)
-    hipLaunchKernelGGL(bwd_f32_kernel<D>, dim3(p.num_kv_heads * p.numseqs, a.num_tiles, z1 - a.z0), dim3(kThreads), 0,
-                       stream, a);
+    launch_documents(a, a.group, [&](int tiles, int waves) {  // dK / dV: the tiles of the group's q heads
+      F32Args b = a;
+      b.num_tiles = tiles;
+      const dim3 grid(p.num_kv_heads * p.numseqs, tiles, z1 - a.z0), block(waves * 64);
+      if (waves == 1)
+        hipLaunchKernelGGL((bwd_f32_kernel<D, 1>), grid, block, 0, stream, b);
+      else if (waves == 2)
+        hipLaunchKernelGGL((bwd_f32_kernel<D, 2>), grid, block, 0, stream, b);
+      else
+        hipLaunchKernelGGL((bwd_f32_kernel<D, 4>), grid, block, 0, stream, b);
+    });
   return hipGetLastError();
 }
 

@@ -218,6 +218,29 @@ def test_f32_tile_edges(device, d, hq, hkv, causal):
         assert torch.equal(x.detach().cpu(), got[name]), name
 
 
+@pytest.mark.parametrize("longest", [1, 32, 33, 64, 65])
+@pytest.mark.parametrize("d,hq,hkv", [(32, 4, 4), (64, 2, 2), (96, 3, 3), (128, 2, 2), (64, 4, 2), (128, 6, 2)])
+def test_f32_waves_of_a_workgroup(device, longest, d, hq, hkv):
+    """One, two or four waves, as many as the longest document (and, for dK / dV, the group's q
+    heads) has tiles for: around one and two tiles, among shorter documents."""
+    lens = [longest, 1, min(7, longest), longest, max(longest - 1, 1)]
+    case = make_case(lens, [n * i // 4 for i, n in enumerate(lens)], hq, hkv, d, seed=d + longest, dtype=torch.float32,
+                     pad_to=sum(lens) + 3, is_causal=False)
+    check(case, device, label=f"f32 waves longest={longest} D={d} heads={hq}/{hkv}")
+
+
+@pytest.mark.parametrize("d,hq,hkv,lo,hi,longest", [(32, 16, 16, 1, 25, 70), (64, 16, 8, 28, 36, 130), (96, 16, 16, 1, 9, 33)])
+def test_f32_short_documents_in_a_launch_of_their_own(device, d, hq, hkv, lo, hi, longest):
+    """Enough documents of one tile (of two, where their mean is above 16 tokens) among a few
+    longer ones; lengths at the line between the two launches."""
+    gen = torch.Generator().manual_seed(d)
+    lens = torch.randint(lo, hi + 1, (66,), generator=gen).tolist()
+    lens[3], lens[20], lens[40:44], lens[65] = longest, longest - 1, [32, 33, 64, 65], longest
+    prefixes = [int(torch.randint(0, n + 1, (1,), generator=gen)) for n in lens]
+    case = make_case(lens, prefixes, hq, hkv, d, seed=d, dtype=torch.float32, pad_to=sum(lens) + 2)
+    check(case, device, label=f"f32 short documents D={d} heads={hq}/{hkv}")
+
+
 @pytest.mark.parametrize("d,o_bound,dq_bound", [(32, 9.0e-8, 2.3e-7), (64, 1.0e-7, 2.6e-7), (96, 1.1e-7, 3.1e-7),
                                                 (128, 1.15e-7, 3.2e-7)])
 def test_f32_error_on_short_documents(device, d, o_bound, dq_bound):
