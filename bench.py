@@ -178,8 +178,8 @@ def working_kernels(d: int, elem: int, handoff: bool) -> dict:
     share a launch in a step, and have one each where the stages are timed.
     """
     if elem == 4:
-        bwd = f"bwd_f32_kernel<{d}>"
-        return {"fwd": f"fwd_f32_kernel<{d}>", "dkdv": f"{bwd} (dK/dV workgroups)", "dq": f"{bwd} (dQ workgroups)"}
+        bwd = f"bwd_f32_kernel<{d}, 4>"  # four waves: documents of more than two 32-row tiles
+        return {"fwd": f"fwd_f32_kernel<{d}, 4>", "dkdv": f"{bwd} (dK/dV workgroups)", "dq": f"{bwd} (dQ workgroups)"}
     if d == 128:
         dkdv = "dkdv_pair_ds_kernel" if handoff else "dkdv_pair_kernel"
     else:
